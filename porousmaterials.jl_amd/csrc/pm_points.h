@@ -29,6 +29,8 @@
 // lands in and the tuning of chunk sizes therefore never change a result.
 #pragma once
 
+#include <type_traits>
+
 #include "pm_device.h"
 
 namespace pmk {
@@ -36,13 +38,13 @@ namespace pmk {
 // Images per spatial tile of an image list (one wave loads a tile).
 constexpr int TILE_IMAGES = 64;
 
-constexpr int ERFC_SEG = 512;      // cubic segments of erfc(alpha r) on [0, r_sr] (FP32 path)
-// The largest float below ERFC_SEG: the scaled distance is clamped to it, so
-// the last segment keeps its own t in [0, 1) up to r_sr, a distance beyond r_sr
-// (a masked term) reads a finite value, and r = 0 (0 * inf = NaN) reads
-// segment ERFC_SEG - 1 rather than a NaN.
-constexpr float ERFC_XMAX = (float)ERFC_SEG - (float)ERFC_SEG / 16777216.0f;
-constexpr int ERFC64_SEG = 512;    // quintic segments of erfc(alpha r) on [0, r_sr] (FP64 path)
+// FP32 path: cubics of erfc(alpha r) on [0, r_sr] in t = r/h - i, h = r_sr / ERFC_SEG, and a
+// last entry, constant at erfc(alpha r_sr), for a scaled distance that rounds up to ERFC_SEG
+constexpr int ERFC_SEG = 512;
+constexpr int ERFC_TAB = ERFC_SEG + 1;
+// FP64 path: quintics of erfc(alpha r) about r = i h, i = 0..ERFC64_SEG, h = r_sr / ERFC64_SEG
+constexpr int ERFC64_SEG = 512;
+constexpr int ERFC64_TAB = 3 * (ERFC64_SEG + 1);  // double2 entries of the table
 constexpr int SCAN_WG = 1024;      // work-items of the scan kernels
 constexpr int GT = PM_MAX_GRAD_TYPES;  // framework types of a gradient run (fixed stride)
 constexpr int GQ = 4;                  // per-type sums per point: d/d eps, d/d sigma, erfc/r, Fourier
@@ -69,9 +71,9 @@ struct RunArgs {
     const int2* tile_rng;    // per tile: first image, image count (<= 64)
     const double4* atoms;    // replicated atoms (fallback path)
     const int* species;
-    const void* ljtab;       // [n_types][nsite] LJP<Real>
-    const float4* erfc_tab;  // ERFC_SEG cubics of erfc(alpha r) in t = r/h - i
-    const double2* erfc64_tab;  // ERFC64_SEG quintics (c0, c1), (c2, c3), (c4, c5) in t = r/h - i
+    const void* ljtab;       // [n_types][nsite] LJC<Real>::type
+    const float4* erfc_tab;  // cubics of erfc(alpha r) in t = r/h - i
+    const double2* erfc64_tab;  // quintics of erfc(alpha r), (c0, c1), (c2, c3), (c4, c5) in t = r/h - i
     double erfc64_inv_h;
     // Fourier box: ma in [0, Ma], mb in [-Mb, Mb], mc in [-Mc, Mc]
     int Ma, Mb, Mc;
@@ -98,7 +100,7 @@ struct RunArgs {
     // parameter gradients (adjoint Widom runs)
     int n_gt;                // framework types (<= GT)
     int pstride;             // doubles per workgroup partial: 3, or GK for a gradient run
-    const void* gtab;        // [n_types][nsite] Real: 4 eps_ts / sigma_ts (d LJ / d sigma_ts factor)
+    const void* gtab;        // [n_types][nsite] double2: sigma_ts^6, 4 eps_ts / sigma_ts
     const double4* jac;      // [n_types][nsite]: d eps_ts/d eps_t, d eps_ts/d sigma_t, d sigma_ts/d eps_t,
                              // d sigma_ts/d sigma_t of the mixing rule
     const double2* A_t;      // per-type Fourier boxes: GT complex coefficients per box entry
@@ -492,8 +494,17 @@ __global__ void slice_items_kernel(const unsigned* count, const unsigned* slice_
 }
 
 // ---------------------------------------------------------------- pairs ----
-// The erfc(alpha r) tables of a run in LDS: FP32 cubics (mixed path) or FP64
-// quintics (FP64 path), each with 1/h of its segments.
+// LJ pair constants.  FP32 pairs: sigma^2 and 4 eps.  FP64 pairs: 4 eps (u^2 - u),
+// u = (sigma^2 / r^2)^3, as r6 (a r6 - b) with r6 = r^-6, a = 4 eps sigma^12,
+// b = 4 eps sigma^6 (one FP64 operation fewer).
+struct LJAB {
+    double a, b;
+};
+template <typename Real>
+using LJC = typename std::conditional<sizeof(Real) == 4, LJP<float>, LJAB>::type;
+
+// The erfc(alpha r) tables of a run in LDS, each with 1/h of its segments: FP32
+// cubics (mixed path) or FP64 quintics (FP64 path).
 struct ErfcTabs {
     float inv_h;
     const float4* tab;
@@ -501,126 +512,115 @@ struct ErfcTabs {
     const double2* tab64;
 };
 
-// The largest double below ERFC64_SEG (the FP64 twin of ERFC_XMAX).
-constexpr double ERFC64_XMAX = (double)ERFC64_SEG - (double)ERFC64_SEG / 9007199254740992.0;
+// The sums a pair adds to.  plj, psr: energies.  s1, s2, sq (gradient runs, for
+// candidates of one framework type): FP32 pairs, s1 = sum of u^2 - u and s2 =
+// sum of u over pairs inside the LJ cutoff; FP64 pairs, the sums of r^-12 and
+// r^-6; sq = sum of erfc(alpha r) / r over pairs inside the real-space cutoff.
+template <typename Real>
+struct PairSums {
+    Real plj = (Real)0, psr = (Real)0, s1 = (Real)0, s2 = (Real)0, sq = (Real)0;
+};
 
-// erfc(alpha r) from the FP64 segment table, Horner in t = r/h - i.  The
-// scaled distance is clamped below ERFC64_SEG: beyond r_sr (a masked term)
-// the last segment gives a finite value, and so does r = NaN (r2 = 0, where
-// the caller's 1/r is +inf).
-__device__ inline double erfc_tab64(double r, const ErfcTabs& et) {
-    const double x = fmin(r * et.inv_h64, ERFC64_XMAX);
-    const int i = (int)x;
-    const double t = x - (double)i;
-    const double2 c01 = et.tab64[3 * i], c23 = et.tab64[3 * i + 1], c45 = et.tab64[3 * i + 2];
-    return fma(fma(fma(fma(fma(c45.y, t, c45.x), t, c23.y), t, c23.x), t, c01.y), t, c01.x);
-}
-
-// 1/sqrt(r2) in FP64: v_rsq_f64 and two Newton steps y <- y (3/2 - r2 y^2 / 2)
-// (the estimate's ~2^-22 relative error squares at each step, so the result
-// is within a few ulp); r2 below the smallest normal gives +inf, as
-// 1 / sqrt(0) does.
-__device__ inline double rsq64(double r2) {
-    double y = __builtin_amdgcn_rsq(r2);
-    const double h = 0.5 * r2;
-    y = fma(y, fma(-(h * y), y, 0.5), y);
-    y = fma(y, fma(-(h * y), y, 0.5), y);
-    return r2 >= 2.2250738585072014e-308 ? y : INFINITY;
-}
-
-// One candidate pair: LJ into plj, real-space Ewald into psr.
-// FP32 pairs: the masked terms accumulate by one FMA each (eps4 * w and
-// q / r * erfc), the table offset is v_fract of the scaled distance, and the
-// candidate's charge arrives in FP32 (qf).  FP64 pairs: 1/r from rsq64,
-// 1/r^2 as its square, erfc(alpha r) from the FP64 table.
-template <int ESM, typename Real>
-__device__ inline void pair_term(double r2, double q, float qf, const LJP<Real>& p, bool is_lj, double r2lj,
-                                 double r2sr, const ErfcTabs& et, bool& ovl, Real& plj, Real& psr) {
-    const float inv_h = et.inv_h;
-    const float4* tab = et.tab;
+// One candidate pair: LJ and real-space Ewald.  The energies are the same
+// operations in the same order with and without GRAD, so a gradient run's
+// energies equal a plain run's bit for bit.  Returns r^2 in Real.
+//
+// The kernels are bound by the issue of these instructions.  Measured on
+// independent streams (wave instructions per CU and ns): FP64 add/multiply/FMA
+// 1.8-2.0, compares, selects, minima, conversions and three-operand integer
+// operations 2.0-2.3, FP32 FMA/multiply/add and plain integer operations up to
+// 3.0-3.7, v_rsq_f32 1.1, v_rsq_f64 0.6, and an LDS read takes the LDS as long
+// for 8 bytes as for 16 (0.58).  So:
+// - a pair outside the cutoff is masked once, through its 1/r (every masked
+//   term is then an exact zero and reads a valid table entry), not term by
+//   term; the overlap test is left to the caller, who follows the smallest r^2
+//   of a tile's candidates (pair_loop) instead of comparing every pair;
+// - FP64: 1/r by v_rsq_f64 and one third-order step, y (1 + e/2 + 3 e^2/8) with
+//   e = 1 - r^2 y^2 (the estimate's 2^-22 cubes to below an ulp); index and
+//   offset of the table by the addition of 1.5 2^52 in place of conversions.
+// NEAR: with the overlap flag and for r^2 too small for a finite 1/r (the other
+// form leaves both to its caller).
+template <int ESM, typename Real, bool GRAD, bool NEAR>
+__device__ __attribute__((always_inline)) inline Real pair_term(double r2, double q, float qf, const LJC<Real>& p,
+                                                                bool is_lj, double r2lj, double r2sr,
+                                                                const ErfcTabs& et, bool& ovl, PairSums<Real>& S) {
     const bool in = r2 < r2lj;
-    ovl |= in & (r2 < R2_OVERLAP) & is_lj;
-    if constexpr (ESM != 0 && sizeof(Real) == 4) {
-        // one transcendental per pair: 1/r from v_rsq, 1/r^2 as its square
-        const float rf2 = (float)r2;
-        const float rinv = __builtin_amdgcn_rsqf(rf2);
-        const float s = p.sig2 * (rinv * rinv);
-        const float s3 = s * s * s;
-        plj = fmaf(p.eps4, in ? fmaf(s3, s3, -s3) : 0.0f, plj);
-        const bool ins = ((ESM == 1) ? in : (r2 < r2sr)) & (qf != 0.0f);
-        const float x = fminf(rf2 * rinv * inv_h, ERFC_XMAX);
-        const int i = (int)x;
-        const float t = __builtin_amdgcn_fractf(x);
-        const float4 c = tab[i];
-        const float ec = fmaf(fmaf(fmaf(c.w, t, c.z), t, c.y), t, c.x);
-        psr = fmaf(ins ? qf * rinv : 0.0f, ec, psr);
-    } else if constexpr (sizeof(Real) == 4) {
-        const float s = p.sig2 * __builtin_amdgcn_rcpf((float)r2);
-        const float s3 = s * s * s;
-        plj = fmaf(p.eps4, in ? fmaf(s3, s3, -s3) : 0.0f, plj);
-    } else {
-        const double y = rsq64(r2);
-        const double s = p.sig2 * (y * y);
-        const double s3 = s * s * s;
-        plj += in ? p.eps4 * s3 * (s3 - 1.0) : 0.0;
-        if constexpr (ESM != 0) {
-            const bool ins = ((ESM == 1) ? in : (r2 < r2sr)) & (q != 0.0);
-            psr += ins ? q * y * erfc_tab64(r2 * y, et) : 0.0;
-        }
-    }
-}
-
-// pair_term with the sums of a gradient run, for a candidate of the framework
-// type the caller is summing: sw += u^2 - u and su += u over pairs inside the
-// LJ cutoff (u = (sigma_ts^2 / r^2)^3), sq += erfc(alpha r) / r over pairs
-// inside the real-space cutoff, all in Real.  d LJ / d eps_ts = 4 (u^2 - u) and
-// d LJ / d sigma_ts = (4 eps_ts / sigma_ts)(12 u^2 - 6 u) = csig (12 sw + 6 su),
-// so the caller forms both per type from sw and su.  The energy terms are
-// pair_term's, operation for operation: a gradient run's energies equal a
-// plain run's bit for bit.
-template <int ESM, typename Real>
-__device__ inline void pair_term_grad(double r2, double q, float qf, const LJP<Real>& p, bool is_lj, double r2lj,
-                                      double r2sr, const ErfcTabs& et, bool& ovl, Real& plj, Real& psr, Real& sw,
-                                      Real& su, Real& sq) {
-    const bool in = r2 < r2lj;
-    ovl |= in & (r2 < R2_OVERLAP) & is_lj;
+    const bool ins = ESM == 2 ? r2 < r2sr : in;
     if constexpr (sizeof(Real) == 4) {
-        const float rf2 = (float)r2;
+        const float u = (float)r2;
+        if constexpr (NEAR) ovl |= in & (r2 < R2_OVERLAP) & is_lj;
         float rinv = 0.0f, s;
         if constexpr (ESM != 0) {
-            rinv = __builtin_amdgcn_rsqf(rf2);
-            s = p.sig2 * (rinv * rinv);
+            // one transcendental per pair: 1/r from v_rsq, 1/r^2 as its square
+            rinv = __builtin_amdgcn_rsqf(u);
+            const float rl = in ? rinv : 0.0f;
+            s = p.sig2 * (rl * rl);
+            rinv = ESM == 2 ? (ins ? rinv : 0.0f) : rl;
         } else {
-            s = p.sig2 * __builtin_amdgcn_rcpf(rf2);
+            const float i2 = __builtin_amdgcn_rcpf(u);
+            s = p.sig2 * (in ? i2 : 0.0f);
         }
         const float s3 = s * s * s;
-        const float wm = in ? fmaf(s3, s3, -s3) : 0.0f;
-        plj = fmaf(p.eps4, wm, plj);
-        sw += wm;
-        su += in ? s3 : 0.0f;
+        const float w = fmaf(s3, s3, -s3);
+        S.plj = fmaf(p.eps4, w, S.plj);
+        if constexpr (GRAD) {
+            S.s1 += w;
+            S.s2 += s3;
+        }
         if constexpr (ESM != 0) {
-            const bool inr = (ESM == 1) ? in : (r2 < r2sr);
-            const float x = fminf(rf2 * rinv * et.inv_h, ERFC_XMAX);
+            float x = u * rinv * et.inv_h;
+            if constexpr (NEAR) x = rinv < INFINITY ? x : 0.0f;  // r = 0: 0 inf
             const int i = (int)x;
             const float t = __builtin_amdgcn_fractf(x);
             const float4 c = et.tab[i];
             const float ec = fmaf(fmaf(fmaf(c.w, t, c.z), t, c.y), t, c.x);
-            psr = fmaf((inr & (qf != 0.0f)) ? qf * rinv : 0.0f, ec, psr);
-            sq += inr ? ec * rinv : 0.0f;
+            if constexpr (NEAR) S.psr = qf != 0.0f ? fmaf(qf * rinv, ec, S.psr) : S.psr;
+            else S.psr = fmaf(qf * rinv, ec, S.psr);
+            if constexpr (GRAD) S.sq = fmaf(ec, rinv, S.sq);
         }
+        return u;
     } else {
-        const double y = rsq64(r2);
-        const double s = p.sig2 * (y * y);
-        const double s3 = s * s * s;
-        plj += in ? p.eps4 * s3 * (s3 - 1.0) : 0.0;
-        sw += in ? s3 * (s3 - 1.0) : 0.0;
-        su += in ? s3 : 0.0;
-        if constexpr (ESM != 0) {
-            const bool inr = (ESM == 1) ? in : (r2 < r2sr);
-            const double ec = erfc_tab64(r2 * y, et);
-            psr += (inr & (q != 0.0)) ? q * y * ec : 0.0;
-            sq += inr ? ec * y : 0.0;
+        double y = __builtin_amdgcn_rsq(r2);
+        {
+            const double e = fma(-(r2 * y), y, 1.0);
+            y = fma(e * y, fma(e, 0.375, 0.5), y);
         }
+        bool il = in, is = ins;
+        if constexpr (NEAR) {
+            ovl |= in & (r2 < R2_OVERLAP) & is_lj;
+            if (r2 < 2.2250738585072014e-308) {  // 1/r = inf
+                if (in) S.plj += p.a * INFINITY;
+                if constexpr (ESM != 0) {
+                    if (ins && q != 0.0) S.psr += q * INFINITY;
+                    if constexpr (GRAD) S.sq += ins ? INFINITY : 0.0;
+                }
+                il = is = false;
+                y = 0.0;
+            }
+        }
+        // the high word of a masked 1/r is cleared: what is left is below 1e-313
+        const double yl = __hiloint2double(il ? __double2hiint(y) : 0, __double2loint(y));
+        const double i2 = yl * yl;
+        const double r6 = i2 * i2 * i2;
+        S.plj = fma(r6, fma(p.a, r6, -p.b), S.plj);
+        if constexpr (GRAD) {
+            S.s1 = fma(r6, r6, S.s1);
+            S.s2 += r6;
+        }
+        if constexpr (ESM != 0) {
+            const double ys = ESM == 2 ? __hiloint2double(is ? __double2hiint(y) : 0, __double2loint(y)) : yl;
+            constexpr double MAGIC = 6755399441055744.0;  // 1.5 2^52: the sum's low word is the nearest integer
+            const double r = r2 * ys;
+            const double xm = fma(r, et.inv_h64, MAGIC);
+            const int i = __double2loint(xm);
+            const double t = fma(r, et.inv_h64, -(xm - MAGIC));
+            const double2* e = et.tab64 + 3 * i;
+            const double2 c01 = e[0], c23 = e[1], c45 = e[2];
+            const double f = fma(fma(fma(fma(fma(c45.y, t, c45.x), t, c23.y), t, c23.x), t, c01.y), t, c01.x);
+            S.psr = fma(q * ys, f, S.psr);
+            if constexpr (GRAD) S.sq = fma(ys, f, S.sq);
+        }
+        return r2;
     }
 }
 
@@ -646,51 +646,119 @@ struct PairLds {
     double* sph;    // per-wave bounding-box and radius partials of the workgroup's sphere
 };
 
+// Candidates [j0, je) of the LDS list for every lane's point, two at a time in
+// FP32 (they share the LDS address registers, and their chains interleave).
+// GRAD: all of one type, whose constants are pt; else each candidate's type
+// selects its constants.  A branch per candidate on the rare close pair kept
+// the compiler from interleaving the two chains, so the loop only follows the
+// smallest r^2 and the overlap flag comes from it afterwards; where that r^2
+// has no finite 1/r, or is so close to the overlap distance that its FP32 value
+// does not decide, the candidates are taken again one by one.
+template <int ESM, typename Real, bool GRAD>
+__device__ __attribute__((always_inline)) inline void pair_loop(const PairLds& L, int j0, int je, double prx, double pry,
+                                                                double prz, int site, const LJC<Real>* s_lj,
+                                                                const LJC<Real>& pt, bool is_lj, double r2lj,
+                                                                double r2sr, const ErfcTabs& et, bool& ovl,
+                                                                PairSums<Real>& S) {
+    constexpr bool F32 = sizeof(Real) == 4;
+    auto dist2 = [&](const double4& c) {
+        const double ddx = c.x - prx, ddy = c.y - pry, ddz = c.z - prz;
+        return ddx * ddx + ddy * ddy + ddz * ddz;
+    };
+    auto consts = [&](const double4& c, int k) {
+        if constexpr (GRAD) return pt;
+        else return s_lj[(F32 ? unpack_t(c.w) : L.t[k]) + site];
+    };
+    const PairSums<Real> S0 = S;
+    Real m = (Real)INFINITY;
+    constexpr int PAIR_UNROLL = F32 ? 2 : 1;
+#pragma unroll PAIR_UNROLL
+    for (int j = j0; j < je; ++j) {
+        const double4 c = L.c[j];
+        const float qf = F32 ? unpack_q(c.w) : 0.0f;  // the FP64 terms take c.w
+        const Real u = pair_term<ESM, Real, GRAD, false>(dist2(c), c.w, qf, consts(c, j), is_lj, r2lj, r2sr, et, ovl, S);
+        if constexpr (F32) m = fminf(m, u);
+        else m = fmin(m, u);
+    }
+    // an overlap: r^2 below R2_OVERLAP and inside the LJ cutoff
+    const double thr = fmin(R2_OVERLAP, r2lj);
+    bool redo;
+    if constexpr (F32) {
+        ovl |= is_lj & (m < (float)thr * (1.0f - 1e-6f));
+        redo = m < 1e-37f || (m >= (float)thr * (1.0f - 1e-6f) && m <= (float)thr * (1.0f + 1e-6f));
+    } else {
+        ovl |= is_lj & (m < thr);
+        redo = m < 2.2250738585072014e-308;
+    }
+    if (__builtin_expect(__ballot(redo) != 0ull, 0)) {
+        S = S0;
+#pragma unroll 1
+        for (int j = j0; j < je; ++j) {
+            const double4 c = L.c[j];
+            const float qf = F32 ? unpack_q(c.w) : 0.0f;
+            pair_term<ESM, Real, GRAD, true>(dist2(c), c.w, qf, consts(c, j), is_lj, r2lj, r2sr, et, ovl, S);
+        }
+    }
+}
+
 // Per-type derivative sums of a gradient run's point, FP64, for NT framework
-// types: g[k] = sum (u^2 - u) (d LJ / d eps_ts = 4 of it), g[NT + k] =
-// d LJ / d sigma_ts, g[2 NT + k] = sum erfc(alpha r) / r.  A run of candidates
-// of one type accumulates in Real (pair_term_grad's sw, su, sq) and is folded
-// in here once.  The image-list path folds with the type known at compile time
-// (add), the all-atoms path with the type in a register (add_dyn, every entry
-// updated: a conditional update of one entry would be folded into a
-// dynamically indexed array held in scratch memory).
+// types: g[k] = sum (u^2 - u) (u = sigma_ts^6 / r^6; d LJ / d eps_ts = 4 of it),
+// g[NT + k] = d LJ / d sigma_ts = (4 eps_ts / sigma_ts) sum (12 u^2 - 6 u),
+// g[2 NT + k] = sum erfc(alpha r) / r.  A run of candidates of one type
+// accumulates in Real (PairSums' s1, s2, sq) and is folded in here once, with
+// gc = (sigma_ts^6, 4 eps_ts / sigma_ts).  The image-list path folds with the
+// type known at compile time (add), the all-atoms path with the type in a
+// register (add_dyn, every entry updated: a conditional update of one entry
+// would be folded into a dynamically indexed array held in scratch memory).
 template <typename Real, int NT>
 struct TypeSums {
     double g[3 * NT];
-    // the all-atoms path: the type (times nsite) being summed and its sums
+    // the all-atoms path: the type (times nsite) being summed
     int cur = -1;
-    Real sw = (Real)0, su = (Real)0, sq = (Real)0, csig = (Real)0;
+    double2 gc = make_double2(0.0, 0.0);
     __device__ TypeSums() {
 #pragma unroll
         for (int k = 0; k < 3 * NT; ++k) g[k] = 0.0;
     }
-    __device__ __attribute__((always_inline)) inline void add(int k, Real w, Real u, Real q, Real cs, bool is_lj) {
-        g[k] += is_lj ? (double)w : 0.0;
-        g[NT + k] += is_lj ? (double)cs * (12.0 * (double)w + 6.0 * (double)u) : 0.0;
-        g[2 * NT + k] += (double)q;
+    // sums of u^2 - u and 12 u^2 - 6 u of a run
+    __device__ static inline double2 sums(const PairSums<Real>& S, double2 c) {
+        if constexpr (sizeof(Real) == 4) {
+            return make_double2((double)S.s1, 12.0 * (double)S.s1 + 6.0 * (double)S.s2);
+        } else {
+            const double v = c.x * S.s2, w = c.x * c.x * S.s1;
+            return make_double2(w - v, 12.0 * w - 6.0 * v);
+        }
     }
-    __device__ __attribute__((always_inline)) inline void add_dyn(int t, bool is_lj) {
-        const double e = is_lj ? (double)sw : 0.0;
-        const double d = is_lj ? (double)csig * (12.0 * (double)sw + 6.0 * (double)su) : 0.0;
-        const double c = (double)sq;
+    __device__ __attribute__((always_inline)) inline void add(int k, const PairSums<Real>& S, double2 c, bool is_lj) {
+        const double2 e = sums(S, c);
+        g[k] += is_lj ? e.x : 0.0;
+        g[NT + k] += is_lj ? c.y * e.y : 0.0;
+        g[2 * NT + k] += (double)S.sq;
+    }
+    __device__ __attribute__((always_inline)) inline void add_dyn(int t, PairSums<Real>& S, bool is_lj) {
+        const double2 f = sums(S, gc);
+        const double e = is_lj ? f.x : 0.0;
+        const double d = is_lj ? gc.y * f.y : 0.0;
+        const double c = (double)S.sq;
 #pragma unroll
         for (int k = 0; k < NT; ++k) {
             g[k] += (k == t) ? e : 0.0;
             g[NT + k] += (k == t) ? d : 0.0;
             g[2 * NT + k] += (k == t) ? c : 0.0;
         }
-        sw = su = sq = (Real)0;
+        S.s1 = S.s2 = S.sq = (Real)0;
     }
-    // all-atoms path: a candidate of type tt (times nsite) with d/d sigma factor cs
-    __device__ __attribute__((always_inline)) inline void type(int tt, int nsite, Real cs, bool is_lj) {
+    // all-atoms path: a candidate of type tt (times nsite) with fold constants c
+    __device__ __attribute__((always_inline)) inline void type(int tt, int nsite, double2 c, PairSums<Real>& S,
+                                                               bool is_lj) {
         if (tt != cur) {
-            if (cur >= 0) add_dyn(cur / nsite, is_lj);
+            if (cur >= 0) add_dyn(cur / nsite, S, is_lj);
             cur = tt;
-            csig = cs;
+            gc = c;
         }
     }
-    __device__ __attribute__((always_inline)) inline void flush(int nsite, bool is_lj) {
-        if (cur >= 0) add_dyn(cur / nsite, is_lj);
+    __device__ __attribute__((always_inline)) inline void flush(int nsite, PairSums<Real>& S, bool is_lj) {
+        if (cur >= 0) add_dyn(cur / nsite, S, is_lj);
     }
 };
 
@@ -708,7 +776,7 @@ struct TypeSums {
 // registers and folded into the type's FP64 sums once.
 template <int ESM, typename Real, int NT>
 __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs& a, bool valid, double px, double py, double pz,
-                                   int site, const LJP<Real>* s_lj, const Real* s_gc,
+                                   int site, const LJC<Real>* s_lj, const double2* s_gc,
                                    PairLds L, double& acc_lj, double& acc_sr, bool& ovl, unsigned long long& n_cand,
                                    TypeSums<Real, (NT > 0 ? NT : 1)>& ts) {
     constexpr bool GRAD = NT > 0;
@@ -725,7 +793,8 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
         // The point and the chunk centre in Cartesian coordinates (FP64).  The
         // images are stored in Cartesian coordinates, so a pair's r^2 depends
         // on the point and the image alone, not on the chunk it was found from.
-        const double prx = f11 * px + f12 * py + f13 * pz;
+        // (a lane without a point is put far from every image)
+        const double prx = valid ? f11 * px + f12 * py + f13 * pz : 1e8;
         const double pry = f22 * py + f23 * pz;
         const double prz = f33 * pz;
         // The workgroup's sphere: the centre of its valid points' bounding box
@@ -843,7 +912,7 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                         // from one scalar word per tile
                         int j = 0;
                         for (int gi = 0; gi < WG / 64; ++gi) {
-                            Real plj = (Real)0, psr = (Real)0;
+                            PairSums<Real> S;
                             const int j0 = j;
                             const unsigned long long ends =
                                 (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(L.ends[2 * gi]) |
@@ -853,43 +922,25 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                             for (int k = 0; k < NT; ++k) {
                                 const int je = j0 + (int)((ends >> (7 * k)) & 127ull);
                                 if (je == j) continue;
-                                const LJP<Real> p = s_lj[k * nsite + site];
-                                const Real cs = s_gc[k * nsite + site];
-                                Real sw = (Real)0, su = (Real)0, sq = (Real)0;
-#pragma unroll 2
-                                for (; j < je; ++j) {
-                                    const double4 c = L.c[j];
-                                    const double ddx = c.x - prx, ddy = c.y - pry, ddz = c.z - prz;
-                                    const double r2 = ddx * ddx + ddy * ddy + ddz * ddz;
-                                    const float qj = sizeof(Real) == 4 ? unpack_q(c.w) : 0.0f;
-                                    pair_term_grad<ESM, Real>(r2, c.w, qj, p, is_lj, r2lj, r2sr, et, ovl, plj, psr, sw,
-                                                              su, sq);
-                                }
-                                ts.add(k, sw, su, sq, cs, is_lj);
+                                const LJC<Real> p = s_lj[k * nsite + site];
+                                S.s1 = S.s2 = S.sq = (Real)0;
+                                pair_loop<ESM, Real, true>(L, j, je, prx, pry, prz, site, s_lj, p, is_lj, r2lj, r2sr,
+                                                           et, ovl, S);
+                                j = je;
+                                ts.add(k, S, s_gc[k * nsite + site], is_lj);
                             }
-                            acc_lj += (double)plj;
-                            acc_sr += (double)psr;
+                            acc_lj += (double)S.plj;
+                            acc_sr += (double)S.psr;
                         }
                     } else {
                         // the candidates of each tile accumulate in Real, flushed to FP64
 #pragma unroll
                         for (int gi = 0; gi < WG / 64; ++gi) {
-                            Real plj = (Real)0, psr = (Real)0;
-                            // two candidates per iteration share the LDS address registers (FP32 energies)
-                            constexpr int PAIR_UNROLL = sizeof(Real) == 4 ? 2 : 1;
-#pragma unroll PAIR_UNROLL
-                            for (int j = woff[gi]; j < woff[gi + 1]; ++j) {
-                                const double4 c = L.c[j];
-                                const double ddx = c.x - prx, ddy = c.y - pry, ddz = c.z - prz;
-                                const double r2 = ddx * ddx + ddy * ddy + ddz * ddz;
-                                const bool f32 = sizeof(Real) == 4;
-                                const int tj = f32 ? unpack_t(c.w) : L.t[j];
-                                const float qj = f32 ? unpack_q(c.w) : 0.0f;  // the FP64 terms take c.w
-                                pair_term<ESM, Real>(r2, c.w, qj, s_lj[tj + site], is_lj, r2lj, r2sr, et, ovl, plj,
-                                                     psr);
-                            }
-                            acc_lj += (double)plj;
-                            acc_sr += (double)psr;
+                            PairSums<Real> S;
+                            pair_loop<ESM, Real, false>(L, woff[gi], woff[gi + 1], prx, pry, prz, site, s_lj,
+                                                        LJC<Real>{}, is_lj, r2lj, r2sr, et, ovl, S);
+                            acc_lj += (double)S.plj;
+                            acc_sr += (double)S.psr;
                         }
                     }
                 }
@@ -909,7 +960,7 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
             n_cand += (unsigned long long)nt;
             if (wave_live) {
                 for (int gi = 0; gi < nt; gi += 64) {
-                    Real plj = (Real)0, psr = (Real)0;
+                    PairSums<Real> S;
                     const int ge = min(nt, gi + 64);
                     for (int j = gi; j < ge; ++j) {
                         const double4 at = L.c[j];
@@ -921,33 +972,33 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                         const double cy = f22 * ey + f23 * ez;
                         const double cz = f33 * ez;
                         const double r2 = cx * cx + cy * cy + cz * cz;
+                        LJC<Real> p;
                         if constexpr (GRAD) {
                             const int tt = __builtin_amdgcn_readfirstlane(L.t[j]);
-                            ts.type(tt, nsite, s_gc[tt + site], is_lj);
-                            pair_term_grad<ESM, Real>(r2, at.w, L.qf[j], s_lj[tt + site], is_lj, r2lj, r2sr, et,
-                                                      ovl, plj, psr, ts.sw, ts.su, ts.sq);
+                            ts.type(tt, nsite, s_gc[tt + site], S, is_lj);
+                            p = s_lj[tt + site];
                         } else {
-                            pair_term<ESM, Real>(r2, at.w, L.qf[j], s_lj[L.t[j] + site], is_lj, r2lj, r2sr, et, ovl,
-                                                 plj, psr);
+                            p = s_lj[L.t[j] + site];
                         }
+                        pair_term<ESM, Real, GRAD, true>(r2, at.w, L.qf[j], p, is_lj, r2lj, r2sr, et, ovl, S);
                     }
-                    acc_lj += (double)plj;
-                    acc_sr += (double)psr;
-                    if constexpr (GRAD) ts.flush(nsite, is_lj);  // FP64 per 64 candidates, as the energies
+                    acc_lj += (double)S.plj;
+                    acc_sr += (double)S.psr;
+                    if constexpr (GRAD) ts.flush(nsite, S, is_lj);  // FP64 per 64 candidates, as the energies
                 }
             }
         }
     }
-    if constexpr (GRAD) ts.flush(nsite, is_lj);
 }
 
 // LDS: TILE candidate records, types and FP32 charges, the selected-tile list,
-// the erfc table (FP32 cubics or FP64 quintics), then the LJ table of the run
-// (and for a gradient run its d/d sigma factors).
+// the erfc table (FP32 cubics or FP64 quintics), the small per-wave arrays, then
+// the LJ table of the run (and for a gradient run its fold constants).
+constexpr int PAIR_LDS_SMALL = (WG / 64) * 80;  // sphere partials, run ends, candidate counts
 template <typename Real>
 constexpr int pair_lds_fixed() {
-    return TILE * (int)(sizeof(double4) + sizeof(int) + sizeof(float) + sizeof(int)) +
-           (sizeof(Real) == 4 ? ERFC_SEG * (int)sizeof(float4) : 3 * ERFC64_SEG * (int)sizeof(double2));
+    return PAIR_LDS_SMALL + TILE * (int)(sizeof(double4) + sizeof(int) + sizeof(float) + sizeof(int)) +
+           (sizeof(Real) == 4 ? ERFC_TAB * (int)sizeof(float4) : ERFC64_TAB * (int)sizeof(double2));
 }
 
 // NT = 0: energies.  NT > 0: a gradient run of at most NT framework types.
@@ -955,9 +1006,6 @@ template <typename Real, int NT>
 __global__ __launch_bounds__(WG) void point_pair_kernel(GroupArgs g) {
     constexpr bool GRAD = NT > 0;
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ int s_wcnt[WG / 64];
-    __shared__ unsigned s_ends[(WG / 64) * 2];
-    __shared__ double s_sph[(WG / 64) * 8];
     PairLds L;
     L.c = reinterpret_cast<double4*>(smem);
     L.t = reinterpret_cast<int*>(smem + TILE * sizeof(double4));
@@ -967,10 +1015,13 @@ __global__ __launch_bounds__(WG) void point_pair_kernel(GroupArgs g) {
     L.erfc = s_erfc;
     double2* s_erfc64 = reinterpret_cast<double2*>(s_erfc);
     L.erfc64 = s_erfc64;
-    L.wcnt = s_wcnt;
-    L.ends = s_ends;
-    L.sph = s_sph;
-    LJP<Real>* s_lj = reinterpret_cast<LJP<Real>*>(smem + pair_lds_fixed<Real>());
+    // (all LDS is dynamic: it then starts at address 0, and the table reads
+    // carry their whole base in the instruction's offset)
+    unsigned char* small = smem + pair_lds_fixed<Real>() - PAIR_LDS_SMALL;
+    L.sph = reinterpret_cast<double*>(small);
+    L.ends = reinterpret_cast<unsigned*>(small + (WG / 64) * 8 * sizeof(double));
+    L.wcnt = reinterpret_cast<int*>(small + (WG / 64) * (8 * sizeof(double) + 2 * sizeof(unsigned)));
+    LJC<Real>* s_lj = reinterpret_cast<LJC<Real>*>(smem + pair_lds_fixed<Real>());
 
     const int tid = threadIdx.x;
     int si;
@@ -984,7 +1035,8 @@ __global__ __launch_bounds__(WG) void point_pair_kernel(GroupArgs g) {
     }
     const SegArgs sg = g.segs[si];
     const RunArgs& a = g.runs[sg.run];
-    Real* s_gc = reinterpret_cast<Real*>(s_lj + a.n_types * a.nsite);
+    // (16-byte aligned: the LJ table's entries are 8 or 16 bytes)
+    double2* s_gc = reinterpret_cast<double2*>(s_lj + ((a.n_types * a.nsite + 1) & ~1));
 
     bool valid;
     long long pid;
@@ -1013,18 +1065,18 @@ __global__ __launch_bounds__(WG) void point_pair_kernel(GroupArgs g) {
         site = 0;
     }
     const int n_tab = a.n_types * a.nsite;
-    const LJP<Real>* gtab = reinterpret_cast<const LJP<Real>*>(a.ljtab);
+    const LJC<Real>* gtab = reinterpret_cast<const LJC<Real>*>(a.ljtab);
     for (int t = tid; t < n_tab; t += WG) s_lj[t] = gtab[t];
     if constexpr (GRAD) {
-        const Real* gc = reinterpret_cast<const Real*>(a.gtab);
+        const double2* gc = reinterpret_cast<const double2*>(a.gtab);
         for (int t = tid; t < n_tab; t += WG) s_gc[t] = gc[t];
     }
     if constexpr (sizeof(Real) == 4)
         if (a.esm != 0)
-            for (int t = tid; t < ERFC_SEG; t += WG) s_erfc[t] = a.erfc_tab[t];
+            for (int t = tid; t < ERFC_TAB; t += WG) s_erfc[t] = a.erfc_tab[t];
     if constexpr (sizeof(Real) == 8)
         if (a.esm != 0)
-            for (int t = tid; t < 3 * ERFC64_SEG; t += WG) s_erfc64[t] = a.erfc64_tab[t];
+            for (int t = tid; t < ERFC64_TAB; t += WG) s_erfc64[t] = a.erfc64_tab[t];
 
     double acc_lj = 0.0, acc_sr = 0.0;
     bool ovl = false;

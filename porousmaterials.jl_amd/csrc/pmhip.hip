@@ -316,8 +316,8 @@ struct pm_ewald {
     int Ma = 0, Mb = 0, Mc = 0;
     double2* d_box = nullptr;
     int2* d_rows = nullptr;    // per (ma, mb) row of the box: kept mc range (lo > hi: empty)
-    float4* d_erfc = nullptr;  // ERFC_SEG cubics of erfc(alpha r) on [0, sr_cutoff]
-    double2* d_erfc64 = nullptr;  // ERFC64_SEG quintics of erfc(alpha r) on [0, sr_cutoff] (FP64)
+    float4* d_erfc = nullptr;  // cubics of erfc(alpha r) on [0, sr_cutoff] (FP32)
+    double2* d_erfc64 = nullptr;  // quintics of erfc(alpha r) about the multiples of sr_cutoff / ERFC64_SEG (FP64)
     double2* d_box_t = nullptr;  // per-type boxes (gradient runs), built on first use
 };
 
@@ -376,6 +376,22 @@ void build_ljtab(const pm_framework* fw, const pm_forcefield* ff, int ns, const 
                 p.eps4 = (Real)(4.0 * ff->eps[idx]);
             }
             t[i * ns + s] = p;
+        }
+}
+
+// The FP64 point engine's form of the same table (a = 4 eps sigma^12, b =
+// 4 eps sigma^6; zero for a site without an LJ sphere).
+void build_ljab(const pm_framework* fw, const pm_forcefield* ff, int ns, const Site* site,
+                const int32_t* site_species, std::vector<unsigned char>& out) {
+    const int nt = (int)fw->species_global.size();
+    out.assign(sizeof(LJAB) * (size_t)std::max(nt, 1) * ns, 0);
+    LJAB* t = reinterpret_cast<LJAB*>(out.data());
+    for (int i = 0; i < nt; ++i)
+        for (int s = 0; s < ns; ++s) {
+            if (!site[s].lj || ff == nullptr) continue;
+            const size_t idx = (size_t)fw->species_global[i] * ff->n + site_species[s];
+            const double s6 = ff->sig2[idx] * ff->sig2[idx] * ff->sig2[idx], b = 4.0 * ff->eps[idx] * s6;
+            t[i * ns + s] = LJAB{b * s6, b};
         }
 }
 
@@ -1128,11 +1144,11 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
     std::vector<long long> part_off(n_runs), grid_off(n_runs);
     for (int i = 0; i < n_runs; ++i) {
         PointRun& r = runs[i];
-        if (fp64) build_ljtab<double>(r.fw, r.ff, r.ns, r.pr->site, r.pr->lj_species, r.tab);
+        if (fp64) build_ljab(r.fw, r.ff, r.ns, r.pr->site, r.pr->lj_species, r.tab);
         else build_ljtab<float>(r.fw, r.ff, r.ns, r.pr->site, r.pr->lj_species, r.tab);
         r.tab_off = tab_total;
         tab_total += align256(r.tab.size());
-        lj_lds = std::max(lj_lds, r.tab.size() + (grad ? r.gtab.size() : 0));
+        lj_lds = std::max(lj_lds, (r.tab.size() + 15) / 16 * 16 + (grad ? r.gtab.size() : 0));
         if (grad) {
             r.gtab_off = tab_total;
             tab_total += align256(r.gtab.size());
@@ -1449,6 +1465,55 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
     return PM_OK;
 }
 
+// The FP32 path's table of erfc(alpha r): cubic Hermite segments on [0,
+// sr_cutoff], h = sr_cutoff / ERFC_SEG, in t = r/h - i: c0 + c1 t + c2 t^2 +
+// c3 t^3 matches erfc and its derivative at both ends (interpolation error <=
+// h^4 max|f^(4)| / 384); the last entry is the value at sr_cutoff.
+void build_erfc_table(double alpha, double sr_cutoff, float4* tab) {
+    const double h = sr_cutoff / ERFC_SEG;
+    const double dscale = -2.0 * alpha / std::sqrt(M_PI);
+    double f0 = 1.0, d0 = h * dscale;
+    for (int i = 0; i < ERFC_SEG; ++i) {
+        const double r1 = (i + 1) * h;
+        const double f1 = std::erfc(alpha * r1), d1 = h * dscale * std::exp(-alpha * alpha * r1 * r1);
+        tab[i] = make_float4((float)f0, (float)d0, (float)(3.0 * (f1 - f0) - 2.0 * d0 - d1),
+                             (float)(2.0 * (f0 - f1) + d0 + d1));
+        f0 = f1;
+        d0 = d1;
+    }
+    tab[ERFC_SEG] = make_float4((float)f0, 0.0f, 0.0f, 0.0f);
+}
+
+// The FP64 path's table of erfc(alpha r): the degree-5 Taylor expansions about
+// r = i h, i = 0..ERFC64_SEG, h = sr_cutoff / ERFC64_SEG, in t = r/h - i,
+// |t| <= 1/2: f^(k)(r) h^k / k! with f^(k)(r) = alpha^k erfc^(k)(alpha r),
+// erfc^(k)(x) = -(2/sqrt(pi)) (-1)^(k-1) H_(k-1)(x) e^(-x^2) (Hermite
+// polynomials); truncation error <= (h/2)^6 max|f^(6)| / 720, below 1e-15 for
+// alpha h <= 0.01 (alpha r_c is about 3 to 4 for Ewald precisions 1e-6 to
+// 1e-8).  Evaluated in long double, stored as (c0, c1), (c2, c3), (c4, c5).
+void build_erfc64_table(double alpha, double sr_cutoff, double2* tab) {
+    const long double h = (long double)sr_cutoff / ERFC64_SEG, al = alpha;
+    const long double two_rpi = 2.0L / std::sqrt((long double)M_PI);
+    for (int i = 0; i <= ERFC64_SEG; ++i) {
+        const long double x = al * h * i;
+        long double H[5];  // H_n(x), n = 0..4: H_(n+1) = 2x H_n - 2n H_(n-1)
+        H[0] = 1.0L;
+        H[1] = 2.0L * x;
+        for (int n = 1; n < 4; ++n) H[n + 1] = 2.0L * x * H[n] - 2.0L * n * H[n - 1];
+        const long double g = std::exp(-x * x);
+        long double d[6];  // f^(k)(r_i) h^k / k!
+        d[0] = std::erfc(x);
+        long double scale = 1.0L;  // (alpha h)^k / k!
+        for (int k = 1; k <= 5; ++k) {
+            scale *= al * h / k;
+            d[k] = -two_rpi * ((k - 1) % 2 ? -1.0L : 1.0L) * H[k - 1] * g * scale;
+        }
+        tab[3 * i] = make_double2((double)d[0], (double)d[1]);
+        tab[3 * i + 1] = make_double2((double)d[2], (double)d[3]);
+        tab[3 * i + 2] = make_double2((double)d[4], (double)d[5]);
+    }
+}
+
 // Per-type Fourier boxes of an Ewald handle (gradient runs), built once: the
 // structure factor of each framework species with unit charges on every atom
 // of that species, on the handle's kept k-vectors.
@@ -1485,34 +1550,28 @@ int ensure_type_boxes(pm_ewald* ew, const pm_framework* fw) {
 }
 
 // Gradient tables of a prepared Widom run: per (compact type t, site s) the
-// factor 4 eps_ts / sigma_ts of d LJ / d sigma_ts (in the pair precision) and
-// the mixing-rule Jacobian from jac[(i * n + j) * 4 + k] (i framework
+// fold constants (sigma_ts^6, 4 eps_ts / sigma_ts) and the mixing-rule Jacobian from jac[(i * n + j) * 4 + k] (i framework
 // species, j probe species, k: d eps_ij/d eps_i, d eps_ij/d sigma_i,
 // d sigma_ij/d eps_i, d sigma_ij/d sigma_i).
-void fill_gradient_tables(PointRun& r, const double* jac, bool fp64) {
+void fill_gradient_tables(PointRun& r, const double* jac) {
     const pm_framework* fw = r.fw;
     const pm_forcefield* ff = r.ff;
     const int nt = (int)fw->species_global.size(), ns = r.ns, n = ff->n;
     r.jac.assign((size_t)std::max(nt, 1) * ns, make_double4(0.0, 0.0, 0.0, 0.0));
-    std::vector<double> gc((size_t)std::max(nt, 1) * ns, 0.0);
+    std::vector<double2> gc((size_t)std::max(nt, 1) * ns, make_double2(0.0, 0.0));
     for (int t = 0; t < nt; ++t)
         for (int s = 0; s < ns; ++s) {
             if (!r.pr->site[s].lj) continue;
             const int i = fw->species_global[t], j = r.pr->lj_species[s];
             const size_t idx = (size_t)i * n + j;
             const double sg = std::sqrt(ff->sig2[idx]);
-            gc[(size_t)t * ns + s] = sg > 0.0 ? 4.0 * ff->eps[idx] / sg : 0.0;
+            const double s2 = ff->sig2[idx];
+            gc[(size_t)t * ns + s] = make_double2(s2 * s2 * s2, sg > 0.0 ? 4.0 * ff->eps[idx] / sg : 0.0);
             const double* J = jac + 4 * idx;
             r.jac[(size_t)t * ns + s] = make_double4(J[0], J[1], J[2], J[3]);
         }
-    if (fp64) {
-        r.gtab.resize(gc.size() * sizeof(double));
-        std::memcpy(r.gtab.data(), gc.data(), r.gtab.size());
-    } else {
-        std::vector<float> f(gc.begin(), gc.end());
-        r.gtab.resize(f.size() * sizeof(float));
-        std::memcpy(r.gtab.data(), f.data(), r.gtab.size());
-    }
+    r.gtab.resize(gc.size() * sizeof(double2));
+    std::memcpy(r.gtab.data(), gc.data(), r.gtab.size());
 }
 
 }  // namespace
@@ -1749,63 +1808,10 @@ int pm_ewald_create(const pm_framework* fw, double alpha, double sr_cutoff, int6
         (void)hipFree(d_m); (void)hipFree(d_w);
         delete ew;
     };
-    // Cubic Hermite segments of erfc(alpha r) on [0, sr_cutoff], h = sr_cutoff /
-    // ERFC_SEG, in t = r/h - i: c0 + c1 t + c2 t^2 + c3 t^3 matches erfc and its
-    // derivative at both ends (interpolation error <= h^4 max|f''''| / 384).
-    std::vector<float4> etab(ERFC_SEG);
-    {
-        const double h = sr_cutoff / ERFC_SEG;
-        const double dscale = -2.0 * alpha / std::sqrt(M_PI);
-        for (int i = 0; i < ERFC_SEG; ++i) {
-            const double r0 = i * h, r1 = (i + 1) * h;
-            const double f0 = std::erfc(alpha * r0), f1 = std::erfc(alpha * r1);
-            const double d0 = h * dscale * std::exp(-alpha * alpha * r0 * r0);
-            const double d1 = h * dscale * std::exp(-alpha * alpha * r1 * r1);
-            etab[i] = make_float4((float)f0, (float)d0, (float)(3.0 * (f1 - f0) - 2.0 * d0 - d1),
-                                  (float)(2.0 * (f0 - f1) + d0 + d1));
-        }
-    }
-    // FP64 path: degree-5 segments of f(r) = erfc(alpha r) on [0, sr_cutoff],
-    // h = sr_cutoff / ERFC64_SEG, in t = r/h - i, from the Taylor expansion about
-    // the segment's midpoint m (in u = t - 1/2: sum_k f^(k)(m) h^k u^k / k!),
-    // re-expanded in powers of t.  f^(k)(r) = alpha^k erfc^(k)(alpha r) with
-    // erfc^(k)(x) = -(2/sqrt(pi)) (-1)^(k-1) H_(k-1)(x) e^(-x^2) (Hermite
-    // polynomials); truncation error <= (h/2)^6 max|f^(6)| / 720, below 1e-15
-    // for alpha h <= 0.01 (alpha r_c is about 3 to 4 for Ewald precisions
-    // 1e-6 to 1e-8).  Evaluated in long double, stored as (c0, c1), (c2, c3),
-    // (c4, c5).
-    std::vector<double2> etab64(3 * ERFC64_SEG);
-    {
-        const long double h = (long double)sr_cutoff / ERFC64_SEG, al = alpha;
-        const long double two_rpi = 2.0L / std::sqrt((long double)M_PI);
-        for (int i = 0; i < ERFC64_SEG; ++i) {
-            const long double x = al * h * (i + 0.5L);
-            long double H[5];  // H_n(x), n = 0..4: H_(n+1) = 2x H_n - 2n H_(n-1)
-            H[0] = 1.0L;
-            H[1] = 2.0L * x;
-            for (int n = 1; n < 4; ++n) H[n + 1] = 2.0L * x * H[n] - 2.0L * n * H[n - 1];
-            const long double g = std::exp(-x * x);
-            long double d[6];  // f^(k)(m) h^k / k!
-            d[0] = std::erfc(x);
-            long double scale = 1.0L;  // (alpha h)^k / k!
-            for (int k = 1; k <= 5; ++k) {
-                scale *= al * h / k;
-                d[k] = -two_rpi * ((k - 1) % 2 ? -1.0L : 1.0L) * H[k - 1] * g * scale;
-            }
-            long double c[6] = {0.0L, 0.0L, 0.0L, 0.0L, 0.0L, 0.0L};
-            for (int k = 0; k <= 5; ++k) {
-                long double binom = 1.0L, pw = 1.0L;  // C(k, j) (-1/2)^(k-j), from j = k down
-                for (int j = k; j >= 0; --j) {
-                    c[j] += d[k] * binom * pw;
-                    binom = binom * j / (k - j + 1);
-                    pw *= -0.5L;
-                }
-            }
-            etab64[3 * i] = make_double2((double)c[0], (double)c[1]);
-            etab64[3 * i + 1] = make_double2((double)c[2], (double)c[3]);
-            etab64[3 * i + 2] = make_double2((double)c[4], (double)c[5]);
-        }
-    }
+    std::vector<float4> etab(ERFC_TAB);
+    build_erfc_table(alpha, sr_cutoff, etab.data());
+    std::vector<double2> etab64(ERFC64_TAB);
+    build_erfc64_table(alpha, sr_cutoff, etab64.data());
     // kept mc range of every (ma, mb) row of the box
     const size_t n_rows = (size_t)(Ma + 1) * (2 * Mb + 1);
     std::vector<int2> rows(n_rows, make_int2(1, 0));
@@ -1816,8 +1822,8 @@ int pm_ewald_create(const pm_framework* fw, double alpha, double sr_cutoff, int6
         else r = make_int2(std::min(r.x, mc), std::max(r.y, mc));
     }
     if (hipMalloc(&ew->d_rows, n_rows * sizeof(int2)) != hipSuccess ||
-        hipMalloc(&ew->d_erfc, ERFC_SEG * sizeof(float4)) != hipSuccess ||
-        hipMalloc(&ew->d_erfc64, 3 * ERFC64_SEG * sizeof(double2)) != hipSuccess ||
+        hipMalloc(&ew->d_erfc, ERFC_TAB * sizeof(float4)) != hipSuccess ||
+        hipMalloc(&ew->d_erfc64, ERFC64_TAB * sizeof(double2)) != hipSuccess ||
         hipMalloc(&ew->d_box, box_n * sizeof(double2)) != hipSuccess ||
         hipMalloc(&ew->d_k, std::max<size_t>(ew->nk, 1) * sizeof(KVec)) != hipSuccess ||
         hipMalloc(&d_m, std::max<size_t>(m.size(), 1) * sizeof(int)) != hipSuccess ||
@@ -1827,10 +1833,10 @@ int pm_ewald_create(const pm_framework* fw, double alpha, double sr_cutoff, int6
     }
     hipError_t e = hipMemsetAsync(ew->d_box, 0, box_n * sizeof(double2), g_ctx.stream);
     if (e == hipSuccess)
-        e = hipMemcpyAsync(ew->d_erfc, etab.data(), ERFC_SEG * sizeof(float4), hipMemcpyHostToDevice,
+        e = hipMemcpyAsync(ew->d_erfc, etab.data(), ERFC_TAB * sizeof(float4), hipMemcpyHostToDevice,
                            g_ctx.stream);
     if (e == hipSuccess)
-        e = hipMemcpyAsync(ew->d_erfc64, etab64.data(), 3 * ERFC64_SEG * sizeof(double2), hipMemcpyHostToDevice,
+        e = hipMemcpyAsync(ew->d_erfc64, etab64.data(), ERFC64_TAB * sizeof(double2), hipMemcpyHostToDevice,
                            g_ctx.stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(ew->d_rows, rows.data(), n_rows * sizeof(int2), hipMemcpyHostToDevice, g_ctx.stream);
@@ -2183,7 +2189,7 @@ int pm_widom_gradient(const pm_framework* fw, const pm_forcefield* ff, const pm_
         r.ra.A_t = r.ew->d_box_t;
     }
     r.ra.n_gt = nt;
-    fill_gradient_tables(r, jac, precision == PM_FP64);
+    fill_gradient_tables(r, jac);
     std::vector<double> gs((size_t)n_blocks * 3 * GT, 0.0);
     if (int rc = execute_points(runs, MODE_WIDOM, precision, out_block_sums, true, gs.data())) return rc;
     for (int64_t k = 0; k < (int64_t)n_blocks * ff->n * 3; ++k) out_block_grads[k] = 0.0;
