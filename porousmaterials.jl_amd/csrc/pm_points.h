@@ -65,8 +65,9 @@ struct RunArgs {
     int fast;                // the image list covers r_cmax + chunk_r around every chunk
     int nsite, n_types, n_img, n_atoms, n_tiles;
     unsigned site_lj_mask, site_q_mask;
-    const double4* img;      // images near the box: Cartesian xyz (A) + charge, in spatial tiles
-    const int* img_type;
+    const double4* img;      // images near the box, in spatial tiles: Cartesian xyz (A), and the charge (FP64 runs)
+                             // or the type and FP32 charge (mixed runs); 64 more at the end
+    const int* img_type;     // compact type
     const double4* tile_sph; // per tile: bounding-sphere centre (Cartesian) and radius
     const int2* tile_rng;    // per tile: first image, image count (<= 64)
     const double4* atoms;    // replicated atoms (fallback path)
@@ -534,7 +535,7 @@ struct PairSums {
 // - a pair outside the cutoff is masked once, through its 1/r (every masked
 //   term is then an exact zero and reads a valid table entry), not term by
 //   term; the overlap test is left to the caller, who follows the smallest r^2
-//   of a tile's candidates (pair_loop) instead of comparing every pair;
+//   of a tile's candidates (tile_close) instead of comparing every pair;
 // - FP64: 1/r by v_rsq_f64 and one third-order step, y (1 + e/2 + 3 e^2/8) with
 //   e = 1 - r^2 y^2 (the estimate's 2^-22 cubes to below an ulp); index and
 //   offset of the table by the addition of 1.5 2^52 in place of conversions.
@@ -624,82 +625,143 @@ __device__ __attribute__((always_inline)) inline Real pair_term(double r2, doubl
     }
 }
 
-// FP32 kernels pack a candidate's type offset (high word) and FP32 charge
-// (low word) into the fourth double of its record, so one 32-byte LDS record
-// carries the candidate (raw bits: no arithmetic touches the packed value).
-__device__ inline double pack_tq(int t, float q) {
-    return __longlong_as_double((long long)(((unsigned long long)(unsigned)t << 32) | (unsigned)__float_as_int(q)));
-}
+// The image list as the pair loops read it: Cartesian xyz, and in the fourth
+// double FP32 kernels take the image's type (high word) and FP32 charge (low
+// word), FP64 kernels its charge and the type from an array of its own.  A
+// candidate's record is the same for every lane, so it comes in by scalar
+// loads, as SGPR operands.
+typedef double vd4 __attribute__((ext_vector_type(4)));
 __device__ inline int unpack_t(double w) { return (int)(__double_as_longlong(w) >> 32); }
 __device__ inline float unpack_q(double w) { return __int_as_float((int)__double_as_longlong(w)); }
 
-struct PairLds {
-    double4* c;     // candidate records: Cartesian xyz; charge (FP64 kernels) or packed type and charge
-    int* t;         // candidate type * nsite
-    float* qf;      // candidate charge in FP32
-    int* sel;       // selected tiles of the current batch
-    unsigned* ends; // gradient runs: per wave's tile, the cumulative kept candidates of types 0..k,
-                    // 7 bits per type (two words)
-    const float4* erfc;    // FP32 kernels
-    const double2* erfc64;  // FP64 kernels
-    int* wcnt;      // per-wave candidate counts
-    double* sph;    // per-wave bounding-box and radius partials of the workgroup's sphere
+// The candidates of one tile, the set bits of a mask over its images, in list
+// order, two ahead of their use.  Beyond the last one it reads the record 63
+// after the tile's first, whose value is not used (the list ends with
+// TILE_IMAGES records that no tile holds).
+template <typename Real>
+struct Candidates {
+    struct Cand {
+        vd4 rec;
+        int t;
+    };
+    gconst_ptr<char> rec;
+    gconst_ptr<char> type;
+    unsigned long long left;
+    Cand c0, c1;
+    __device__ __attribute__((always_inline)) inline Cand fetch() {
+        // (a bit is always found: the index stays in 0..63, and 63 once none is left)
+        const int i = __builtin_ctzll(left | (1ull << 63));
+        asm("s_bitset0_b64 %0, %1" : "+s"(left) : "s"(i));
+        Cand c;
+        c.rec = *reinterpret_cast<gconst_ptr<vd4>>(rec + i * 32);
+        if constexpr (sizeof(Real) == 4) c.t = unpack_t(c.rec.w);
+        else c.t = *reinterpret_cast<gconst_ptr<int>>(type + i * 4);
+        return c;
+    }
+    __device__ __attribute__((always_inline)) inline Candidates(gconst_ptr<vd4> r, gconst_ptr<int> ty, int first,
+                                                                unsigned long long mask)
+        : rec(reinterpret_cast<gconst_ptr<char>>(r + first)), type(reinterpret_cast<gconst_ptr<char>>(ty + first)),
+          left(mask) {
+        c0 = fetch();
+        c1 = fetch();
+    }
+    __device__ __attribute__((always_inline)) inline Cand take() {
+        const Cand c = c0;
+        c0 = c1;
+        c1 = fetch();
+        return c;
+    }
 };
 
-// Candidates [j0, je) of the LDS list for every lane's point, two at a time in
-// FP32 (they share the LDS address registers, and their chains interleave).
-// GRAD: all of one type, whose constants are pt; else each candidate's type
-// selects its constants.  A branch per candidate on the rare close pair kept
-// the compiler from interleaving the two chains, so the loop only follows the
-// smallest r^2 and the overlap flag comes from it afterwards; where that r^2
-// has no finite 1/r, or is so close to the overlap distance that its FP32 value
-// does not decide, the candidates are taken again one by one.
+// r^2 from absolute Cartesian coordinates: it depends on the point and the image
+// alone, not on the chunk it was found from.
+struct PairPoint {
+    double x, y, z;
+};
+__device__ __attribute__((always_inline)) inline double image_r2(const PairPoint& P, const vd4& c) {
+    const double ddx = c.x - P.x, ddy = c.y - P.y, ddz = c.z - P.z;
+    return ddx * ddx + ddy * ddy + ddz * ddz;
+}
+
+// The next n candidates for every lane's point.  GRAD: all of one type, whose
+// constants are pt; else each candidate's type selects its constants (lj: the
+// site's first entry, `stride` bytes from type to type).  Two candidates at a
+// time, their chains interleaved.  A branch per candidate on the rare close pair
+// would keep the compiler from interleaving them, so the loop only follows the
+// smallest r^2 (m); tile_close does the rest.
+template <typename Real>
+__device__ inline LJC<Real> lj_consts(const LJC<Real>* lj, int t, int stride) {
+    return *reinterpret_cast<const LJC<Real>*>(reinterpret_cast<const char*>(lj) + t * stride);
+}
+
 template <int ESM, typename Real, bool GRAD>
-__device__ __attribute__((always_inline)) inline void pair_loop(const PairLds& L, int j0, int je, double prx, double pry,
-                                                                double prz, int site, const LJC<Real>* s_lj,
-                                                                const LJC<Real>& pt, bool is_lj, double r2lj,
-                                                                double r2sr, const ErfcTabs& et, bool& ovl,
+__device__ __attribute__((always_inline)) inline void pair_loop(Candidates<Real>& C, int n, const PairPoint& P,
+                                                                int stride, const LJC<Real>* lj, const LJC<Real>& pt,
+                                                                double r2lj, double r2sr, const ErfcTabs& et, Real& m,
                                                                 PairSums<Real>& S) {
-    constexpr bool F32 = sizeof(Real) == 4;
-    auto dist2 = [&](const double4& c) {
-        const double ddx = c.x - prx, ddy = c.y - pry, ddz = c.z - prz;
-        return ddx * ddx + ddy * ddy + ddz * ddz;
+    auto term = [&](const typename Candidates<Real>::Cand& c) {
+        const LJC<Real> p = GRAD ? pt : lj_consts<Real>(lj, c.t, stride);
+        bool unused = false;
+        return pair_term<ESM, Real, GRAD, false>(image_r2(P, c.rec), c.rec.w, unpack_q(c.rec.w), p, false, r2lj, r2sr,
+                                                 et, unused, S);
     };
-    auto consts = [&](const double4& c, int k) {
-        if constexpr (GRAD) return pt;
-        else return s_lj[(F32 ? unpack_t(c.w) : L.t[k]) + site];
-    };
-    const PairSums<Real> S0 = S;
-    Real m = (Real)INFINITY;
-    constexpr int PAIR_UNROLL = F32 ? 2 : 1;
-#pragma unroll PAIR_UNROLL
-    for (int j = j0; j < je; ++j) {
-        const double4 c = L.c[j];
-        const float qf = F32 ? unpack_q(c.w) : 0.0f;  // the FP64 terms take c.w
-        const Real u = pair_term<ESM, Real, GRAD, false>(dist2(c), c.w, qf, consts(c, j), is_lj, r2lj, r2sr, et, ovl, S);
-        if constexpr (F32) m = fminf(m, u);
+    for (; n >= 2; n -= 2) {
+        const auto a = C.c0, b = C.c1;
+        C.c0 = C.fetch();
+        C.c1 = C.fetch();
+        const Real u0 = term(a), u1 = term(b);
+        if constexpr (sizeof(Real) == 4) m = fminf(m, fminf(u0, u1));
+        else m = fmin(m, fmin(u0, u1));
+    }
+    if (n != 0) {
+        const Real u = term(C.take());
+        if constexpr (sizeof(Real) == 4) m = fminf(m, u);
         else m = fmin(m, u);
     }
-    // an overlap: r^2 below R2_OVERLAP and inside the LJ cutoff
+}
+
+// After a tile: the overlap flag (r^2 below R2_OVERLAP and inside the LJ cutoff)
+// from the smallest r^2, m.  Where m has no finite 1/r, or is so close to the
+// overlap distance that its FP32 value does not decide, the tile's energies are
+// taken again with the flag and the limit of small r in every term.  (The
+// derivative sums of a gradient run stay: they are used only if the energies
+// are finite.)
+template <int ESM, typename Real>
+__device__ __attribute__((always_inline)) inline void tile_close(Candidates<Real> C, unsigned long long mask,
+                                                                 const PairPoint& P, int stride, const LJC<Real>* lj,
+                                                                 bool is_lj, double r2lj, double r2sr,
+                                                                 const ErfcTabs& et, Real m, bool& ovl, Real& plj,
+                                                                 Real& psr) {
     const double thr = fmin(R2_OVERLAP, r2lj);
     bool redo;
-    if constexpr (F32) {
+    if constexpr (sizeof(Real) == 4) {
         ovl |= is_lj & (m < (float)thr * (1.0f - 1e-6f));
         redo = m < 1e-37f || (m >= (float)thr * (1.0f - 1e-6f) && m <= (float)thr * (1.0f + 1e-6f));
     } else {
         ovl |= is_lj & (m < thr);
         redo = m < 2.2250738585072014e-308;
     }
-    if (__builtin_expect(__ballot(redo) != 0ull, 0)) {
-        S = S0;
+    if (__builtin_expect(__ballot(redo) == 0ull, 1)) return;
+    PairSums<Real> S;
+    C.left = mask;
 #pragma unroll 1
-        for (int j = j0; j < je; ++j) {
-            const double4 c = L.c[j];
-            const float qf = F32 ? unpack_q(c.w) : 0.0f;
-            pair_term<ESM, Real, GRAD, true>(dist2(c), c.w, qf, consts(c, j), is_lj, r2lj, r2sr, et, ovl, S);
-        }
+    while (C.left != 0ull) {
+        const auto a = C.fetch();
+        pair_term<ESM, Real, false, true>(image_r2(P, a.rec), a.rec.w, unpack_q(a.rec.w),
+                                          lj_consts<Real>(lj, a.t, stride), is_lj, r2lj, r2sr, et, ovl, S);
     }
+    plj = S.plj;
+    psr = S.psr;
 }
+
+// LDS of the pair kernels.
+struct PairLds {
+    const float4* erfc;     // FP32 kernels
+    const double2* erfc64;  // FP64 kernels
+    // all-atoms path
+    double4* c;             // replicated atoms: fractional xyz, charge
+    int* t;                 // type * nsite
+};
 
 // Per-type derivative sums of a gradient run's point, FP64, for NT framework
 // types: g[k] = sum (u^2 - u) (u = sigma_ts^6 / r^6; d LJ / d eps_ts = 4 of it),
@@ -762,58 +824,48 @@ struct TypeSums {
     }
 };
 
-// The pair loops of one workgroup's chunk.  Fast path: bound the workgroup's
-// points by a sphere, scan the image list, keep the images within r_cmax of
-// the sphere by a wave-ballot compaction into LDS, evaluate every lane's point
-// against them (an image outside a point's cutoffs adds exact zeros, so the
-// sums do not depend on the sphere).
-// Slow path: every replicated atom, nearest image per pair.  NT > 0 (a
-// gradient run of at most NT framework types) adds the per-type derivative
-// sums: on the fast path the images of a tile come in type order (the image
-// list is sorted by species inside each spatial bin, and a tile never spans
-// two bins), so each tile's kept candidates are runs of one type each, counted
-// per type at compaction; a run is summed with its type's parameters held in
-// registers and folded into the type's FP64 sums once.
+// The pair loops of one workgroup's chunk.  Fast path, each wave by itself:
+// bound the wave's points by a sphere, test the tiles of the image list against
+// it, then the images of each tile that meets it, one per lane, and evaluate
+// every lane's point against the images within r_cmax of the sphere, whose
+// records the wave reads by scalar loads (an image outside a point's cutoffs
+// adds exact zeros, so the sums do not depend on the sphere).  With the
+// candidates staged in LDS by the workgroup instead, every candidate cost two
+// LDS reads more per wave (the LDS was busy 69% of the time) and every four
+// tiles three barriers.  Slow path: every replicated atom, nearest image per
+// pair.  NT > 0 (a gradient run of at most NT framework types) adds the
+// per-type derivative sums: on the fast path the images of a tile come in type
+// order (the image list is sorted by species inside each spatial bin, and a
+// tile never spans two bins), so each tile's candidates are taken type by type,
+// with the type's parameters held in registers, and folded into the type's FP64
+// sums once.
 template <int ESM, typename Real, int NT>
 __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs& a, bool valid, double px, double py, double pz,
                                    int site, const LJC<Real>* s_lj, const double2* s_gc,
-                                   PairLds L, double& acc_lj, double& acc_sr, bool& ovl, unsigned long long& n_cand,
-                                   TypeSums<Real, (NT > 0 ? NT : 1)>& ts) {
+                                   const PairLds& L, double& acc_lj, double& acc_sr, bool& ovl,
+                                   unsigned long long& n_cand, TypeSums<Real, (NT > 0 ? NT : 1)>& ts) {
     constexpr bool GRAD = NT > 0;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
     const double f11 = a.f11, f12 = a.f12, f13 = a.f13, f22 = a.f22, f23 = a.f23, f33 = a.f33;
     const double r2lj = a.r2_lj, r2sr = a.r2_sr;
     const ErfcTabs et{(float)a.erfc_inv_h, L.erfc, a.erfc64_inv_h, L.erfc64};
     const bool is_lj = (a.site_lj_mask >> site) & 1u;
     const int nsite = a.nsite;
-    // a wave with no valid point skips the pair loops; it still takes part in
-    // the tile scans and barriers
     const bool wave_live = __ballot(valid) != 0ull;
     if (a.fast) {
-        // The point and the chunk centre in Cartesian coordinates (FP64).  The
-        // images are stored in Cartesian coordinates, so a pair's r^2 depends
-        // on the point and the image alone, not on the chunk it was found from.
+        if (!wave_live) return;
         // (a lane without a point is put far from every image)
         const double prx = valid ? f11 * px + f12 * py + f13 * pz : 1e8;
         const double pry = f22 * py + f23 * pz;
         const double prz = f33 * pz;
-        // The workgroup's sphere: the centre of its valid points' bounding box
-        // and their largest distance from it (inside the chunk's sphere, and
-        // smaller where the points leave the chunk's corners empty).
+        // The wave's sphere: the centre of its points' bounding box and their
+        // largest distance from it.
         double bx[6] = {valid ? prx : INFINITY,  valid ? pry : INFINITY,  valid ? prz : INFINITY,
                         valid ? -prx : INFINITY, valid ? -pry : INFINITY, valid ? -prz : INFINITY};
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1)
 #pragma unroll
             for (int i = 0; i < 6; ++i) bx[i] = fmin(bx[i], __shfl_xor(bx[i], off, 64));
-        if (lane == 0)
-#pragma unroll
-            for (int i = 0; i < 6; ++i) L.sph[wave * 8 + i] = bx[i];
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < WG / 64; ++w)
-#pragma unroll
-            for (int i = 0; i < 6; ++i) bx[i] = fmin(bx[i], L.sph[w * 8 + i]);
         const double ccx = 0.5 * (bx[0] - bx[3]), ccy = 0.5 * (bx[1] - bx[4]), ccz = 0.5 * (bx[2] - bx[5]);
         double d2 = 0.0;
         if (valid) {
@@ -822,128 +874,59 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
         }
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) d2 = fmax(d2, __shfl_xor(d2, off, 64));
-        if (lane == 0) L.sph[wave * 8 + 6] = d2;
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < WG / 64; ++w) d2 = fmax(d2, L.sph[w * 8 + 6]);
         const double Rc = a.r_cmax + sqrt(d2) + 1e-3;
         const double R2 = Rc * Rc;
-        const int n_tiles = a.n_tiles;
-        for (int tb = 0; tb < n_tiles; tb += WG) {
-            // the tiles of this batch whose bounding sphere meets the chunk's
+        const PairPoint P{prx, pry, prz};
+        const gconst_ptr<vd4> rec = uniform_ptr(reinterpret_cast<const vd4*>(a.img));
+        const gconst_ptr<int> types = uniform_ptr(a.img_type);
+        const gconst_ptr<int> rngs = uniform_ptr(reinterpret_cast<const int*>(a.tile_rng));
+        const double4* const img = a.img;
+        const LJC<Real>* const lj_site = s_lj + site;
+        const int lj_stride = __builtin_amdgcn_readfirstlane(nsite * (int)sizeof(LJC<Real>));
+        const int n_tiles = __builtin_amdgcn_readfirstlane(a.n_tiles);
+        for (int tb = 0; tb < n_tiles; tb += 64) {
+            // the tiles of this batch whose bounding sphere meets the wave's
             bool hit = false;
-            const int ti = tb + tid;
-            if (ti < n_tiles) {
-                const double4 sp = a.tile_sph[ti];
+            if (tb + lane < n_tiles) {
+                const double4 sp = a.tile_sph[tb + lane];
                 const double sx = sp.x - ccx, sy = sp.y - ccy, sz = sp.z - ccz;
                 const double rr = Rc + sp.w;
                 hit = sx * sx + sy * sy + sz * sz < rr * rr;
             }
-            const unsigned long long hm = __ballot(hit);
-            const int hb = __popcll(hm & ((1ull << lane) - 1ull));
-            __syncthreads();  // the previous batch's tile list and candidates are consumed
-            if (lane == 0) L.wcnt[wave] = __popcll(hm);
-            __syncthreads();
-            int hoff = 0, n_hit = 0;
-#pragma unroll
-            for (int w = 0; w < WG / 64; ++w) {
-                const int c = L.wcnt[w];
-                hoff += w < wave ? c : 0;
-                n_hit += c;
-            }
-            if (hit) L.sel[hoff + hb] = ti;
-            __syncthreads();
-            // rounds of WG / 64 selected tiles, one per wave, in tile order
-            for (int k = 0; k < n_hit; k += WG / 64) {
+            for (unsigned long long hm = __ballot(hit); hm != 0ull; hm &= hm - 1ull) {
+                const int ti = tb + __builtin_ctzll(hm);
+                const int first = rngs[2 * ti], count = rngs[2 * ti + 1];
                 bool keep = false;
-                double4 rec = make_double4(0.0, 0.0, 0.0, 0.0);
-                int ty = 0;
-                if (k + wave < n_hit) {
-                    const int2 rg = a.tile_rng[L.sel[k + wave]];
-                    if (lane < rg.y) {
-                        rec = a.img[rg.x + lane];
-                        const double cx = rec.x - ccx, cy = rec.y - ccy, cz = rec.z - ccz;
-                        keep = cx * cx + cy * cy + cz * cz < R2;
-                        ty = a.img_type[rg.x + lane] * nsite;
-                    }
+                if (lane < count) {
+                    const double4 v = img[first + lane];
+                    const double cx = v.x - ccx, cy = v.y - ccy, cz = v.z - ccz;
+                    keep = cx * cx + cy * cy + cz * cz < R2;
                 }
                 const unsigned long long m = __ballot(keep);
-                const int before = __popcll(m & ((1ull << lane) - 1ull));
-                int tc[NT > 0 ? NT : 1];
+                if (m == 0ull) continue;
+                n_cand += (unsigned long long)__popcll(m);
+                Candidates<Real> C(rec, types, first, m);
+                // the candidates of a tile accumulate in Real, folded into FP64
+                PairSums<Real> S;
+                Real small = (Real)INFINITY;
                 if constexpr (GRAD) {
+                    const int ty = lane < count ? a.img_type[first + lane] : -1;
 #pragma unroll
-                    for (int k = 0; k < NT; ++k) tc[k] = __popcll(__ballot(keep && ty == k * nsite));
-                }
-                __syncthreads();  // the previous round's candidates (and the tile counts) are consumed
-                if (lane == 0) {
-                    L.wcnt[wave] = __popcll(m);
-                    if constexpr (GRAD) {
-                        // cumulative counts, 7 bits per type (a tile holds at most 64)
-                        unsigned long long ends = 0ull;
-                        int cum = 0;
-#pragma unroll
-                        for (int k = 0; k < NT; ++k) {
-                            cum += tc[k];
-                            ends |= (unsigned long long)cum << (7 * k);
-                        }
-                        L.ends[2 * wave] = (unsigned)ends;
-                        L.ends[2 * wave + 1] = (unsigned)(ends >> 32);
+                    for (int k = 0; k < NT; ++k) {
+                        const unsigned long long mk = __ballot(keep && ty == k);
+                        if (mk == 0ull) continue;
+                        S.s1 = S.s2 = S.sq = (Real)0;
+                        pair_loop<ESM, Real, true>(C, __popcll(mk), P, 0, lj_site, lj_site[k * nsite], r2lj, r2sr, et,
+                                                   small, S);
+                        ts.add(k, S, s_gc[k * nsite + site], is_lj);
                     }
+                } else {
+                    pair_loop<ESM, Real, false>(C, __popcll(m), P, lj_stride, lj_site, LJC<Real>{}, r2lj, r2sr, et,
+                                                small, S);
                 }
-                __syncthreads();
-                int woff[WG / 64 + 1];
-                woff[0] = 0;
-#pragma unroll
-                for (int w = 0; w < WG / 64; ++w) woff[w + 1] = woff[w] + L.wcnt[w];
-                if (keep) {
-                    if constexpr (sizeof(Real) == 4) {
-                        L.c[woff[wave] + before] = make_double4(rec.x, rec.y, rec.z, pack_tq(ty, (float)rec.w));
-                    } else {
-                        L.c[woff[wave] + before] = rec;
-                        L.t[woff[wave] + before] = ty;
-                    }
-                }
-                __syncthreads();
-                n_cand += (unsigned long long)woff[WG / 64];
-                if (wave_live) {
-                    if constexpr (GRAD) {
-                        // tile by tile (the energies' FP32 sums fold per tile, as below),
-                        // type run by type run inside each tile; the runs' ends come
-                        // from one scalar word per tile
-                        int j = 0;
-                        for (int gi = 0; gi < WG / 64; ++gi) {
-                            PairSums<Real> S;
-                            const int j0 = j;
-                            const unsigned long long ends =
-                                (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(L.ends[2 * gi]) |
-                                (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(L.ends[2 * gi + 1])
-                                    << 32;
-#pragma unroll
-                            for (int k = 0; k < NT; ++k) {
-                                const int je = j0 + (int)((ends >> (7 * k)) & 127ull);
-                                if (je == j) continue;
-                                const LJC<Real> p = s_lj[k * nsite + site];
-                                S.s1 = S.s2 = S.sq = (Real)0;
-                                pair_loop<ESM, Real, true>(L, j, je, prx, pry, prz, site, s_lj, p, is_lj, r2lj, r2sr,
-                                                           et, ovl, S);
-                                j = je;
-                                ts.add(k, S, s_gc[k * nsite + site], is_lj);
-                            }
-                            acc_lj += (double)S.plj;
-                            acc_sr += (double)S.psr;
-                        }
-                    } else {
-                        // the candidates of each tile accumulate in Real, flushed to FP64
-#pragma unroll
-                        for (int gi = 0; gi < WG / 64; ++gi) {
-                            PairSums<Real> S;
-                            pair_loop<ESM, Real, false>(L, woff[gi], woff[gi + 1], prx, pry, prz, site, s_lj,
-                                                        LJC<Real>{}, is_lj, r2lj, r2sr, et, ovl, S);
-                            acc_lj += (double)S.plj;
-                            acc_sr += (double)S.psr;
-                        }
-                    }
-                }
+                tile_close<ESM, Real>(C, m, P, lj_stride, lj_site, is_lj, r2lj, r2sr, et, small, ovl, S.plj, S.psr);
+                acc_lj += (double)S.plj;
+                acc_sr += (double)S.psr;
             }
         }
     } else {
@@ -954,7 +937,6 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
             if (tid < nt) {
                 L.c[tid] = a.atoms[base + tid];
                 L.t[tid] = a.species[base + tid] * nsite;
-                L.qf[tid] = (float)a.atoms[base + tid].w;
             }
             __syncthreads();
             n_cand += (unsigned long long)nt;
@@ -972,15 +954,10 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                         const double cy = f22 * ey + f23 * ez;
                         const double cz = f33 * ez;
                         const double r2 = cx * cx + cy * cy + cz * cz;
-                        LJC<Real> p;
-                        if constexpr (GRAD) {
-                            const int tt = __builtin_amdgcn_readfirstlane(L.t[j]);
-                            ts.type(tt, nsite, s_gc[tt + site], S, is_lj);
-                            p = s_lj[tt + site];
-                        } else {
-                            p = s_lj[L.t[j] + site];
-                        }
-                        pair_term<ESM, Real, GRAD, true>(r2, at.w, L.qf[j], p, is_lj, r2lj, r2sr, et, ovl, S);
+                        const int tt = __builtin_amdgcn_readfirstlane(L.t[j]);
+                        if constexpr (GRAD) ts.type(tt, nsite, s_gc[tt + site], S, is_lj);
+                        pair_term<ESM, Real, GRAD, true>(r2, at.w, (float)at.w, s_lj[tt + site], is_lj, r2lj, r2sr, et,
+                                                         ovl, S);
                     }
                     acc_lj += (double)S.plj;
                     acc_sr += (double)S.psr;
@@ -991,37 +968,34 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
     }
 }
 
-// LDS: TILE candidate records, types and FP32 charges, the selected-tile list,
-// the erfc table (FP32 cubics or FP64 quintics), the small per-wave arrays, then
-// the LJ table of the run (and for a gradient run its fold constants).
-constexpr int PAIR_LDS_SMALL = (WG / 64) * 80;  // sphere partials, run ends, candidate counts
+// LDS, all of it dynamic (it then starts at address 0, and table reads carry
+// their whole base in the instruction's offset): the erfc table (FP32 cubics or
+// FP64 quintics), the LJ table of the run (and for a gradient run its fold
+// constants), and for a launch with a run on the all-atoms path TILE atoms.
 template <typename Real>
 constexpr int pair_lds_fixed() {
-    return PAIR_LDS_SMALL + TILE * (int)(sizeof(double4) + sizeof(int) + sizeof(float) + sizeof(int)) +
-           (sizeof(Real) == 4 ? ERFC_TAB * (int)sizeof(float4) : ERFC64_TAB * (int)sizeof(double2));
+    return sizeof(Real) == 4 ? ERFC_TAB * (int)sizeof(float4) : ERFC64_TAB * (int)sizeof(double2);
+}
+constexpr int PAIR_LDS_ATOMS = TILE * (int)(sizeof(double4) + sizeof(int));
+
+template <typename Real, int NT>
+constexpr int pair_waves() {
+    return sizeof(Real) == 4 && NT == 6 ? 4 : 1;
 }
 
 // NT = 0: energies.  NT > 0: a gradient run of at most NT framework types.
 template <typename Real, int NT>
-__global__ __launch_bounds__(WG) void point_pair_kernel(GroupArgs g) {
+__global__ __launch_bounds__(WG, (pair_waves<Real, NT>())) void point_pair_kernel(GroupArgs g, int atoms_off) {
     constexpr bool GRAD = NT > 0;
     extern __shared__ __align__(16) unsigned char smem[];
-    PairLds L;
-    L.c = reinterpret_cast<double4*>(smem);
-    L.t = reinterpret_cast<int*>(smem + TILE * sizeof(double4));
-    L.qf = reinterpret_cast<float*>(smem + TILE * (sizeof(double4) + sizeof(int)));
-    L.sel = reinterpret_cast<int*>(smem + TILE * (sizeof(double4) + sizeof(int) + sizeof(float)));
-    float4* s_erfc = reinterpret_cast<float4*>(smem + TILE * (sizeof(double4) + 2 * sizeof(int) + sizeof(float)));
-    L.erfc = s_erfc;
-    double2* s_erfc64 = reinterpret_cast<double2*>(s_erfc);
-    L.erfc64 = s_erfc64;
-    // (all LDS is dynamic: it then starts at address 0, and the table reads
-    // carry their whole base in the instruction's offset)
-    unsigned char* small = smem + pair_lds_fixed<Real>() - PAIR_LDS_SMALL;
-    L.sph = reinterpret_cast<double*>(small);
-    L.ends = reinterpret_cast<unsigned*>(small + (WG / 64) * 8 * sizeof(double));
-    L.wcnt = reinterpret_cast<int*>(small + (WG / 64) * (8 * sizeof(double) + 2 * sizeof(unsigned)));
+    float4* s_erfc = reinterpret_cast<float4*>(smem);
+    double2* s_erfc64 = reinterpret_cast<double2*>(smem);
     LJC<Real>* s_lj = reinterpret_cast<LJC<Real>*>(smem + pair_lds_fixed<Real>());
+    PairLds L;
+    L.erfc = s_erfc;
+    L.erfc64 = s_erfc64;
+    L.c = reinterpret_cast<double4*>(smem + atoms_off);
+    L.t = reinterpret_cast<int*>(L.c + TILE);
 
     const int tid = threadIdx.x;
     int si;
@@ -1077,6 +1051,7 @@ __global__ __launch_bounds__(WG) void point_pair_kernel(GroupArgs g) {
     if constexpr (sizeof(Real) == 8)
         if (a.esm != 0)
             for (int t = tid; t < ERFC64_TAB; t += WG) s_erfc64[t] = a.erfc64_tab[t];
+    __syncthreads();
 
     double acc_lj = 0.0, acc_sr = 0.0;
     bool ovl = false;

@@ -296,6 +296,7 @@ struct pm_framework {
         int64_t n = 0;
         int64_t n_tiles = 0;
         double4* d_img = nullptr;
+        double4* d_img_m = nullptr;     // the same with (type, FP32 charge) in the charge's place (mixed runs)
         int32_t* d_type = nullptr;
         double4* d_tile_sph = nullptr;  // tile bounding spheres
         int2* d_tile_rng = nullptr;     // tile (first image, count)
@@ -539,6 +540,14 @@ int run_poses(const pm_framework* fw, const pm_forcefield* ff, const pm_ewald* e
 // span it); stored in Cartesian coordinates.  Lists are cached
 // per framework and radius, so a run's list -- and with it the order of its
 // FP32 partial sums -- depends on the framework and the radius alone.
+void free_images(pm_framework::Images& im) {
+    (void)hipFree(im.d_img);
+    (void)hipFree(im.d_img_m);
+    (void)hipFree(im.d_type);
+    (void)hipFree(im.d_tile_sph);
+    (void)hipFree(im.d_tile_rng);
+}
+
 const pm_framework::Images* find_images(const pm_framework* fw, double r) {
     for (const auto& im : fw->images)
         if (im.r == r) return &im;
@@ -662,27 +671,36 @@ int get_images(pm_framework* fw, double r, const pm_framework::Images** out) {
     im.n = (int64_t)img.size();
     im.n_tiles = (int64_t)sph.size();
     if (im.n > (int64_t)INT32_MAX) return fail(PM_ERR_ARG, "image list too large");
-    const size_t n = std::max<size_t>(img.size(), 1);
+    // unused records after the last image, which Candidates::fetch may read
+    const size_t n = img.size() + TILE_IMAGES;
+    std::vector<double4> rec(n, make_double4(0.0, 0.0, 0.0, 0.0)), rec_m(rec);
+    std::vector<int32_t> types(n, 0);
+    for (size_t i = 0; i < img.size(); ++i) {
+        rec[i] = rec_m[i] = img[i];
+        types[i] = ty[i];
+        const float qf = (float)img[i].w;
+        uint32_t bits;
+        std::memcpy(&bits, &qf, sizeof(bits));
+        const uint64_t w = ((uint64_t)(uint32_t)ty[i] << 32) | bits;
+        std::memcpy(&rec_m[i].w, &w, sizeof(w));
+    }
     const size_t nt = std::max<size_t>(sph.size(), 1);
-    PM_HIP(hipMalloc(&im.d_img, n * sizeof(double4)));
-    hipError_t e = hipMalloc(&im.d_type, n * sizeof(int32_t));
+    hipError_t e = hipMalloc(&im.d_img, n * sizeof(double4));
+    if (e == hipSuccess) e = hipMalloc(&im.d_img_m, n * sizeof(double4));
+    if (e == hipSuccess) e = hipMalloc(&im.d_type, n * sizeof(int32_t));
     if (e == hipSuccess) e = hipMalloc(&im.d_tile_sph, nt * sizeof(double4));
     if (e == hipSuccess) e = hipMalloc(&im.d_tile_rng, nt * sizeof(int2));
-    if (e == hipSuccess && !img.empty()) {
-        e = hipMemcpy(im.d_img, img.data(), img.size() * sizeof(double4), hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = hipMemcpy(im.d_type, ty.data(), ty.size() * sizeof(int32_t), hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = hipMemcpy(im.d_tile_sph, sph.data(), sph.size() * sizeof(double4), hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = hipMemcpy(im.d_tile_rng, rng.data(), rng.size() * sizeof(int2), hipMemcpyHostToDevice);
-    }
+    if (e == hipSuccess) e = hipMemcpy(im.d_img, rec.data(), n * sizeof(double4), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(im.d_img_m, rec_m.data(), n * sizeof(double4), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(im.d_type, types.data(), n * sizeof(int32_t), hipMemcpyHostToDevice);
+    if (e == hipSuccess && !sph.empty())
+        e = hipMemcpy(im.d_tile_sph, sph.data(), sph.size() * sizeof(double4), hipMemcpyHostToDevice);
+    if (e == hipSuccess && !rng.empty())
+        e = hipMemcpy(im.d_tile_rng, rng.data(), rng.size() * sizeof(int2), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
-        (void)hipFree(im.d_img);
-        (void)hipFree(im.d_type);
-        (void)hipFree(im.d_tile_sph);
-        (void)hipFree(im.d_tile_rng);
-        return fail(PM_ERR_DEVICE, std::string("image list upload: ") + hipGetErrorString(e));
+        free_images(im);
+        return fail(e == hipErrorOutOfMemory ? PM_ERR_OOM : PM_ERR_DEVICE,
+                    std::string("image list upload: ") + hipGetErrorString(e));
     }
     fw->images.push_back(im);
     *out = &fw->images.back();
@@ -921,8 +939,8 @@ int grid_prepare(const pm_grid_run& in, PointRun& r) {
 }
 
 template <typename Real, int NT>
-void pair_launch_t(const GroupArgs& g, int n_wg, size_t shm) {
-    hipLaunchKernelGGL((point_pair_kernel<Real, NT>), dim3(n_wg), dim3(WG), shm, g_ctx.stream, g);
+void pair_launch_t(const GroupArgs& g, int n_wg, size_t shm, int atoms_off) {
+    hipLaunchKernelGGL((point_pair_kernel<Real, NT>), dim3(n_wg), dim3(WG), shm, g_ctx.stream, g, atoms_off);
 }
 
 // Compiled type counts of the gradient kernels: a gradient run of n_gt
@@ -931,12 +949,12 @@ void pair_launch_t(const GroupArgs& g, int n_wg, size_t shm) {
 int grad_nt(int n_gt) { return n_gt <= 2 ? 2 : n_gt <= 4 ? 4 : n_gt <= 6 ? 6 : GT; }
 
 template <typename Real>
-void pair_launch_grad(const GroupArgs& g, int n_wg, size_t shm, int nt) {
+void pair_launch_grad(const GroupArgs& g, int n_wg, size_t shm, int atoms_off, int nt) {
     switch (nt) {
-        case 2: pair_launch_t<Real, 2>(g, n_wg, shm); break;
-        case 4: pair_launch_t<Real, 4>(g, n_wg, shm); break;
-        case 6: pair_launch_t<Real, 6>(g, n_wg, shm); break;
-        default: pair_launch_t<Real, GT>(g, n_wg, shm); break;
+        case 2: pair_launch_t<Real, 2>(g, n_wg, shm, atoms_off); break;
+        case 4: pair_launch_t<Real, 4>(g, n_wg, shm, atoms_off); break;
+        case 6: pair_launch_t<Real, 6>(g, n_wg, shm, atoms_off); break;
+        default: pair_launch_t<Real, GT>(g, n_wg, shm, atoms_off); break;
     }
 }
 
@@ -1028,7 +1046,7 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
             }
             if (rc == PM_OK) {
                 a.fast = 1;
-                a.img = im->d_img;
+                a.img = fp64 ? im->d_img : im->d_img_m;
                 a.img_type = im->d_type;
                 a.n_img = (int)im->n;
                 a.tile_sph = im->d_tile_sph;
@@ -1293,7 +1311,11 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
     g.cand_pairs = d_cand;
     g.out_g = grad ? reinterpret_cast<double*>(base + o_g) : nullptr;
     g.g_stride = max_slots;
-    const size_t shm = (fp64 ? pair_lds_fixed<double>() : pair_lds_fixed<float>()) + std::max<size_t>(lj_lds, 16);
+    bool all_fast = true;
+    for (const PointRun& r : runs) all_fast = all_fast && r.ra.fast != 0;
+    const int atoms_off =
+        (fp64 ? pair_lds_fixed<double>() : pair_lds_fixed<float>()) + (int)((std::max<size_t>(lj_lds, 16) + 15) / 16 * 16);
+    const size_t shm = (size_t)atoms_off + (all_fast ? 0 : PAIR_LDS_ATOMS);
 
     // the counter is cleared by a kernel (Widom: the first cell-count fill),
     // which a caller's graph capture records safely
@@ -1332,11 +1354,11 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
         }
         PM_HIP(hipEventRecord(g_ctx.evp0, g_ctx.stream));
         if (grad) {
-            if (fp64) pair_launch_grad<double>(g, (int)pair_wg, shm, nt_grad);
-            else pair_launch_grad<float>(g, (int)pair_wg, shm, nt_grad);
+            if (fp64) pair_launch_grad<double>(g, (int)pair_wg, shm, atoms_off, nt_grad);
+            else pair_launch_grad<float>(g, (int)pair_wg, shm, atoms_off, nt_grad);
         } else {
-            if (fp64) pair_launch_t<double, 0>(g, (int)pair_wg, shm);
-            else pair_launch_t<float, 0>(g, (int)pair_wg, shm);
+            if (fp64) pair_launch_t<double, 0>(g, (int)pair_wg, shm, atoms_off);
+            else pair_launch_t<float, 0>(g, (int)pair_wg, shm, atoms_off);
         }
         PM_HIP(hipEventRecord(g_ctx.evp1, g_ctx.stream));
         const long long slot_wg = (gr.n_slots + WG - 1) / WG;
@@ -1720,12 +1742,7 @@ int pm_framework_destroy(pm_framework* fw) {
     (void)hipFree(fw->d_atoms);
     (void)hipFree(fw->d_species);
     (void)hipFree(fw->d_unit_q);
-    for (auto& im : fw->images) {
-        (void)hipFree(im.d_img);
-        (void)hipFree(im.d_type);
-        (void)hipFree(im.d_tile_sph);
-        (void)hipFree(im.d_tile_rng);
-    }
+    for (auto& im : fw->images) free_images(im);
     delete fw;
     return PM_OK;
 }
