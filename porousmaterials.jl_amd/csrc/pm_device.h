@@ -11,18 +11,16 @@
 //   Widom          src/henry.jl:212-243           per-block sum e^{-E/T}, E e^{-E/T}
 //   energy grid    src/grid.jl:313-355            point (i,j,k)/(n-1) ./ rep
 //
-// Two execution schemes share the pair arithmetic:
-//   pose_kernel       one work-item per pose (all of its sites), every framework
-//                     atom streamed through LDS, nearest image per pair; serves the
-//                     explicit-pose API (vdw_energy, electrostatic_potential_energy).
-//   point engine      every probe site is an independent point.  Points are grouped
-//                     into spatially compact chunks (one cell of a counting sort, or
-//                     one brick of a grid) of <= 256 per workgroup.  A chunk scans an
-//                     image list of the framework that covers every image within
-//                     r_c + chunk radius of any cell, keeps those images (Cartesian,
-//                     FP64, relative to the chunk centre) in LDS and evaluates only
-//                     them: no per-pair wrap or basis change, ~1/4 of the pairs.
-//                     The Fourier part runs in its own FP64 kernel.
+// Two execution schemes:
+//   pm_poses.h    one workgroup per pose, every replicated atom, nearest image
+//                 per pair; serves the explicit-pose API (vdw_energy,
+//                 electrostatic_potential_energy, forces).
+//   pm_points.h   every probe site is an independent point.  Points are grouped
+//                 into spatially compact chunks (one cell of a counting sort, or
+//                 one brick of a grid) of <= 256 per workgroup, evaluated against
+//                 an image list of the framework that covers every image within
+//                 r_c of any point: no per-pair wrap or basis change, ~1/4 of the
+//                 pairs.  The Fourier part runs in its own FP64 kernel.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -35,7 +33,6 @@ namespace pmk {
 
 constexpr int WG = 256;      // work-items per workgroup (4 waves)
 constexpr int TILE = 256;    // framework atoms per LDS tile
-constexpr int KTILE = 128;   // k-vectors per LDS tile (pose kernel)
 constexpr double R2_OVERLAP = 0.1;  // src/vdw_energetics.jl:2
 
 enum { MODE_WIDOM = 0, MODE_GRID = 2 };
@@ -180,210 +177,6 @@ __device__ inline void block_sum3(double v0, double v1, double v2, double* out) 
         double t0 = 0.0, t1 = 0.0, t2 = 0.0;
         for (int w = 0; w < WG / 64; ++w) { t0 += red[0][w]; t1 += red[1][w]; t2 += red[2][w]; }
         out[0] = t0; out[1] = t1; out[2] = t2;
-    }
-}
-
-// =========================================================================
-// Explicit poses: one work-item per pose, NS sites each.
-// =========================================================================
-struct PoseArgs {
-    int ns, n_atoms, n_types, nk;
-    long long n_items;
-    double f11, f12, f13, f22, f23, f33;  // replicated-box f_to_c (upper triangular)
-    double c2f[9];                        // replicated-box c_to_f, column-major (forces)
-    double repd[3];                       // replication factors (unit-cell phases)
-    double r2_lj, r2_sr, alpha, inv4pe;
-    Site site[PM_MAX_SITES];
-    const double4* atoms;  // replicated atoms: fractional xyz + charge
-    const int* species;
-    const void* ljtab;     // [n_types][ns] of LJP<Real>
-    const KVec* kv;
-    const double* pose_xf; // n_items x ns x 3
-    double* out_e;         // n_items x 3: (vdw, sr, lr)
-    double* out_g;         // GRAD: n_items x ns x 3, dE/d(site Cartesian xyz) in K/A
-};
-
-// One wave per pose: the workgroup's four poses share LDS tiles of framework
-// atoms (and of k-vectors), the wave's lanes stride over a tile, and FP64 lane
-// partials are reduced by a fixed shuffle tree.  GRAD adds the gradient of the
-// pose's energy with respect to every site's Cartesian position:
-//   LJ      d/dx_s = 6 eps4 (2u^2 - u) / r^2 * d,   u = (sigma^2 / r^2)^3
-//   real    d/dx_s = q_s q_a [erfc(a r) / r + 2a/sqrt(pi) e^{-a^2 r^2}] / r^2 * d / (4 pi eps0)
-//   Fourier d/dx_s = q_s 2 pi C^T sum_k (-A_re sin th + A_im cos th) (m o rep),  th = 2 pi m.(rep o x)
-// with d = x_atom - x_s (nearest image, Cartesian) and C the replicated box's c_to_f.
-template <int NS, bool ES, typename Real, bool GRAD>
-__global__ __launch_bounds__(WG) void pose_kernel(PoseArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    constexpr int ATOM_BYTES = TILE * (int)sizeof(double4);
-    constexpr int K_BYTES = KTILE * (int)sizeof(KVec);
-    constexpr int REGION = ATOM_BYTES > K_BYTES ? ATOM_BYTES : K_BYTES;
-    double4* s_atoms = reinterpret_cast<double4*>(smem);
-    KVec* s_k = reinterpret_cast<KVec*>(smem);
-    int* s_type = reinterpret_cast<int*>(smem + REGION);
-    LJP<Real>* s_lj = reinterpret_cast<LJP<Real>*>(smem + REGION + TILE * sizeof(int));
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const LJP<Real>* gtab = reinterpret_cast<const LJP<Real>*>(a.ljtab);
-    for (int i = tid; i < a.n_types * NS; i += WG) s_lj[i] = gtab[i];
-
-    const long long item = (long long)blockIdx.x * (WG / 64) + wave;
-    const bool valid = item < a.n_items;
-    const long long it = valid ? item : 0;
-    double sx[NS], sy[NS], sz[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        const double* p = a.pose_xf + (it * NS + s) * 3;
-        sx[s] = p[0]; sy[s] = p[1]; sz[s] = p[2];
-    }
-
-    double acc_lj[NS], acc_sr[NS];
-    double gx[NS], gy[NS], gz[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        acc_lj[s] = 0.0; acc_sr[s] = 0.0;
-        gx[s] = 0.0; gy[s] = 0.0; gz[s] = 0.0;
-    }
-    bool ovl = false;
-    const double f11 = a.f11, f12 = a.f12, f13 = a.f13, f22 = a.f22, f23 = a.f23, f33 = a.f33;
-    const double r2lj = a.r2_lj, r2sr = a.r2_sr, alpha = a.alpha;
-    const double two_a_rpi = 2.0 * alpha * 0.56418958354775628;  // 2 alpha / sqrt(pi)
-    for (int base = 0; base < a.n_atoms; base += TILE) {
-        const int nt = min(TILE, a.n_atoms - base);
-        __syncthreads();
-        if (tid < nt) {
-            s_atoms[tid] = a.atoms[base + tid];
-            s_type[tid] = a.species[base + tid];
-        }
-        __syncthreads();
-        if (!valid) continue;
-        for (int j = lane; j < nt; j += 64) {
-            const double4 at = s_atoms[j];
-            const int t = s_type[j];
-#pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                double dx = at.x - sx[s], dy = at.y - sy[s], dz = at.z - sz[s];
-                dx -= rint(dx);
-                dy -= rint(dy);
-                dz -= rint(dz);
-                const double cx = f11 * dx + f12 * dy + f13 * dz;
-                const double cy = f22 * dy + f23 * dz;
-                const double cz = f33 * dz;
-                const double r2 = cx * cx + cy * cy + cz * cz;
-                const LJP<Real> p = s_lj[t * NS + s];
-                const bool in = r2 < r2lj;
-                ovl |= in & (r2 < R2_OVERLAP) & (a.site[s].lj != 0);
-                const Real e = PairMath<Real>::lj(r2, p.sig2, p.eps4);
-                acc_lj[s] += in ? (double)e : 0.0;
-                if (GRAD) {
-                    // 6 eps4 (2u^2 - u) / r^2
-                    const double rr = 1.0 / r2;
-                    const double sg = (double)p.sig2 * rr;
-                    const double u = sg * sg * sg;
-                    const double f = in ? 6.0 * (double)p.eps4 * u * (2.0 * u - 1.0) * rr : 0.0;
-                    gx[s] += f * cx;
-                    gy[s] += f * cy;
-                    gz[s] += f * cz;
-                }
-                if (ES) {
-                    const bool ins = (r2 < r2sr) & (at.w != 0.0);
-                    const Real c = PairMath<Real>::coul(r2, at.w, alpha);
-                    acc_sr[s] += ins ? (double)c : 0.0;
-                    if (GRAD) {
-                        const double r = sqrt(r2);
-                        const double f = ins ? at.w * (erfc(alpha * r) / r + two_a_rpi * exp(-alpha * alpha * r2)) /
-                                                   r2 * a.site[s].q * a.inv4pe
-                                             : 0.0;
-                        gx[s] += f * cx;
-                        gy[s] += f * cy;
-                        gz[s] += f * cz;
-                    }
-                }
-            }
-        }
-    }
-
-    double acc_lr[NS];
-    double hx[NS], hy[NS], hz[NS];  // Fourier gradient in (m o rep) space
-#pragma unroll
-    for (int s = 0; s < NS; ++s) { acc_lr[s] = 0.0; hx[s] = 0.0; hy[s] = 0.0; hz[s] = 0.0; }
-    if (ES) {
-        double ux[NS], uy[NS], uz[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            ux[s] = sx[s] * a.repd[0];
-            uy[s] = sy[s] * a.repd[1];
-            uz[s] = sz[s] * a.repd[2];
-        }
-        for (int base = 0; base < a.nk; base += KTILE) {
-            const int nt = min(KTILE, a.nk - base);
-            __syncthreads();
-            if (tid < nt) s_k[tid] = a.kv[base + tid];
-            __syncthreads();
-            if (!valid) continue;
-            for (int k = lane; k < nt; k += 64) {
-                const KVec kv = s_k[k];
-#pragma unroll
-                for (int s = 0; s < NS; ++s) {
-                    if (a.site[s].q != 0.0) {
-                        double t = kv.ma * ux[s] + kv.mb * uy[s] + kv.mc * uz[s];
-                        t -= rint(t);
-                        double sn, cs;
-                        sincospi(2.0 * t, &sn, &cs);
-                        acc_lr[s] += kv.are * cs + kv.aim * sn;
-                        if (GRAD) {
-                            const double d = kv.aim * cs - kv.are * sn;
-                            hx[s] += d * kv.ma;
-                            hy[s] += d * kv.mb;
-                            hz[s] += d * kv.mc;
-                        }
-                    }
-                }
-            }
-        }
-    }
-
-    // fixed-order reductions over the wave's lanes
-    double vdw = 0.0, sr = 0.0, lr = 0.0;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        vdw += wave_sum(acc_lj[s]);
-        if (ES) {
-            sr += a.site[s].q * wave_sum(acc_sr[s]);
-            lr += a.site[s].q * wave_sum(acc_lr[s]);
-        }
-    }
-    ovl = __ballot(ovl) != 0ull;
-    if (ovl) vdw = INFINITY;
-    if (GRAD) {
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            gx[s] = wave_sum(gx[s]);
-            gy[s] = wave_sum(gy[s]);
-            gz[s] = wave_sum(gz[s]);
-            if (ES) {
-                hx[s] = wave_sum(hx[s]);
-                hy[s] = wave_sum(hy[s]);
-                hz[s] = wave_sum(hz[s]);
-            }
-        }
-    }
-    if (valid && lane == 0) {
-        a.out_e[3 * item + 0] = vdw;
-        a.out_e[3 * item + 1] = sr * a.inv4pe;
-        a.out_e[3 * item + 2] = lr;
-        if (GRAD) {
-#pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                // Fourier: 2 pi q_s C^T (h o rep)
-                const double q2p = 2.0 * M_PI * a.site[s].q;
-                const double vx = hx[s] * a.repd[0] * q2p, vy = hy[s] * a.repd[1] * q2p, vz = hz[s] * a.repd[2] * q2p;
-                const double* C = a.c2f;
-                double* o = a.out_g + (item * NS + s) * 3;
-                o[0] = gx[s] + C[0] * vx + C[1] * vy + C[2] * vz;
-                o[1] = gy[s] + C[3] * vx + C[4] * vy + C[5] * vz;
-                o[2] = gz[s] + C[6] * vx + C[7] * vy + C[8] * vz;
-            }
-        }
     }
 }
 

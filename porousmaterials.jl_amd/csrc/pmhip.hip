@@ -19,6 +19,7 @@
 #include "pm_gcmc.h"
 #include "pm_pockets.h"
 #include "pm_points.h"
+#include "pm_poses.h"
 #include "pmhip.h"
 
 #define PM_VERSION "pmhip 0.2.0 (gfx950)"
@@ -44,6 +45,7 @@ constexpr size_t MAX_IMAGE_LISTS = 8;             // image lists (radii) per fra
 constexpr long long MAX_GROUP_CELLS = 1LL << 24;  // cells of one launch group
 constexpr double SB_POINTS = 32768.0;             // target points per super-bin of the Widom sort
 constexpr double ZSLAB_POINTS = 64.0;             // target points per slab of a Widom cell
+constexpr int64_t MAX_POSE_PHASE_BYTES = 32768;   // phase powers of a pose in LDS
 constexpr int MAX_RUN_CELLS = 65536;              // cells of one Widom run
 static_assert(MAX_POINT_SLOTS <= (long long)pmk::SB_SLOT_MASK + 1, "a super-bin slot fits below the copy bits");
 static_assert(MAX_GROUP_CELLS <= (long long)pmk::CELL_MASK + 1, "a group's cell index fits below the slab bits");
@@ -287,6 +289,7 @@ struct pm_framework {
     double net_charge = 0.0;
     bool charged = false;
     double4* d_atoms = nullptr;
+    float4* d_atoms_f = nullptr;  // FP32 positions in [0, 1), in d_atoms' allocation
     int32_t* d_species = nullptr;
     double4* d_unit_q = nullptr;
     // Image lists, one per cutoff radius r: every periodic image within r of
@@ -435,11 +438,6 @@ int check_species(const pm_framework* fw, const pm_forcefield* ff) {
 }
 
 // ----------------------------------------------------------- poses ----
-size_t pose_lds_bytes(int n_types, int ns, bool fp64) {
-    size_t region = std::max((size_t)TILE * sizeof(double4), (size_t)KTILE * sizeof(KVec));
-    return region + TILE * sizeof(int) + (size_t)std::max(n_types, 1) * ns * (fp64 ? 16 : 8);
-}
-
 template <int NS, bool ES, typename Real, bool GRAD>
 void pose_launch_t(const PoseArgs& a, int n_wg, size_t shm) {
     hipLaunchKernelGGL((pose_kernel<NS, ES, Real, GRAD>), dim3(n_wg), dim3(WG), shm, g_ctx.stream, a);
@@ -482,19 +480,41 @@ int run_poses(const pm_framework* fw, const pm_forcefield* ff, const pm_ewald* e
     a.n_atoms = (int)fw->n_rep;
     a.n_types = (int)fw->species_global.size();
     a.atoms = fw->d_atoms;
+    a.atoms_f = fw->d_atoms_f;
     a.species = fw->d_species;
     a.inv4pe = INV_4PI_EPS0;
     a.r2_lj = ff ? ff->r2_cutoff : 0.0;
+    const bool fp64 = precision == PM_FP64;
+    const bool table = es && (fp64 || out_grad != nullptr);
+    a.nz = 0;
     if (es) {
         a.alpha = ew->alpha;
         a.r2_sr = ew->sr_cutoff * ew->sr_cutoff;
+        a.erfc64_inv_h = ERFC64_SEG / ew->sr_cutoff;
+        a.erfc64_tab = ew->d_erfc64;
         a.kv = ew->d_k;
         a.nk = (int)ew->nk;
+        a.Ma = ew->Ma;
+        a.Mb = ew->Mb;
+        a.Mc = ew->Mc;
+        const int64_t nz = (int64_t)ew->Ma + ew->Mb + ew->Mc + 3;
+        if (nz * a.ns * 16 <= MAX_POSE_PHASE_BYTES) a.nz = (int)nz;
     } else {
         a.alpha = 1.0;
         a.r2_sr = 0.0;
         a.kv = nullptr;
         a.nk = 0;
+    }
+    // FP32 squared distances below which a pair is looked at in FP64.  A distance
+    // from FP32 fractional coordinates is off by a few 2^-24 of the box's edges.
+    // In a box narrower than the cutoff sphere the FP32 nearest image may be
+    // another one than the FP64 one: every pair is looked at.
+    {
+        const double r2 = std::max(a.r2_lj, a.r2_sr), rc = std::sqrt(r2);
+        double edge = rc;
+        for (int c = 0; c < 3; ++c) edge += std::fabs(fw->F[3 * c]) + std::fabs(fw->F[3 * c + 1]) + std::fabs(fw->F[3 * c + 2]);
+        const double wide = std::min(fw->width[0], std::min(fw->width[1], fw->width[2]));
+        a.r2_keep = wide >= 2.0 * rc ? (float)(r2 + 4e-6 * rc * edge + 1e-9) : INFINITY;
     }
     size_t tab_bytes = 0;
     if (int rc = stage_ljtab(fw, ff, a.ns, a.site, site_species, precision, &tab_bytes)) return rc;
@@ -514,9 +534,8 @@ int run_poses(const pm_framework* fw, const pm_forcefield* ff, const pm_ewald* e
     a.pose_xf = d_pose;
     a.out_e = d_out;
     a.out_g = out_grad ? reinterpret_cast<double*>(base + o_grad) : nullptr;
-    const bool fp64 = precision == PM_FP64;
-    const size_t shm = pose_lds_bytes(a.n_types, a.ns, fp64);
-    const int n_wg = (int)((n + WG / 64 - 1) / (WG / 64));  // one wave per pose
+    const size_t shm = (size_t)pose_lds(es, table, a.nz, a.n_types, a.ns, fp64, out_grad != nullptr).bytes;
+    const int n_wg = (int)n;  // one workgroup per pose
     PM_HIP(hipEventRecord(g_ctx.ev0, g_ctx.stream));
     const int rc = out_grad ? pose_launch<true>(a, n_wg, shm, fp64, es) : pose_launch<false>(a, n_wg, shm, fp64, es);
     if (rc != PM_OK) return rc;
@@ -1689,7 +1708,11 @@ int pm_framework_create(const double f_to_c[9], const int32_t rep[3], int64_t n_
             fw->unit_q[i] = charge[i];
         }
     }
-    std::vector<double4> atoms((size_t)fw->n_rep);
+    // replicated atoms, then their FP32 positions
+    size_t na = (size_t)(fw->n_rep > 0 ? fw->n_rep : 1);
+    const size_t atoms_bytes = na * (sizeof(double4) + sizeof(float4));
+    std::vector<double4> atoms(na + (na + 1) / 2);
+    float4* const atoms_f = reinterpret_cast<float4*>(atoms.data() + na);
     std::vector<int32_t> sp((size_t)fw->n_rep);
     std::vector<double4> uq;
     int64_t k = 0;
@@ -1700,6 +1723,9 @@ int pm_framework_create(const double f_to_c[9], const int32_t rep[3], int64_t n_
                     atoms[k] = make_double4((xf[3 * i] + 1.0 * ra) / rep[0],
                                             (xf[3 * i + 1] + 1.0 * rb) / rep[1],
                                             (xf[3 * i + 2] + 1.0 * rc) / rep[2], fw->unit_q[i]);
+                    const double4& at = atoms[k];
+                    atoms_f[k] = make_float4((float)(at.x - std::floor(at.x)), (float)(at.y - std::floor(at.y)),
+                                             (float)(at.z - std::floor(at.z)), 0.0f);
                     sp[k] = fw->unit_type[i];
                 }
     for (int64_t i = 0; i < n_atoms; ++i) {
@@ -1713,15 +1739,14 @@ int pm_framework_create(const double f_to_c[9], const int32_t rep[3], int64_t n_
         (void)hipFree(fw->d_atoms); (void)hipFree(fw->d_species); (void)hipFree(fw->d_unit_q);
         delete fw;
     };
-    size_t na = (size_t)(fw->n_rep > 0 ? fw->n_rep : 1);
-    if (hipMalloc(&fw->d_atoms, na * sizeof(double4)) != hipSuccess ||
+    if (hipMalloc(&fw->d_atoms, atoms_bytes) != hipSuccess ||
         hipMalloc(&fw->d_species, na * sizeof(int32_t)) != hipSuccess ||
         hipMalloc(&fw->d_unit_q, (uq.empty() ? 1 : uq.size()) * sizeof(double4)) != hipSuccess) {
         cleanup();
         return fail(PM_ERR_OOM, "pm_framework_create: device allocation failed");
     }
     if (fw->n_rep > 0) {
-        if (hipMemcpy(fw->d_atoms, atoms.data(), fw->n_rep * sizeof(double4), hipMemcpyHostToDevice) != hipSuccess ||
+        if (hipMemcpy(fw->d_atoms, atoms.data(), atoms_bytes, hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy(fw->d_species, sp.data(), fw->n_rep * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess) {
             cleanup();
             return fail(PM_ERR_DEVICE, "pm_framework_create: host-to-device copy failed");
@@ -1732,6 +1757,7 @@ int pm_framework_create(const double f_to_c[9], const int32_t rep[3], int64_t n_
         cleanup();
         return fail(PM_ERR_DEVICE, "pm_framework_create: host-to-device copy failed");
     }
+    fw->d_atoms_f = reinterpret_cast<float4*>(fw->d_atoms + na);
     *out = fw;
     return PM_OK;
 }
