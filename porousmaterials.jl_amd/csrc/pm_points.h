@@ -51,6 +51,9 @@ constexpr int GQ = 4;                  // per-type sums per point: d/d eps, d/d 
 constexpr int GK = 3 + 3 * GT;         // per-workgroup partials of a gradient run
 static_assert(7 * GT <= 64, "a tile's cumulative type counts (at most 64, 7 bits each) fill one 64-bit word");
 
+// Points of a grid brick (a pair workgroup's points) per axis.
+constexpr int GRID_BRICK[3] = {8, 8, 4};
+
 // One Widom run or grid of a call (device memory).
 struct RunArgs {
     // replicated box
@@ -94,7 +97,7 @@ struct RunArgs {
     const unsigned char* acc;  // nullable: accessibility grid over the unit cell, i fastest
     int acc_n[3];
     // grid
-    int grid_n[3], brick[3], nbrick[3];
+    int grid_n[3], nbrick[3];
     double grid_q;
     double* grid_d;          // FP64 output, or
     float* grid_f;           // FP32 output
@@ -754,8 +757,21 @@ __device__ __attribute__((always_inline)) inline void tile_close(Candidates<Real
     psr = S.psr;
 }
 
+// The image list in LIST_PARTS parts of (nearly) equally many tiles, part p from
+// tile ceil(p n / LIST_PARTS): a point's FP64 sums run over the tiles of a part,
+// then over the parts, so that the parts may be summed by different waves (the
+// SPLIT kernels) with the same result bit for bit.
+constexpr int LIST_PARTS = 16;
+__device__ inline int part_first_tile(int p, int n_tiles) {
+    return (int)(((long long)p * n_tiles + LIST_PARTS - 1) / LIST_PARTS);
+}
+__device__ inline int tile_part(int t, int n_tiles) {
+    return (int)((double)LIST_PARTS * t / n_tiles);  // exact: quotients are whole or at least 1/n_tiles from it
+}
+
 // LDS of the pair kernels.
 struct PairLds {
+    double* part;           // SPLIT kernels: the parts' sums
     const float4* erfc;     // FP32 kernels
     const double2* erfc64;  // FP64 kernels
     // all-atoms path
@@ -839,7 +855,7 @@ struct TypeSums {
 // tile never spans two bins), so each tile's candidates are taken type by type,
 // with the type's parameters held in registers, and folded into the type's FP64
 // sums once.
-template <int ESM, typename Real, int NT>
+template <int ESM, typename Real, int NT, int SPLIT>
 __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs& a, bool valid, double px, double py, double pz,
                                    int site, const LJC<Real>* s_lj, const double2* s_gc,
                                    const PairLds& L, double& acc_lj, double& acc_sr, bool& ovl,
@@ -884,17 +900,40 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
         const LJC<Real>* const lj_site = s_lj + site;
         const int lj_stride = __builtin_amdgcn_readfirstlane(nsite * (int)sizeof(LJC<Real>));
         const int n_tiles = __builtin_amdgcn_readfirstlane(a.n_tiles);
+        // the current part of the list, its sums and the first tile after it
+        int part = 0, part_end = part_first_tile(1, n_tiles);
+        double part_lj = 0.0, part_sr = 0.0;
+        auto close_part = [&]() {
+            if constexpr (SPLIT == 1) {
+                acc_lj += part_lj;
+                acc_sr += part_sr;
+            } else {
+                // (each part belongs to one wave of the workgroup)
+                if (part_lj != 0.0) L.part[part * 64 + lane] = part_lj;
+                if (part_sr != 0.0) L.part[(LIST_PARTS + part) * 64 + lane] = part_sr;
+            }
+            part_lj = 0.0;
+            part_sr = 0.0;
+        };
         for (int tb = 0; tb < n_tiles; tb += 64) {
             // the tiles of this batch whose bounding sphere meets the wave's
+            // (and that lie in one of the wave's parts)
             bool hit = false;
             if (tb + lane < n_tiles) {
                 const double4 sp = a.tile_sph[tb + lane];
                 const double sx = sp.x - ccx, sy = sp.y - ccy, sz = sp.z - ccz;
                 const double rr = Rc + sp.w;
                 hit = sx * sx + sy * sy + sz * sz < rr * rr;
+                if constexpr (SPLIT > 1)
+                    hit = hit && (tile_part(tb + lane, n_tiles) & (SPLIT - 1)) == (tid >> 6);
             }
             for (unsigned long long hm = __ballot(hit); hm != 0ull; hm &= hm - 1ull) {
                 const int ti = tb + __builtin_ctzll(hm);
+                while (ti >= part_end) {
+                    close_part();
+                    ++part;
+                    part_end = part_first_tile(part + 1, n_tiles);
+                }
                 const int first = rngs[2 * ti], count = rngs[2 * ti + 1];
                 bool keep = false;
                 if (lane < count) {
@@ -925,10 +964,11 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                                                 small, S);
                 }
                 tile_close<ESM, Real>(C, m, P, lj_stride, lj_site, is_lj, r2lj, r2sr, et, small, ovl, S.plj, S.psr);
-                acc_lj += (double)S.plj;
-                acc_sr += (double)S.psr;
+                part_lj += (double)S.plj;
+                part_sr += (double)S.psr;
             }
         }
+        close_part();
     } else {
         const int n_atoms = a.n_atoms;
         for (int base = 0; base < n_atoms; base += TILE) {
@@ -983,10 +1023,28 @@ constexpr int pair_waves() {
     return sizeof(Real) == 4 && NT == 6 ? 4 : 1;
 }
 
+// Work-items of a pair workgroup.  SPLIT = 1: a slice of WG points, a wave for 64
+// of them.  SPLIT = 4, 16: 64 points, whose image list SPLIT waves share out.
+constexpr int pair_wg(int split) { return split == 16 ? 1024 : WG; }
+// LDS of the SPLIT kernels for the parts' LJ and real-space sums [part][point]
+// and the waves' overlap masks.
+constexpr int pair_lds_parts(int split) {
+    return split > 1 ? (2 * LIST_PARTS * 64 + split) * (int)sizeof(double) : 0;
+}
+
 // NT = 0: energies.  NT > 0: a gradient run of at most NT framework types.
-template <typename Real, int NT>
-__global__ __launch_bounds__(WG, (pair_waves<Real, NT>())) void point_pair_kernel(GroupArgs g, int atoms_off) {
+// SPLIT (energies, image-list path): a small launch leaves most of the 1024
+// SIMDs without a wave while a few walk the whole list, one dependent load after
+// another; with the list shared out each wave's chain is SPLIT times shorter, for
+// SPLIT times the tile tests and table loads (1000 CH4 insertions, 424 atoms: 70
+// -> 28 us; 1000 CO2, 600 atoms: 182 -> 55, in FP64 252 -> 80).  The first wave
+// adds the parts' sums from LDS.
+template <typename Real, int NT, int SPLIT>
+__global__ __launch_bounds__(pair_wg(SPLIT), (pair_waves<Real, NT>())) void point_pair_kernel(GroupArgs g, int extra_off) {
     constexpr bool GRAD = NT > 0;
+    static_assert(!GRAD || SPLIT == 1, "gradient runs are not split");
+    constexpr int SUB = SPLIT == 1 ? 1 : WG / 64;  // workgroups per slice or brick
+    constexpr int NTH = pair_wg(SPLIT);
     extern __shared__ __align__(16) unsigned char smem[];
     float4* s_erfc = reinterpret_cast<float4*>(smem);
     double2* s_erfc64 = reinterpret_cast<double2*>(smem);
@@ -994,18 +1052,21 @@ __global__ __launch_bounds__(WG, (pair_waves<Real, NT>())) void point_pair_kerne
     PairLds L;
     L.erfc = s_erfc;
     L.erfc64 = s_erfc64;
-    L.c = reinterpret_cast<double4*>(smem + atoms_off);
+    L.part = reinterpret_cast<double*>(smem + extra_off);
+    L.c = reinterpret_cast<double4*>(smem + extra_off);
     L.t = reinterpret_cast<int*>(L.c + TILE);
 
     const int tid = threadIdx.x;
+    const unsigned wg = blockIdx.x / SUB;                                            // slice or brick
+    const int pt = SPLIT == 1 ? tid : (int)(blockIdx.x % SUB) * 64 + (tid & 63);     // point of it
     int si;
     uint4 it = make_uint4(0u, 0u, 0u, 0u);
     if (g.mode == MODE_WIDOM) {
-        if (blockIdx.x >= *g.n_items) return;  // the whole workgroup leaves
-        it = g.items[blockIdx.x];
+        if (wg >= *g.n_items) return;  // the whole workgroup leaves
+        it = g.items[wg];
         si = (int)it.z;
     } else {
-        si = find_segment<SEG_BY_WG>(g.segs, g.n_seg, blockIdx.x);
+        si = find_segment<SEG_BY_WG>(g.segs, g.n_seg, wg);
     }
     const SegArgs sg = g.segs[si];
     const RunArgs& a = g.runs[sg.run];
@@ -1017,19 +1078,21 @@ __global__ __launch_bounds__(WG, (pair_waves<Real, NT>())) void point_pair_kerne
     double px, py, pz;
     int site;
     if (g.mode == MODE_WIDOM) {
-        const unsigned k = g.point_off[it.x] + it.y * WG + tid;
+        const unsigned k = g.point_off[it.x] + it.y * WG + pt;
         valid = k < g.point_off[it.x + 1];
         pid = valid ? (long long)g.order[k] : sg.slot_base;
         const double4 p = valid ? g.pos[pid] : make_double4(0.0, 0.0, 0.0, 0.0);
         px = p.x; py = p.y; pz = p.z;
         site = (int)((pid - sg.slot_base) % a.nsite);
     } else {
-        const int lb = (int)blockIdx.x - sg.wg_base;
+        const int lb = (int)wg - sg.wg_base;
         const int nb0 = a.nbrick[0], nb1 = a.nbrick[1];
         const int bi = lb % nb0, bj = (lb / nb0) % nb1, bk = lb / (nb0 * nb1);
-        const int i0 = bi * a.brick[0], j0 = bj * a.brick[1], k0 = bk * a.brick[2];
-        const int ti = tid % a.brick[0], tj = (tid / a.brick[0]) % a.brick[1], tk = tid / (a.brick[0] * a.brick[1]);
-        const int i = i0 + ti, j = j0 + tj, k = k0 + tk;
+        // a wave's 64 points: a 4 x 4 x 4 part of the brick (planes of 8 x 8 x 1
+        // have a 1.3 times larger sphere: 76 -> 64 us for 50^3 CH4 points)
+        const int i = bi * GRID_BRICK[0] + (pt & 64 ? 4 : 0) + (pt & 3);
+        const int j = bj * GRID_BRICK[1] + (pt & 128 ? 4 : 0) + ((pt >> 2) & 3);
+        const int k = bk * GRID_BRICK[2] + ((pt >> 4) & 3);
         const int n1 = a.grid_n[0], n2 = a.grid_n[1], n3 = a.grid_n[2];
         valid = i < n1 && j < n2 && k < n3;
         pid = sg.slot_base + (valid ? (long long)i + (long long)n1 * ((long long)j + (long long)n2 * k) : 0);
@@ -1038,19 +1101,23 @@ __global__ __launch_bounds__(WG, (pair_waves<Real, NT>())) void point_pair_kerne
         pz = grid_coord(k, n3, a.repd[2]);
         site = 0;
     }
+    if constexpr (SPLIT > 1)
+        if (__ballot(valid) == 0ull) return;  // the whole workgroup: its waves hold the same points
     const int n_tab = a.n_types * a.nsite;
     const LJC<Real>* gtab = reinterpret_cast<const LJC<Real>*>(a.ljtab);
-    for (int t = tid; t < n_tab; t += WG) s_lj[t] = gtab[t];
+    for (int t = tid; t < n_tab; t += NTH) s_lj[t] = gtab[t];
     if constexpr (GRAD) {
         const double2* gc = reinterpret_cast<const double2*>(a.gtab);
-        for (int t = tid; t < n_tab; t += WG) s_gc[t] = gc[t];
+        for (int t = tid; t < n_tab; t += NTH) s_gc[t] = gc[t];
     }
     if constexpr (sizeof(Real) == 4)
         if (a.esm != 0)
-            for (int t = tid; t < ERFC_TAB; t += WG) s_erfc[t] = a.erfc_tab[t];
+            for (int t = tid; t < ERFC_TAB; t += NTH) s_erfc[t] = a.erfc_tab[t];
     if constexpr (sizeof(Real) == 8)
         if (a.esm != 0)
-            for (int t = tid; t < ERFC64_TAB; t += WG) s_erfc64[t] = a.erfc64_tab[t];
+            for (int t = tid; t < ERFC64_TAB; t += NTH) s_erfc64[t] = a.erfc64_tab[t];
+    if constexpr (SPLIT > 1)
+        for (int t = tid; t < 2 * LIST_PARTS * 64; t += NTH) L.part[t] = 0.0;
     __syncthreads();
 
     double acc_lj = 0.0, acc_sr = 0.0;
@@ -1058,14 +1125,34 @@ __global__ __launch_bounds__(WG, (pair_waves<Real, NT>())) void point_pair_kerne
     unsigned long long n_cand = 0;
     TypeSums<Real, (NT > 0 ? NT : 1)> ts;
     if (a.esm == 0)
-        chunk_pairs<0, Real, NT>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
+        chunk_pairs<0, Real, NT, SPLIT>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
                                  n_cand, ts);
     else if (a.esm == 1)
-        chunk_pairs<1, Real, NT>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
+        chunk_pairs<1, Real, NT, SPLIT>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
                                  n_cand, ts);
     else
-        chunk_pairs<2, Real, NT>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
+        chunk_pairs<2, Real, NT, SPLIT>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
                                  n_cand, ts);
+    if (g.cand_pairs != nullptr) {
+        const unsigned long long m = __ballot(valid);
+        if ((tid & 63) == 0 && m != 0ull)
+            atomicAdd(g.cand_pairs, (unsigned long long)__popcll(m) * n_cand);
+    }
+    if constexpr (SPLIT > 1) {
+        // the first wave adds up the parts' sums, in the order of the list
+        unsigned long long* const s_ovl = reinterpret_cast<unsigned long long*>(L.part + 2 * LIST_PARTS * 64);
+        const unsigned long long om = __ballot(ovl);
+        if ((tid & 63) == 0) s_ovl[tid >> 6] = om;
+        __syncthreads();
+        if (tid >= 64) return;
+        unsigned long long any = 0ull;
+        for (int w = 0; w < SPLIT; ++w) any |= s_ovl[w];
+        ovl = (any >> tid) & 1ull;
+        for (int p = 0; p < LIST_PARTS; ++p) {
+            acc_lj += L.part[p * 64 + tid];
+            acc_sr += L.part[(LIST_PARTS + p) * 64 + tid];
+        }
+    }
     if (valid) {
         g.out_lj[pid] = ovl ? INFINITY : acc_lj;
         g.out_sr[pid] = acc_sr;
@@ -1080,11 +1167,6 @@ __global__ __launch_bounds__(WG, (pair_waves<Real, NT>())) void point_pair_kerne
                 o[(2 * GT + k) * gs] = ts.g[2 * NT + k];
             }
         }
-    }
-    if (g.cand_pairs != nullptr) {
-        const unsigned long long m = __ballot(valid);
-        if ((tid & 63) == 0 && m != 0ull)
-            atomicAdd(g.cand_pairs, (unsigned long long)__popcll(m) * n_cand);
     }
 }
 

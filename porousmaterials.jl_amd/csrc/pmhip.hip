@@ -920,9 +920,8 @@ int grid_prepare(const pm_grid_run& in, PointRun& r) {
     }
     const bool es = fw->charged && pr->charged;
     if (es && !ew) return fail(PM_ERR_ARG, "pm_energy_grid: charged probe needs an Ewald handle");
-    const int brick[3] = {8, 8, 4};
     int nbrick[3];
-    for (int i = 0; i < 3; ++i) nbrick[i] = (in.n_pts[i] + brick[i] - 1) / brick[i];
+    for (int i = 0; i < 3; ++i) nbrick[i] = (in.n_pts[i] + GRID_BRICK[i] - 1) / GRID_BRICK[i];
     const long long n_bricks = (long long)nbrick[0] * nbrick[1] * nbrick[2];
     const long long n_pts = (long long)in.n_pts[0] * in.n_pts[1] * in.n_pts[2];
     if (n_bricks > INT32_MAX / 2 || n_pts > (1LL << 40))
@@ -940,7 +939,6 @@ int grid_prepare(const pm_grid_run& in, PointRun& r) {
     fill_run_pair(a, fw, pr->site[0].lj ? ff : nullptr, es ? ew : nullptr, es, 1, pr->site);
     for (int i = 0; i < 3; ++i) {
         a.grid_n[i] = in.n_pts[i];
-        a.brick[i] = brick[i];
         a.nbrick[i] = nbrick[i];
     }
     a.grid_q = pr->site[0].q;
@@ -948,7 +946,7 @@ int grid_prepare(const pm_grid_run& in, PointRun& r) {
     double ed[3][3];
     for (int d = 0; d < 3; ++d) {
         const double step =
-            in.n_pts[d] > 1 ? (double)(brick[d] - 1) / (double)(in.n_pts[d] - 1) / fw->rep[d] : 0.0;
+            in.n_pts[d] > 1 ? (double)(GRID_BRICK[d] - 1) / (double)(in.n_pts[d] - 1) / fw->rep[d] : 0.0;
         for (int i = 0; i < 3; ++i) ed[d][i] = fw->F[3 * d + i] * step;
     }
     a.chunk_r = half_diagonal(ed[0], ed[1], ed[2]);
@@ -957,9 +955,28 @@ int grid_prepare(const pm_grid_run& in, PointRun& r) {
     return PM_OK;
 }
 
-template <typename Real, int NT>
-void pair_launch_t(const GroupArgs& g, int n_wg, size_t shm, int atoms_off) {
-    hipLaunchKernelGGL((point_pair_kernel<Real, NT>), dim3(n_wg), dim3(WG), shm, g_ctx.stream, g, atoms_off);
+template <typename Real, int NT, int SPLIT = 1>
+void pair_launch_t(const GroupArgs& g, int n_wg, size_t shm, int extra_off) {
+    constexpr int sub = SPLIT == 1 ? 1 : WG / 64;
+    hipLaunchKernelGGL((point_pair_kernel<Real, NT, SPLIT>), dim3(n_wg * sub), dim3(pair_wg(SPLIT)),
+                       shm + pair_lds_parts(SPLIT), g_ctx.stream, g, extra_off);
+}
+
+// Waves that share out the image list of 64 points, by the 64-point waves of the
+// launch: one from a wave per SIMD on, four below, sixteen where even four leave
+// most SIMDs idle.  Pair kernel with 1, 4 and 16 (us): 156 waves (CH4 insertions)
+// 153, 85, 52; 469 (CO2) 146, 99, 126; 469 (CH4) 121, 76, 119; 1406 (CO2) 142,
+// 129, 335, in FP64 212, 238, 367; 1562 (CH4) 118, 129, 361; 2197 (50^3 grid) 64,
+// 131, 447.
+int pair_split(long long n_waves) { return n_waves >= 1024 ? 1 : n_waves >= 192 ? 4 : 16; }
+
+template <typename Real>
+void pair_launch_plain(const GroupArgs& g, int n_wg, size_t shm, int extra_off, int split) {
+    switch (split) {
+        case 16: pair_launch_t<Real, 0, 16>(g, n_wg, shm, extra_off); break;
+        case 4: pair_launch_t<Real, 0, 4>(g, n_wg, shm, extra_off); break;
+        default: pair_launch_t<Real, 0>(g, n_wg, shm, extra_off); break;
+    }
 }
 
 // Compiled type counts of the gradient kernels: a gradient run of n_gt
@@ -968,12 +985,12 @@ void pair_launch_t(const GroupArgs& g, int n_wg, size_t shm, int atoms_off) {
 int grad_nt(int n_gt) { return n_gt <= 2 ? 2 : n_gt <= 4 ? 4 : n_gt <= 6 ? 6 : GT; }
 
 template <typename Real>
-void pair_launch_grad(const GroupArgs& g, int n_wg, size_t shm, int atoms_off, int nt) {
+void pair_launch_grad(const GroupArgs& g, int n_wg, size_t shm, int extra_off, int nt) {
     switch (nt) {
-        case 2: pair_launch_t<Real, 2>(g, n_wg, shm, atoms_off); break;
-        case 4: pair_launch_t<Real, 4>(g, n_wg, shm, atoms_off); break;
-        case 6: pair_launch_t<Real, 6>(g, n_wg, shm, atoms_off); break;
-        default: pair_launch_t<Real, GT>(g, n_wg, shm, atoms_off); break;
+        case 2: pair_launch_t<Real, 2>(g, n_wg, shm, extra_off); break;
+        case 4: pair_launch_t<Real, 4>(g, n_wg, shm, extra_off); break;
+        case 6: pair_launch_t<Real, 6>(g, n_wg, shm, extra_off); break;
+        default: pair_launch_t<Real, GT>(g, n_wg, shm, extra_off); break;
     }
 }
 
@@ -1332,9 +1349,9 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
     g.g_stride = max_slots;
     bool all_fast = true;
     for (const PointRun& r : runs) all_fast = all_fast && r.ra.fast != 0;
-    const int atoms_off =
+    const int extra_off =
         (fp64 ? pair_lds_fixed<double>() : pair_lds_fixed<float>()) + (int)((std::max<size_t>(lj_lds, 16) + 15) / 16 * 16);
-    const size_t shm = (size_t)atoms_off + (all_fast ? 0 : PAIR_LDS_ATOMS);
+    const size_t shm = (size_t)extra_off + (all_fast ? 0 : PAIR_LDS_ATOMS);
 
     // the counter is cleared by a kernel (Widom: the first cell-count fill),
     // which a caller's graph capture records safely
@@ -1373,11 +1390,16 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
         }
         PM_HIP(hipEventRecord(g_ctx.evp0, g_ctx.stream));
         if (grad) {
-            if (fp64) pair_launch_grad<double>(g, (int)pair_wg, shm, atoms_off, nt_grad);
-            else pair_launch_grad<float>(g, (int)pair_wg, shm, atoms_off, nt_grad);
+            if (fp64) pair_launch_grad<double>(g, (int)pair_wg, shm, extra_off, nt_grad);
+            else pair_launch_grad<float>(g, (int)pair_wg, shm, extra_off, nt_grad);
         } else {
-            if (fp64) pair_launch_t<double, 0>(g, (int)pair_wg, shm, atoms_off);
-            else pair_launch_t<float, 0>(g, (int)pair_wg, shm, atoms_off);
+            // (a run on the all-atoms path is not split, nor one whose tables fill
+            // the LDS that any kernel may take)
+            const long long n_waves = (widom ? gr.n_slots : gr.n_wg * WG) / 64;
+            const bool can_split = all_fast && shm + pair_lds_parts(16) <= 65536;
+            const int split = can_split ? pair_split(n_waves) : 1;
+            if (fp64) pair_launch_plain<double>(g, (int)pair_wg, shm, extra_off, split);
+            else pair_launch_plain<float>(g, (int)pair_wg, shm, extra_off, split);
         }
         PM_HIP(hipEventRecord(g_ctx.evp1, g_ctx.stream));
         const long long slot_wg = (gr.n_slots + WG - 1) / WG;
