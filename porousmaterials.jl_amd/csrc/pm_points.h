@@ -83,6 +83,8 @@ struct RunArgs {
     int Ma, Mb, Mc;
     const double2* A;        // wt * N_R * S(m), zeros off the kept set
     const int2* krows;       // per (ma, mb) row: kept mc range (lo > hi: empty row)
+    const double* fold;      // folded coefficients (fold_box_kernel)
+    const int2* frows;
     // Widom
     unsigned long long seed;
     long long n_per_block;
@@ -1083,7 +1085,7 @@ __global__ __launch_bounds__(pair_wg(SPLIT), (pair_waves<Real, NT>())) void poin
         pid = valid ? (long long)g.order[k] : sg.slot_base;
         const double4 p = valid ? g.pos[pid] : make_double4(0.0, 0.0, 0.0, 0.0);
         px = p.x; py = p.y; pz = p.z;
-        site = (int)((pid - sg.slot_base) % a.nsite);
+        site = (int)((unsigned)(pid - sg.slot_base) % (unsigned)a.nsite);  // (fewer than 2^32 slots)
     } else {
         const int lb = (int)wg - sg.wg_base;
         const int nb0 = a.nbrick[0], nb1 = a.nbrick[1];
@@ -1175,6 +1177,13 @@ __device__ inline double2 cmul(double2 a, double2 b) {
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
+// (c, s) of an angle to those of the angle plus another
+__device__ inline void rotate_phase(double& c, double& s, double c1, double s1) {
+    const double t = fma(c, c1, -(s * s1));
+    s = fma(s, c1, c * s1);
+    c = t;
+}
+
 // Points per work-item of the Fourier kernel: the points of a work-item share
 // every coefficient load and the loop control, and their Horner chains
 // interleave.
@@ -1194,20 +1203,11 @@ __device__ inline FourierPoint fourier_point(const GroupArgs& g, const SegArgs& 
     P.pid = pid;
     const long long lp = pid - sg.slot_base;
     bool valid = lp < sg.n_slots;
-    double x = 0.0, y = 0.0, z = 0.0;
-    int site = 0;
-    if (g.mode == MODE_WIDOM) {
-        const double4 p = valid ? g.pos[pid] : make_double4(0.0, 0.0, 0.0, 0.0);
-        valid = valid && p.w != 0.0;
-        x = p.x; y = p.y; z = p.z;
-        site = (int)(lp % a.nsite);
-    } else if (valid) {
-        const int n1 = a.grid_n[0], n2 = a.grid_n[1], n3 = a.grid_n[2];
-        const long long i = lp % n1, j = (lp / n1) % n2, k = lp / ((long long)n1 * n2);
-        x = grid_coord((double)i, n1, a.repd[0]);
-        y = grid_coord((double)j, n2, a.repd[1]);
-        z = grid_coord((double)k, n3, a.repd[2]);
-    }
+    const double4 p = valid ? g.pos[pid] : make_double4(0.0, 0.0, 0.0, 0.0);
+    valid = valid && p.w != 0.0;
+    const double x = p.x, y = p.y, z = p.z;
+    // (a launch group holds fewer than 2^32 slots: a 64-bit remainder is 130 instructions)
+    const unsigned site = (unsigned)lp % (unsigned)a.nsite;
     P.valid = valid;
     P.charged = valid && ((a.site_q_mask >> site) & 1u);
     double t0 = x * a.repd[0], t1 = y * a.repd[1], t2 = z * a.repd[2];
@@ -1225,15 +1225,139 @@ __device__ inline FourierPoint fourier_point(const GroupArgs& g, const SegArgs& 
     return P;
 }
 
+// Folded coefficients of the Fourier part (fold_box_kernel): with z = c - i s on
+// each axis, the kept entries (ma, +-mb, +-mc) of the box combine to
+//   z_a^ma [ (Uc c_mc + Us s_mc) cos(mb b) + (Vc c_mc + Vs s_mc) sin(mb b) ],
+// c_mc, s_mc = cos, sin(2 pi mc u_c), Uc, Us, Vc, Vs complex.  Stream, row by row
+// of (ma, mb >= 0): Uc, Vc of mc = 0 (4 doubles), then Uc, Us, Vc, Vs of mc = 1
+// .. hi (8 doubles each); frows: per row the stream offset and hi (-1: empty row).
+constexpr int FOLD_HEAD = 4, FOLD_CELL = 8, FOLD_PAD = 16;
+
+__global__ void fold_box_kernel(const double2* box, int Ma, int Mb, int Mc, const int2* frows, double* fold) {
+    const long long n = (long long)(Ma + 1) * (Mb + 1) * (Mc + 1);
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const int mc = (int)(t % (Mc + 1)), mb = (int)(t / (Mc + 1) % (Mb + 1)), ma = (int)(t / (Mc + 1) / (Mb + 1));
+    const int2 fr = frows[ma * (Mb + 1) + mb];
+    if (mc > fr.y) return;
+    auto A = [&](int b, int c) { return box[((long long)ma * (2 * Mb + 1) + b + Mb) * (2 * Mc + 1) + c + Mc]; };
+    const double2 zero = make_double2(0.0, 0.0);
+    const double2 pp = A(mb, mc), pm = mc > 0 ? A(mb, -mc) : zero, mp = mb > 0 ? A(-mb, mc) : zero,
+                  mm = mb > 0 && mc > 0 ? A(-mb, -mc) : zero;
+    // sums over the signs, times -i per sine
+    const double uc[2] = {(pp.x + pm.x) + (mp.x + mm.x), (pp.y + pm.y) + (mp.y + mm.y)};
+    const double us[2] = {(pp.y - pm.y) + (mp.y - mm.y), -((pp.x - pm.x) + (mp.x - mm.x))};
+    const double vc[2] = {(pp.y + pm.y) - (mp.y + mm.y), -((pp.x + pm.x) - (mp.x + mm.x))};
+    const double vs[2] = {-((pp.x - pm.x) - (mp.x - mm.x)), -((pp.y - pm.y) - (mp.y - mm.y))};
+    double* o = fold + fr.x;
+    if (mc > 0) o += FOLD_HEAD + (mc - 1) * FOLD_CELL;
+    for (int d = 0; d < 2; ++d) {
+        o[d] = uc[d];
+        if (mc == 0) {
+            o[2 + d] = mb > 0 ? vc[d] : 0.0;
+        } else {
+            o[2 + d] = us[d];
+            o[4 + d] = mb > 0 ? vc[d] : 0.0;
+            o[6 + d] = mb > 0 ? vs[d] : 0.0;
+        }
+    }
+}
+
+// f(0), f(1), ... as compile-time constants while it returns true
+template <typename F, int... I>
+__device__ __attribute__((always_inline)) inline void while_each(F& f, std::integer_sequence<int, I...>) {
+    (void)(f(std::integral_constant<int, I>{}) && ...);
+}
+
+// One (ma, mb) row of the folded coefficients: T += U cos(mb b) + V sin(mb b)
+// (V = false: mb = 0, where V is zero).
+template <int MC, bool V>
+__device__ __attribute__((always_inline)) inline void fourier_row(const gconst_ptr<double> co, int hi, const double (&cc)[FOURIER_PTS][MC > 0 ? MC + 1 : 2],
+                                   const double (&sc)[FOURIER_PTS][MC > 0 ? MC + 1 : 2],
+                                   const double (&cb)[FOURIER_PTS], const double (&sb)[FOURIER_PTS],
+                                   double (&Tr)[FOURIER_PTS], double (&Ti)[FOURIER_PTS]) {
+    double Ur[FOURIER_PTS], Ui[FOURIER_PTS], Vr[FOURIER_PTS], Vi[FOURIER_PTS];
+#pragma unroll
+    for (int k = 0; k < FOURIER_PTS; ++k) {
+        Ur[k] = co[0];
+        Ui[k] = co[1];
+        Vr[k] = co[2];
+        Vi[k] = co[3];
+    }
+    gconst_ptr<double> e = co + FOLD_HEAD;
+    double w[FOLD_CELL];  // the next cell (past the row's end: the next row's or the padding)
+#pragma unroll
+    for (int d = 0; d < FOLD_CELL; ++d) w[d] = e[d];
+    auto cell = [&](const double (&cm)[FOURIER_PTS], const double (&sm)[FOURIER_PTS]) {
+        double v[FOLD_CELL];
+#pragma unroll
+        for (int d = 0; d < FOLD_CELL; ++d) v[d] = w[d];
+        e += FOLD_CELL;
+#pragma unroll
+        for (int d = 0; d < FOLD_CELL; ++d) w[d] = e[d];
+#pragma unroll
+        for (int k = 0; k < FOURIER_PTS; ++k) {
+            Ur[k] = fma(v[2], sm[k], fma(v[0], cm[k], Ur[k]));
+            Ui[k] = fma(v[3], sm[k], fma(v[1], cm[k], Ui[k]));
+            if constexpr (V) {
+                Vr[k] = fma(v[6], sm[k], fma(v[4], cm[k], Vr[k]));
+                Vi[k] = fma(v[7], sm[k], fma(v[5], cm[k], Vi[k]));
+            }
+        }
+        // used here, so that the load of the next cell is issued before this one's FMAs
+        asm volatile("" ::"s"(w[0]), "s"(w[1]), "s"(w[2]), "s"(w[3]), "s"(w[4]), "s"(w[5]), "s"(w[6]), "s"(w[7]));
+    };
+    if constexpr (MC > 0) {
+        // (unrolled by the pack: the basis stays in registers)
+        auto step = [&](auto mi) {
+            constexpr int m = decltype(mi)::value + 1;
+            if (m > hi) return false;
+            double cm[FOURIER_PTS], sm[FOURIER_PTS];
+#pragma unroll
+            for (int k = 0; k < FOURIER_PTS; ++k) {
+                cm[k] = cc[k][m];
+                sm[k] = sc[k][m];
+            }
+            cell(cm, sm);
+            return true;
+        };
+        while_each(step, std::make_integer_sequence<int, MC>{});
+    } else {
+        double cm[FOURIER_PTS], sm[FOURIER_PTS];
+#pragma unroll
+        for (int k = 0; k < FOURIER_PTS; ++k) {
+            cm[k] = cc[k][1];
+            sm[k] = sc[k][1];
+        }
+        for (int m = 1; m <= hi; ++m) {
+            cell(cm, sm);
+#pragma unroll
+            for (int k = 0; k < FOURIER_PTS; ++k) rotate_phase(cm[k], sm[k], cc[k][1], sc[k][1]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < FOURIER_PTS; ++k) {
+        Tr[k] = fma(Ur[k], cb[k], Tr[k]);
+        Ti[k] = fma(Ui[k], cb[k], Ti[k]);
+        if constexpr (V) {
+            Tr[k] = fma(Vr[k], sb[k], Tr[k]);
+            Ti[k] = fma(Vi[k], sb[k], Ti[k]);
+        }
+    }
+}
+
 // Fourier part per point: sum_m Re(A_m e^{-i 2 pi m.u}), u = R o x (unit-cell
-// fractional), FP64.  With z_a = e^{-i 2 pi u_a}: for every (ma, mb) row the
-// sum over the row's kept mc range is evaluated as two polynomials by Horner,
-// sum_{mc >= 0} A_mc z_c^mc and z_c^* sum_{j >= 1} A_{-j} (z_c^*)^{j-1}, and
-// multiplied by z_a^ma z_b^mb, carried along the rows by recurrence.  The
-// coefficients are the same for every lane: they are read by scalar loads
-// (through the scalar cache, into SGPR operands of the FMAs) rather than
-// broadcast from LDS, which would move 64 copies of each one.  Point slots of
-// a segment start at a multiple of WG, so a workgroup lies in one segment.
+// fractional), FP64, from the folded coefficients: two FMAs per kept k-vector
+// and point, where complex Horner steps took four.  The coefficients are the same
+// for every lane: they are read by scalar loads (through the scalar cache, into
+// SGPR operands of the FMAs), a cell ahead of their use.  The cosines and sines
+// of the c axis are held in registers (MC >= the runs' Mc) or, MC = 0, stepped
+// along each row by the same recurrence, with the same bits.  Bound by FP64
+// issue: of some 3700 instructions per wave (461 k-vectors, 128 points) half are
+// these FMAs, a quarter the 33 rows' own, a quarter the phases.  3e6 points, 461
+// k-vectors: 379 -> 212 us; 48 screening runs: 424 -> 297.  Point slots of a
+// segment start at a multiple of WG, so a workgroup lies in one segment.
+template <int MC>
 __global__ __launch_bounds__(FOURIER_WG) void point_fourier_kernel(GroupArgs g) {
     const int tid = threadIdx.x;
     const long long p0 = (long long)blockIdx.x * WG;  // WG slots per workgroup, FOURIER_PTS per work-item
@@ -1241,100 +1365,46 @@ __global__ __launch_bounds__(FOURIER_WG) void point_fourier_kernel(GroupArgs g) 
     const RunArgs& a = g.runs[sg.run];
     if (a.esm == 0) return;  // uniform: the whole workgroup leaves
     FourierPoint P[FOURIER_PTS];
-    double nzr[FOURIER_PTS], nzi[FOURIER_PTS];
+    double cc[FOURIER_PTS][MC > 0 ? MC + 1 : 2], sc[FOURIER_PTS][MC > 0 ? MC + 1 : 2];
+    double ca[FOURIER_PTS], sa[FOURIER_PTS], acc[FOURIER_PTS];
 #pragma unroll
     for (int k = 0; k < FOURIER_PTS; ++k) {
         P[k] = fourier_point(g, sg, a, p0 + tid + k * FOURIER_WG);
-        // opaque to the optimiser, which would fold -q * -z back to q * z
-        nzr[k] = -P[k].zr;
-        nzi[k] = -P[k].zi;
-        asm volatile("" : "+v"(nzr[k]));
-        asm volatile("" : "+v"(nzi[k]));
+        cc[k][0] = 1.0;
+        sc[k][0] = 0.0;
+        cc[k][1] = P[k].zr;
+        sc[k][1] = -P[k].zi;
+#pragma unroll
+        for (int m = 2; m <= MC; ++m) {
+            cc[k][m] = cc[k][m - 1];
+            sc[k][m] = sc[k][m - 1];
+            rotate_phase(cc[k][m], sc[k][m], cc[k][1], sc[k][1]);
+        }
+        ca[k] = 1.0;
+        sa[k] = acc[k] = 0.0;
     }
     // wave-uniform: scalar loop control (the loads are not provably uniform)
-    const int Ma = __builtin_amdgcn_readfirstlane(a.Ma), Mb = __builtin_amdgcn_readfirstlane(a.Mb),
-              Mc = __builtin_amdgcn_readfirstlane(a.Mc);
-    // per m_a: T = sum_mb z_b^(mb + Mb) R(ma, mb) by Horner in z_b over the rows
-    // (mb from Mb down to -Mb), then acc += Re(z_a^ma z_b^-Mb T)
-    double2 Eb_neg[FOURIER_PTS], Pa[FOURIER_PTS];  // z_b^-Mb, z_a^ma
-    double acc[FOURIER_PTS];
-#pragma unroll
-    for (int k = 0; k < FOURIER_PTS; ++k) {
-        Eb_neg[k] = make_double2(1.0, 0.0);
-        const double2 Eb_c = make_double2(P[k].Eb.x, -P[k].Eb.y);
-        for (int q = 0; q < Mb; ++q) Eb_neg[k] = cmul(Eb_neg[k], Eb_c);
-        Pa[k] = make_double2(1.0, 0.0);
-        acc[k] = 0.0;
-    }
-
-    const int rowlen = 2 * Mc + 1, nb = 2 * Mb + 1;
-    // (plain scalars through these pointers: the vector types have no copy
-    // from that address space)
-    const gconst_ptr<double> Abox = uniform_ptr(reinterpret_cast<const double*>(a.A));
-    const gconst_ptr<int> krows = uniform_ptr(reinterpret_cast<const int*>(a.krows));
+    const int Ma = __builtin_amdgcn_readfirstlane(a.Ma), Mb = __builtin_amdgcn_readfirstlane(a.Mb);
+    const gconst_ptr<double> fold = uniform_ptr(a.fold);
+    gconst_ptr<int> fr = uniform_ptr(reinterpret_cast<const int*>(a.frows));
     for (int ma = 0; ma <= Ma; ++ma) {
-        double Tr[FOURIER_PTS], Ti[FOURIER_PTS];
+        double Tr[FOURIER_PTS], Ti[FOURIER_PTS], cb[FOURIER_PTS], sb[FOURIER_PTS];
 #pragma unroll
-        for (int k = 0; k < FOURIER_PTS; ++k) Tr[k] = Ti[k] = 0.0;
-        for (int jb = nb - 1; jb >= 0; --jb) {
-            const int r = ma * nb + jb;
-            const int2 lh = make_int2(krows[2 * r], krows[2 * r + 1]);
-            double Rr[FOURIER_PTS], Ri[FOURIER_PTS];  // the row's sum_mc A z_c^mc
+        for (int k = 0; k < FOURIER_PTS; ++k) {
+            Tr[k] = Ti[k] = sb[k] = 0.0;
+            cb[k] = 1.0;
+        }
+        if (fr[1] >= 0) fourier_row<MC, false>(fold + fr[0], fr[1], cc, sc, cb, sb, Tr, Ti);
+        fr += 2;
+        for (int mb = 1; mb <= Mb; ++mb, fr += 2) {
 #pragma unroll
-            for (int k = 0; k < FOURIER_PTS; ++k) Rr[k] = Ri[k] = 0.0;
-            if (lh.x <= lh.y) {
-                const gconst_ptr<double> row = Abox + 2 * ((long long)r * rowlen + Mc);  // mc in [-Mc, Mc]
-                // Every inner FMA carries a negated operand (-q * -z where the sign
-                // is not wanted), which keeps it in the three-operand form that
-                // takes the scalar coefficient directly; the products are exact
-                // negations of each other, so the sums are unchanged.
-                double qr[FOURIER_PTS], qi[FOURIER_PTS];  // sum_{mc >= 0} A_mc z^mc
-#pragma unroll
-                for (int k = 0; k < FOURIER_PTS; ++k) qr[k] = qi[k] = 0.0;
-#pragma unroll 2
-                for (int mc = lh.y; mc >= 0; --mc) {
-                    const double Ar = row[2 * mc], Ai = row[2 * mc + 1];
-#pragma unroll
-                    for (int k = 0; k < FOURIER_PTS; ++k) {
-                        const double nr = fma(qr[k], P[k].zr, fma(-qi[k], P[k].zi, Ar));
-                        qi[k] = fma(qr[k], P[k].zi, fma(-qi[k], nzr[k], Ai));
-                        qr[k] = nr;
-                    }
-                }
-                double nr_[FOURIER_PTS], ni_[FOURIER_PTS];  // sum_{j >= 1} A_{-j} (z*)^{j-1}
-#pragma unroll
-                for (int k = 0; k < FOURIER_PTS; ++k) nr_[k] = ni_[k] = 0.0;
-#pragma unroll 2
-                for (int j = -lh.x; j >= 1; --j) {
-                    const double Ar = row[-2 * j], Ai = row[-2 * j + 1];
-#pragma unroll
-                    for (int k = 0; k < FOURIER_PTS; ++k) {
-                        const double tr = fma(nr_[k], P[k].zr, fma(-ni_[k], nzi[k], Ar));
-                        ni_[k] = fma(ni_[k], P[k].zr, fma(-nr_[k], P[k].zi, Ai));
-                        nr_[k] = tr;
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < FOURIER_PTS; ++k) {
-                    // R = q + z* n
-                    const double zr = P[k].zr, zi = P[k].zi;
-                    Rr[k] = qr[k] + (zr * nr_[k] + zi * ni_[k]);
-                    Ri[k] = qi[k] + (zr * ni_[k] - zi * nr_[k]);
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < FOURIER_PTS; ++k) {
-                // T = T z_b + R
-                const double tr = fma(Tr[k], P[k].Eb.x, fma(-Ti[k], P[k].Eb.y, Rr[k]));
-                Ti[k] = fma(Tr[k], P[k].Eb.y, fma(Ti[k], P[k].Eb.x, Ri[k]));
-                Tr[k] = tr;
-            }
+            for (int k = 0; k < FOURIER_PTS; ++k) rotate_phase(cb[k], sb[k], P[k].Eb.x, -P[k].Eb.y);
+            if (fr[1] >= 0) fourier_row<MC, true>(fold + fr[0], fr[1], cc, sc, cb, sb, Tr, Ti);
         }
 #pragma unroll
         for (int k = 0; k < FOURIER_PTS; ++k) {
-            const double2 Q = cmul(Pa[k], Eb_neg[k]);
-            acc[k] += Q.x * Tr[k] - Q.y * Ti[k];
-            Pa[k] = cmul(Pa[k], P[k].Ea);
+            acc[k] += fma(ca[k], Tr[k], sa[k] * Ti[k]);  // Re(z_a^ma T)
+            rotate_phase(ca[k], sa[k], P[k].Ea.x, -P[k].Ea.y);
         }
     }
 #pragma unroll
@@ -1622,17 +1692,31 @@ __global__ __launch_bounds__(FOURIER_WG) void point_fourier_grad_kernel(GroupArg
             for (int k = 0; k < FOURIER_PTS; ++k) Q[k] = cmul(Pb[k], Z[k]);
             // entry (r, mc): 2 GT doubles from At + 2 GT ((r rowlen) + mc + Mc)
             const gconst_ptr<double> row = At + 2LL * GT * ((long long)r * rowlen + Mc);
-#pragma unroll 2
+            gconst_ptr<double> e = row + 2LL * GT * lo;
+            double w[2 * NT];
+#pragma unroll
+            for (int d = 0; d < 2 * NT; ++d) w[d] = e[d];
+#pragma unroll
+            for (int d = 0; d < 2 * NT; ++d) asm volatile("" ::"s"(w[d]));
             for (int mc = lo; mc <= hi; ++mc) {
-                const gconst_ptr<double> e = row + 2LL * GT * mc;
+                // the next entry is loaded before this one's FMAs (past the last: the
+                // padding); the empty statement keeps the load up here
+                double v[2 * NT];
+                e += 2 * GT;
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const double Ar = e[2 * t], Ai = e[2 * t + 1];
-#pragma unroll
-                    for (int k = 0; k < FOURIER_PTS; ++k) acc[k][t] = fma(Ar, Q[k].x, fma(-Ai, Q[k].y, acc[k][t]));
+                for (int d = 0; d < 2 * NT; ++d) {
+                    v[d] = w[d];
+                    w[d] = e[d];
                 }
 #pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int k = 0; k < FOURIER_PTS; ++k)
+                        acc[k][t] = fma(v[2 * t], Q[k].x, fma(-v[2 * t + 1], Q[k].y, acc[k][t]));
+#pragma unroll
                 for (int k = 0; k < FOURIER_PTS; ++k) Q[k] = cmul(Q[k], Zc[k]);
+#pragma unroll
+                for (int d = 0; d < 2 * NT; ++d) asm volatile("" ::"s"(w[d]));
             }
         }
 #pragma unroll

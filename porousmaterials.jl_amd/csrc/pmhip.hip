@@ -320,6 +320,8 @@ struct pm_ewald {
     int Ma = 0, Mb = 0, Mc = 0;
     double2* d_box = nullptr;
     int2* d_rows = nullptr;    // per (ma, mb) row of the box: kept mc range (lo > hi: empty)
+    int2* d_frows = nullptr;   // after d_rows: rows of the folded coefficients
+    double* d_fold = nullptr;  // after the box: the folded coefficients (fold_box_kernel)
     float4* d_erfc = nullptr;  // cubics of erfc(alpha r) on [0, sr_cutoff] (FP32)
     double2* d_erfc64 = nullptr;  // quintics of erfc(alpha r) about the multiples of sr_cutoff / ERFC64_SEG (FP64)
     double2* d_box_t = nullptr;  // per-type boxes (gradient runs), built on first use
@@ -760,6 +762,8 @@ void fill_run_pair(RunArgs& a, const pm_framework* fw, const pm_forcefield* ff, 
         a.Mc = ew->Mc;
         a.A = ew->d_box;
         a.krows = ew->d_rows;
+        a.frows = ew->d_frows;
+        a.fold = ew->d_fold;
     }
 }
 
@@ -992,6 +996,23 @@ void pair_launch_grad(const GroupArgs& g, int n_wg, size_t shm, int extra_off, i
         case 6: pair_launch_t<Real, 6>(g, n_wg, shm, extra_off); break;
         default: pair_launch_t<Real, GT>(g, n_wg, shm, extra_off); break;
     }
+}
+
+// The Fourier kernel by the group's largest third index: the smallest that holds
+// it, whose registers (66 + 8 per index) allow the most waves per SIMD; past 12
+// (3 waves) the one that steps the phases along each row.  Held and stepped: 3e6
+// points of index 5 206 and 292 us, 48 runs of index up to 10 297 and 316.
+template <int MC>
+void fourier_launch_t(const GroupArgs& g, unsigned n_wg) {
+    hipLaunchKernelGGL(point_fourier_kernel<MC>, dim3(n_wg), dim3(FOURIER_WG), 0, g_ctx.stream, g);
+}
+void fourier_launch(const GroupArgs& g, unsigned n_wg, int mc_max) {
+    if (mc_max <= 4) fourier_launch_t<4>(g, n_wg);
+    else if (mc_max <= 6) fourier_launch_t<6>(g, n_wg);
+    else if (mc_max <= 8) fourier_launch_t<8>(g, n_wg);
+    else if (mc_max <= 10) fourier_launch_t<10>(g, n_wg);
+    else if (mc_max <= 12) fourier_launch_t<12>(g, n_wg);
+    else fourier_launch_t<0>(g, n_wg);
 }
 
 template <int NT>
@@ -1404,7 +1425,10 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
         PM_HIP(hipEventRecord(g_ctx.evp1, g_ctx.stream));
         const long long slot_wg = (gr.n_slots + WG - 1) / WG;
         if (gr.es && widom) {
-            hipLaunchKernelGGL(point_fourier_kernel, dim3((unsigned)slot_wg), dim3(FOURIER_WG), 0, g_ctx.stream, g);
+            int mc_max = 0;
+            for (int si = 0; si < gr.n_seg; ++si)
+                if (const PointRun& r = runs[segs[gr.seg0 + si].run]; r.es) mc_max = std::max(mc_max, r.ra.Mc);
+            fourier_launch(g, (unsigned)slot_wg, mc_max);
         } else if (gr.es) {
             // grids: the separable form, run by run
             for (int si = 0; si < gr.n_seg; ++si) {
@@ -1592,9 +1616,10 @@ int ensure_type_boxes(pm_ewald* ew, const pm_framework* fw) {
     double4* d_ua = nullptr;
     double2* d_bt = nullptr;
     PM_HIP(hipStreamSynchronize(g_ctx.stream));
-    hipError_t e = hipMalloc(&d_bt, box_n * GT * sizeof(double2));
+    // (one entry more: the gradient kernel loads an entry ahead)
+    hipError_t e = hipMalloc(&d_bt, (box_n + 1) * GT * sizeof(double2));
     if (e == hipSuccess) e = hipMalloc(&d_ua, ua.size() * sizeof(double4));
-    if (e == hipSuccess) e = hipMemsetAsync(d_bt, 0, box_n * GT * sizeof(double2), g_ctx.stream);
+    if (e == hipSuccess) e = hipMemsetAsync(d_bt, 0, (box_n + 1) * GT * sizeof(double2), g_ctx.stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(d_ua, ua.data(), ua.size() * sizeof(double4), hipMemcpyHostToDevice, g_ctx.stream);
     if (e == hipSuccess && ew->nk > 0 && fw->n_unit > 0) {
@@ -1886,17 +1911,31 @@ int pm_ewald_create(const pm_framework* fw, double alpha, double sr_cutoff, int6
         if (r.x > r.y) r = make_int2(mc, mc);
         else r = make_int2(std::min(r.x, mc), std::max(r.y, mc));
     }
-    if (hipMalloc(&ew->d_rows, n_rows * sizeof(int2)) != hipSuccess ||
+    // rows of the folded coefficients, after them
+    size_t n_fold = 0;
+    for (int ma = 0; ma <= Ma; ++ma)
+        for (int mb = 0; mb <= Mb; ++mb) {
+            const int2 rp = rows[(size_t)ma * (2 * Mb + 1) + Mb + mb], rm = rows[(size_t)ma * (2 * Mb + 1) + Mb - mb];
+            int hi = -1;
+            if (rp.x <= rp.y) hi = std::max(std::abs(rp.x), std::abs(rp.y));
+            if (rm.x <= rm.y) hi = std::max(hi, std::max(std::abs(rm.x), std::abs(rm.y)));
+            rows.push_back(make_int2((int)n_fold, hi));
+            if (hi >= 0) n_fold += FOLD_HEAD + (size_t)hi * FOLD_CELL;
+        }
+    n_fold += FOLD_PAD;  // the loads run a cell ahead
+    if (hipMalloc(&ew->d_rows, rows.size() * sizeof(int2)) != hipSuccess ||
         hipMalloc(&ew->d_erfc, ERFC_TAB * sizeof(float4)) != hipSuccess ||
         hipMalloc(&ew->d_erfc64, ERFC64_TAB * sizeof(double2)) != hipSuccess ||
-        hipMalloc(&ew->d_box, box_n * sizeof(double2)) != hipSuccess ||
+        hipMalloc(&ew->d_box, box_n * sizeof(double2) + n_fold * sizeof(double)) != hipSuccess ||
         hipMalloc(&ew->d_k, std::max<size_t>(ew->nk, 1) * sizeof(KVec)) != hipSuccess ||
         hipMalloc(&d_m, std::max<size_t>(m.size(), 1) * sizeof(int)) != hipSuccess ||
         hipMalloc(&d_w, std::max<size_t>(w.size(), 1) * sizeof(double)) != hipSuccess) {
         cleanup();
         return fail(PM_ERR_OOM, "pm_ewald_create: device allocation failed");
     }
-    hipError_t e = hipMemsetAsync(ew->d_box, 0, box_n * sizeof(double2), g_ctx.stream);
+    ew->d_frows = ew->d_rows + n_rows;
+    ew->d_fold = reinterpret_cast<double*>(ew->d_box + box_n);
+    hipError_t e = hipMemsetAsync(ew->d_box, 0, box_n * sizeof(double2) + n_fold * sizeof(double), g_ctx.stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(ew->d_erfc, etab.data(), ERFC_TAB * sizeof(float4), hipMemcpyHostToDevice,
                            g_ctx.stream);
@@ -1904,7 +1943,7 @@ int pm_ewald_create(const pm_framework* fw, double alpha, double sr_cutoff, int6
         e = hipMemcpyAsync(ew->d_erfc64, etab64.data(), ERFC64_TAB * sizeof(double2), hipMemcpyHostToDevice,
                            g_ctx.stream);
     if (e == hipSuccess)
-        e = hipMemcpyAsync(ew->d_rows, rows.data(), n_rows * sizeof(int2), hipMemcpyHostToDevice, g_ctx.stream);
+        e = hipMemcpyAsync(ew->d_rows, rows.data(), rows.size() * sizeof(int2), hipMemcpyHostToDevice, g_ctx.stream);
     if (e == hipSuccess && ew->nk > 0) {
         e = hipMemcpyAsync(d_m, m.data(), m.size() * sizeof(int), hipMemcpyHostToDevice, g_ctx.stream);
         if (e == hipSuccess)
@@ -1918,6 +1957,9 @@ int pm_ewald_create(const pm_framework* fw, double alpha, double sr_cutoff, int6
         if (e == hipSuccess) {
             hipLaunchKernelGGL(fourier_box_kernel, dim3((unsigned)((ew->nk + 255) / 256)), dim3(256), 0,
                                g_ctx.stream, ew->d_k, (int)ew->nk, Mb, Mc, ew->d_box);
+            const long long n_cells = (long long)(Ma + 1) * (Mb + 1) * (Mc + 1);
+            hipLaunchKernelGGL(fold_box_kernel, dim3((unsigned)((n_cells + 255) / 256)), dim3(256), 0, g_ctx.stream,
+                               ew->d_box, Ma, Mb, Mc, ew->d_frows, ew->d_fold);
             e = hipGetLastError();
         }
     }
