@@ -771,6 +771,16 @@ __device__ inline int tile_part(int t, int n_tiles) {
     return (int)((double)LIST_PARTS * t / n_tiles);  // exact: quotients are whole or at least 1/n_tiles from it
 }
 
+// The records of the mixed runs' image list: (type, FP32 charge) in the charge's
+// place.
+__global__ void mixed_images_kernel(const double4* img, const int* type, long long n, double4* out) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double4 v = img[i];
+    v.w = __hiloint2double(type[i], __float_as_int((float)v.w));
+    out[i] = v;
+}
+
 // LDS of the pair kernels.
 struct PairLds {
     double* part;           // SPLIT kernels: the parts' sums

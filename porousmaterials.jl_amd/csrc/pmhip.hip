@@ -288,8 +288,8 @@ struct pm_framework {
     std::vector<int32_t> unit_type;
     double net_charge = 0.0;
     bool charged = false;
-    double4* d_atoms = nullptr;
-    float4* d_atoms_f = nullptr;  // FP32 positions in [0, 1), in d_atoms' allocation
+    double4* d_atoms = nullptr;   // first of the framework's one allocation
+    float4* d_atoms_f = nullptr;  // FP32 positions in [0, 1)
     int32_t* d_species = nullptr;
     double4* d_unit_q = nullptr;
     // Image lists, one per cutoff radius r: every periodic image within r of
@@ -298,13 +298,36 @@ struct pm_framework {
         double r = 0.0;
         int64_t n = 0;
         int64_t n_tiles = 0;
-        double4* d_img = nullptr;
+        double4* d_img = nullptr;       // first of the list's one allocation
         double4* d_img_m = nullptr;     // the same with (type, FP32 charge) in the charge's place (mixed runs)
         int32_t* d_type = nullptr;
         double4* d_tile_sph = nullptr;  // tile bounding spheres
         int2* d_tile_rng = nullptr;     // tile (first image, count)
     };
     std::vector<Images> images;
+};
+
+// Host arrays laid out one after the other, 256-byte aligned, to be uploaded into
+// one device allocation by one copy (an allocation or a copy of its own costs each
+// array some 10 us, whatever its size).
+struct Upload {
+    std::vector<unsigned char> host;
+    size_t add(const void* src, size_t bytes) {
+        const size_t off = (host.size() + 255) / 256 * 256;
+        host.resize(off + bytes);
+        if (src && bytes) std::memcpy(host.data() + off, src, bytes);
+        return off;
+    }
+    // device memory of max(extra_end, the arrays' size) bytes, the arrays copied
+    hipError_t send(unsigned char** d, size_t total = 0) const {
+        hipError_t e = hipMalloc(d, std::max<size_t>(std::max(total, host.size()), 1));
+        if (e == hipSuccess && !host.empty()) e = hipMemcpy(*d, host.data(), host.size(), hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            (void)hipFree(*d);
+            *d = nullptr;
+        }
+        return e;
+    }
 };
 
 struct pm_forcefield {
@@ -316,6 +339,7 @@ struct pm_forcefield {
 struct pm_ewald {
     double alpha = 0.0, sr_cutoff = 0.0;
     int64_t nk = 0;
+    unsigned char* d_mem = nullptr;  // the one allocation of all but d_box_t
     KVec* d_k = nullptr;
     int Ma = 0, Mb = 0, Mc = 0;
     double2* d_box = nullptr;
@@ -552,6 +576,8 @@ int run_poses(const pm_framework* fw, const pm_forcefield* ff, const pm_ewald* e
     return finish_timing((double)n * a.ns * fw->n_rep);
 }
 
+unsigned grid1d(long long n, int block) { return (unsigned)((n + block - 1) / block); }
+
 // ---------------------------------------------------- point engine ----
 // Image list for radius r: every periodic image (x_unit + t) / rep whose
 // replicated-box fractional coordinates lie within [-m_a, 1 / rep_a + m_a] on
@@ -563,10 +589,6 @@ int run_poses(const pm_framework* fw, const pm_forcefield* ff, const pm_ewald* e
 // FP32 partial sums -- depends on the framework and the radius alone.
 void free_images(pm_framework::Images& im) {
     (void)hipFree(im.d_img);
-    (void)hipFree(im.d_img_m);
-    (void)hipFree(im.d_type);
-    (void)hipFree(im.d_tile_sph);
-    (void)hipFree(im.d_tile_rng);
 }
 
 const pm_framework::Images* find_images(const pm_framework* fw, double r) {
@@ -621,9 +643,18 @@ int get_images(pm_framework* fw, double r, const pm_framework::Images** out) {
     // sphere.  A chunk visits only the tiles whose sphere meets its own; the
     // FP32 partial sums of a point run per tile, so they depend on this list
     // alone.
+    const size_t n_img = img.size();
+    // unused records after the last image, which Candidates::fetch may read
+    const size_t n = n_img + TILE_IMAGES;
+    Upload up;
+    up.host.reserve(n * (sizeof(double4) + sizeof(int32_t)) + (n_img / 8 + 64) * (sizeof(double4) + sizeof(int2)));
+    const size_t o_img = up.add(nullptr, n * sizeof(double4));
+    const size_t o_type = up.add(nullptr, n * sizeof(int32_t));
     std::vector<double4> sph;
     std::vector<int2> rng;
-    if (!img.empty()) {
+    if (n_img > 0) {
+        double4* const rec = reinterpret_cast<double4*>(up.host.data() + o_img);
+        int32_t* const types = reinterpret_cast<int32_t*>(up.host.data() + o_type);
         double lo[3] = {img[0].x, img[0].y, img[0].z}, hi[3] = {lo[0], lo[1], lo[2]};
         for (const auto& v : img) {
             const double c[3] = {v.x, v.y, v.z};
@@ -637,39 +668,43 @@ int get_images(pm_framework* fw, double r, const pm_framework::Images** out) {
             ext[d] = std::max(hi[d] - lo[d], 1e-6);
             bvol *= ext[d];
         }
-        const double b = std::cbrt(bvol * TILE_IMAGES / (double)img.size());
+        const double b = std::cbrt(bvol * TILE_IMAGES / (double)n_img);
         int nb[3];
         for (int d = 0; d < 3; ++d) nb[d] = (int)std::max(1.0, std::min(4096.0, std::ceil(ext[d] / b)));
-        std::vector<int64_t> key(img.size());
-        for (size_t i = 0; i < img.size(); ++i) {
+        std::vector<uint64_t> key(n_img);
+        for (size_t i = 0; i < n_img; ++i) {
             const double c[3] = {img[i].x, img[i].y, img[i].z};
-            int64_t k = 0;
+            uint64_t k = 0;
             for (int d = 0; d < 3; ++d) {
                 const int q = std::min(nb[d] - 1, std::max(0, (int)((c[d] - lo[d]) / ext[d] * nb[d])));
                 k = k * nb[d] + q;
             }
             key[i] = k;
         }
-        std::vector<size_t> perm(img.size());
-        for (size_t i = 0; i < perm.size(); ++i) perm[i] = i;
-        std::stable_sort(perm.begin(), perm.end(), [&](size_t x, size_t y) {
-            return key[x] != key[y] ? key[x] < key[y] : ty[x] < ty[y];
-        });
-        std::vector<double4> img2(img.size());
-        std::vector<int32_t> ty2(ty.size());
-        for (size_t i = 0; i < perm.size(); ++i) {
-            img2[i] = img[perm[i]];
-            ty2[i] = ty[perm[i]];
+        // by bin, stably (the images come by species): a counting sort, unless a
+        // flat list's bins outnumber its images
+        std::vector<uint32_t> perm(n_img);
+        const uint64_t n_bins = (uint64_t)nb[0] * nb[1] * nb[2];
+        if (n_bins <= 4 * n_img + 1024) {
+            std::vector<uint32_t> at((size_t)n_bins + 1, 0);
+            for (uint64_t k : key) ++at[k + 1];
+            for (size_t k = 1; k <= n_bins; ++k) at[k] += at[k - 1];
+            for (size_t i = 0; i < n_img; ++i) perm[at[key[i]]++] = (uint32_t)i;
+        } else {
+            for (size_t i = 0; i < n_img; ++i) perm[i] = (uint32_t)i;
+            std::stable_sort(perm.begin(), perm.end(), [&](uint32_t x, uint32_t y) { return key[x] < key[y]; });
         }
-        img.swap(img2);
-        ty.swap(ty2);
+        for (size_t i = 0; i < n_img; ++i) {
+            rec[i] = img[perm[i]];
+            types[i] = ty[perm[i]];
+        }
         size_t i0 = 0;
-        while (i0 < img.size()) {
+        while (i0 < n_img) {
             size_t i1 = i0 + 1;
-            while (i1 < img.size() && i1 - i0 < (size_t)TILE_IMAGES && key[perm[i1]] == key[perm[i0]]) ++i1;
-            double bl[3] = {img[i0].x, img[i0].y, img[i0].z}, bh[3] = {bl[0], bl[1], bl[2]};
+            while (i1 < n_img && i1 - i0 < (size_t)TILE_IMAGES && key[perm[i1]] == key[perm[i0]]) ++i1;
+            double bl[3] = {rec[i0].x, rec[i0].y, rec[i0].z}, bh[3] = {bl[0], bl[1], bl[2]};
             for (size_t i = i0; i < i1; ++i) {
-                const double c[3] = {img[i].x, img[i].y, img[i].z};
+                const double c[3] = {rec[i].x, rec[i].y, rec[i].z};
                 for (int d = 0; d < 3; ++d) {
                     bl[d] = std::min(bl[d], c[d]);
                     bh[d] = std::max(bh[d], c[d]);
@@ -678,7 +713,7 @@ int get_images(pm_framework* fw, double r, const pm_framework::Images** out) {
             const double cx = 0.5 * (bl[0] + bh[0]), cy = 0.5 * (bl[1] + bh[1]), cz = 0.5 * (bl[2] + bh[2]);
             double r2 = 0.0;
             for (size_t i = i0; i < i1; ++i) {
-                const double dx = img[i].x - cx, dy = img[i].y - cy, dz = img[i].z - cz;
+                const double dx = rec[i].x - cx, dy = rec[i].y - cy, dz = rec[i].z - cz;
                 r2 = std::max(r2, dx * dx + dy * dy + dz * dz);
             }
             // slack for the kernel's rounding of the sphere test
@@ -689,40 +724,28 @@ int get_images(pm_framework* fw, double r, const pm_framework::Images** out) {
     }
     pm_framework::Images im;
     im.r = r;
-    im.n = (int64_t)img.size();
+    im.n = (int64_t)n_img;
     im.n_tiles = (int64_t)sph.size();
     if (im.n > (int64_t)INT32_MAX) return fail(PM_ERR_ARG, "image list too large");
-    // unused records after the last image, which Candidates::fetch may read
-    const size_t n = img.size() + TILE_IMAGES;
-    std::vector<double4> rec(n, make_double4(0.0, 0.0, 0.0, 0.0)), rec_m(rec);
-    std::vector<int32_t> types(n, 0);
-    for (size_t i = 0; i < img.size(); ++i) {
-        rec[i] = rec_m[i] = img[i];
-        types[i] = ty[i];
-        const float qf = (float)img[i].w;
-        uint32_t bits;
-        std::memcpy(&bits, &qf, sizeof(bits));
-        const uint64_t w = ((uint64_t)(uint32_t)ty[i] << 32) | bits;
-        std::memcpy(&rec_m[i].w, &w, sizeof(w));
+    const size_t o_sph = up.add(sph.data(), sph.size() * sizeof(double4));
+    const size_t o_rng = up.add(rng.data(), rng.size() * sizeof(int2));
+    const size_t o_m = (up.host.size() + 255) / 256 * 256;
+    unsigned char* d = nullptr;
+    hipError_t e = up.send(&d, o_m + n * sizeof(double4));
+    if (e == hipSuccess) {
+        im.d_img = reinterpret_cast<double4*>(d + o_img);
+        im.d_type = reinterpret_cast<int32_t*>(d + o_type);
+        im.d_tile_sph = reinterpret_cast<double4*>(d + o_sph);
+        im.d_tile_rng = reinterpret_cast<int2*>(d + o_rng);
+        im.d_img_m = reinterpret_cast<double4*>(d + o_m);
+        hipLaunchKernelGGL(mixed_images_kernel, dim3(grid1d((long long)n, 256)), dim3(256), 0, g_ctx.stream, im.d_img,
+                           im.d_type, (long long)n, im.d_img_m);
+        e = hipGetLastError();
+        if (e != hipSuccess) free_images(im);
     }
-    const size_t nt = std::max<size_t>(sph.size(), 1);
-    hipError_t e = hipMalloc(&im.d_img, n * sizeof(double4));
-    if (e == hipSuccess) e = hipMalloc(&im.d_img_m, n * sizeof(double4));
-    if (e == hipSuccess) e = hipMalloc(&im.d_type, n * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(&im.d_tile_sph, nt * sizeof(double4));
-    if (e == hipSuccess) e = hipMalloc(&im.d_tile_rng, nt * sizeof(int2));
-    if (e == hipSuccess) e = hipMemcpy(im.d_img, rec.data(), n * sizeof(double4), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(im.d_img_m, rec_m.data(), n * sizeof(double4), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(im.d_type, types.data(), n * sizeof(int32_t), hipMemcpyHostToDevice);
-    if (e == hipSuccess && !sph.empty())
-        e = hipMemcpy(im.d_tile_sph, sph.data(), sph.size() * sizeof(double4), hipMemcpyHostToDevice);
-    if (e == hipSuccess && !rng.empty())
-        e = hipMemcpy(im.d_tile_rng, rng.data(), rng.size() * sizeof(int2), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        free_images(im);
+    if (e != hipSuccess)
         return fail(e == hipErrorOutOfMemory ? PM_ERR_OOM : PM_ERR_DEVICE,
                     std::string("image list upload: ") + hipGetErrorString(e));
-    }
     fw->images.push_back(im);
     *out = &fw->images.back();
     return PM_OK;
@@ -1053,7 +1076,6 @@ void fourier_grad_launch(const GroupArgs& g, unsigned n_wg, int n_gt) {
     }
 }
 
-unsigned grid1d(long long n, int block) { return (unsigned)((n + block - 1) / block); }
 
 // Device memory a call must use instead of the library's growable scratch
 // (pm_widom_noalloc): the call then allocates nothing, and fails before any
@@ -1755,12 +1777,15 @@ int pm_framework_create(const double f_to_c[9], const int32_t rep[3], int64_t n_
             fw->unit_q[i] = charge[i];
         }
     }
-    // replicated atoms, then their FP32 positions
-    size_t na = (size_t)(fw->n_rep > 0 ? fw->n_rep : 1);
-    const size_t atoms_bytes = na * (sizeof(double4) + sizeof(float4));
-    std::vector<double4> atoms(na + (na + 1) / 2);
-    float4* const atoms_f = reinterpret_cast<float4*>(atoms.data() + na);
-    std::vector<int32_t> sp((size_t)fw->n_rep);
+    const size_t na = (size_t)(fw->n_rep > 0 ? fw->n_rep : 1);
+    Upload up;
+    up.host.reserve(na * (sizeof(double4) + sizeof(float4) + sizeof(int32_t)) + (size_t)n_atoms * sizeof(double4) + 1024);
+    const size_t o_atoms = up.add(nullptr, na * sizeof(double4));
+    const size_t o_atoms_f = up.add(nullptr, na * sizeof(float4));
+    const size_t o_species = up.add(nullptr, na * sizeof(int32_t));
+    double4* const atoms = reinterpret_cast<double4*>(up.host.data() + o_atoms);
+    float4* const atoms_f = reinterpret_cast<float4*>(up.host.data() + o_atoms_f);
+    int32_t* const sp = reinterpret_cast<int32_t*>(up.host.data() + o_species);
     std::vector<double4> uq;
     int64_t k = 0;
     for (int ra = 0; ra < rep[0]; ++ra)
@@ -1782,29 +1807,18 @@ int pm_framework_create(const double f_to_c[9], const int32_t rep[3], int64_t n_
     }
     fw->n_unit_q = (int64_t)uq.size();
     fw->charged = fw->n_unit_q > 0;
-    auto cleanup = [&]() {
-        (void)hipFree(fw->d_atoms); (void)hipFree(fw->d_species); (void)hipFree(fw->d_unit_q);
+    const size_t o_uq = up.add(uq.data(), uq.size() * sizeof(double4));
+    unsigned char* d = nullptr;
+    const hipError_t e = up.send(&d);
+    if (e != hipSuccess) {
         delete fw;
-    };
-    if (hipMalloc(&fw->d_atoms, atoms_bytes) != hipSuccess ||
-        hipMalloc(&fw->d_species, na * sizeof(int32_t)) != hipSuccess ||
-        hipMalloc(&fw->d_unit_q, (uq.empty() ? 1 : uq.size()) * sizeof(double4)) != hipSuccess) {
-        cleanup();
-        return fail(PM_ERR_OOM, "pm_framework_create: device allocation failed");
+        return e == hipErrorOutOfMemory ? fail(PM_ERR_OOM, "pm_framework_create: device allocation failed")
+                                        : fail(PM_ERR_DEVICE, "pm_framework_create: host-to-device copy failed");
     }
-    if (fw->n_rep > 0) {
-        if (hipMemcpy(fw->d_atoms, atoms.data(), atoms_bytes, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(fw->d_species, sp.data(), fw->n_rep * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess) {
-            cleanup();
-            return fail(PM_ERR_DEVICE, "pm_framework_create: host-to-device copy failed");
-        }
-    }
-    if (!uq.empty() &&
-        hipMemcpy(fw->d_unit_q, uq.data(), uq.size() * sizeof(double4), hipMemcpyHostToDevice) != hipSuccess) {
-        cleanup();
-        return fail(PM_ERR_DEVICE, "pm_framework_create: host-to-device copy failed");
-    }
-    fw->d_atoms_f = reinterpret_cast<float4*>(fw->d_atoms + na);
+    fw->d_atoms = reinterpret_cast<double4*>(d + o_atoms);
+    fw->d_atoms_f = reinterpret_cast<float4*>(d + o_atoms_f);
+    fw->d_species = reinterpret_cast<int32_t*>(d + o_species);
+    fw->d_unit_q = reinterpret_cast<double4*>(d + o_uq);
     *out = fw;
     return PM_OK;
 }
@@ -1813,8 +1827,6 @@ int pm_framework_destroy(pm_framework* fw) {
     std::lock_guard<std::mutex> lk(g_mu);
     if (!fw) return PM_OK;
     (void)hipFree(fw->d_atoms);
-    (void)hipFree(fw->d_species);
-    (void)hipFree(fw->d_unit_q);
     for (auto& im : fw->images) free_images(im);
     delete fw;
     return PM_OK;
@@ -1890,14 +1902,6 @@ int pm_ewald_create(const pm_framework* fw, double alpha, double sr_cutoff, int6
     ew->nk = (int64_t)w.size();
     ew->Ma = Ma; ew->Mb = Mb; ew->Mc = Mc;
     size_t box_n = (size_t)(Ma + 1) * (2 * Mb + 1) * (2 * Mc + 1);
-    int* d_m = nullptr;
-    double* d_w = nullptr;
-    auto cleanup = [&]() {
-        (void)hipFree(ew->d_k); (void)hipFree(ew->d_box); (void)hipFree(ew->d_erfc); (void)hipFree(ew->d_rows);
-        (void)hipFree(ew->d_erfc64);
-        (void)hipFree(d_m); (void)hipFree(d_w);
-        delete ew;
-    };
     std::vector<float4> etab(ERFC_TAB);
     build_erfc_table(alpha, sr_cutoff, etab.data());
     std::vector<double2> etab64(ERFC64_TAB);
@@ -1923,54 +1927,50 @@ int pm_ewald_create(const pm_framework* fw, double alpha, double sr_cutoff, int6
             if (hi >= 0) n_fold += FOLD_HEAD + (size_t)hi * FOLD_CELL;
         }
     n_fold += FOLD_PAD;  // the loads run a cell ahead
-    if (hipMalloc(&ew->d_rows, rows.size() * sizeof(int2)) != hipSuccess ||
-        hipMalloc(&ew->d_erfc, ERFC_TAB * sizeof(float4)) != hipSuccess ||
-        hipMalloc(&ew->d_erfc64, ERFC64_TAB * sizeof(double2)) != hipSuccess ||
-        hipMalloc(&ew->d_box, box_n * sizeof(double2) + n_fold * sizeof(double)) != hipSuccess ||
-        hipMalloc(&ew->d_k, std::max<size_t>(ew->nk, 1) * sizeof(KVec)) != hipSuccess ||
-        hipMalloc(&d_m, std::max<size_t>(m.size(), 1) * sizeof(int)) != hipSuccess ||
-        hipMalloc(&d_w, std::max<size_t>(w.size(), 1) * sizeof(double)) != hipSuccess) {
-        cleanup();
-        return fail(PM_ERR_OOM, "pm_ewald_create: device allocation failed");
+    // one allocation: what is uploaded (the set-up's k-vectors with it), then what
+    // the set-up kernels fill, the box and the folded coefficients cleared first
+    Upload up;
+    const size_t o_rows = up.add(rows.data(), rows.size() * sizeof(int2));
+    const size_t o_erfc = up.add(etab.data(), ERFC_TAB * sizeof(float4));
+    const size_t o_erfc64 = up.add(etab64.data(), ERFC64_TAB * sizeof(double2));
+    const size_t o_m = up.add(m.data(), m.size() * sizeof(int32_t));
+    const size_t o_w = up.add(w.data(), w.size() * sizeof(double));
+    Arena ar;
+    (void)ar.take(up.host.size());
+    const size_t clear_bytes = box_n * sizeof(double2) + n_fold * sizeof(double);
+    const size_t o_box = ar.take(clear_bytes);
+    const size_t o_k = ar.take(std::max<size_t>((size_t)ew->nk, 1) * sizeof(KVec));
+    hipError_t e = up.send(&ew->d_mem, ar.used);
+    if (e != hipSuccess) {
+        delete ew;
+        return e == hipErrorOutOfMemory ? fail(PM_ERR_OOM, "pm_ewald_create: device allocation failed")
+                                        : fail(PM_ERR_DEVICE, std::string("pm_ewald_create: ") + hipGetErrorString(e));
     }
+    ew->d_rows = reinterpret_cast<int2*>(ew->d_mem + o_rows);
     ew->d_frows = ew->d_rows + n_rows;
+    ew->d_erfc = reinterpret_cast<float4*>(ew->d_mem + o_erfc);
+    ew->d_erfc64 = reinterpret_cast<double2*>(ew->d_mem + o_erfc64);
+    ew->d_box = reinterpret_cast<double2*>(ew->d_mem + o_box);
     ew->d_fold = reinterpret_cast<double*>(ew->d_box + box_n);
-    hipError_t e = hipMemsetAsync(ew->d_box, 0, box_n * sizeof(double2) + n_fold * sizeof(double), g_ctx.stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(ew->d_erfc, etab.data(), ERFC_TAB * sizeof(float4), hipMemcpyHostToDevice,
-                           g_ctx.stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(ew->d_erfc64, etab64.data(), ERFC64_TAB * sizeof(double2), hipMemcpyHostToDevice,
-                           g_ctx.stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(ew->d_rows, rows.data(), rows.size() * sizeof(int2), hipMemcpyHostToDevice, g_ctx.stream);
+    ew->d_k = reinterpret_cast<KVec*>(ew->d_mem + o_k);
+    e = hipMemsetAsync(ew->d_box, 0, clear_bytes, g_ctx.stream);
     if (e == hipSuccess && ew->nk > 0) {
-        e = hipMemcpyAsync(d_m, m.data(), m.size() * sizeof(int), hipMemcpyHostToDevice, g_ctx.stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(d_w, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice, g_ctx.stream);
-        double nr = (double)fw->rep[0] * fw->rep[1] * fw->rep[2];
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(structure_factor_kernel, dim3((unsigned)ew->nk), dim3(64), 0, g_ctx.stream,
-                               fw->d_unit_q, (long long)fw->n_unit_q, d_m, d_w, nr, ew->d_k);
-            e = hipGetLastError();
-        }
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(fourier_box_kernel, dim3((unsigned)((ew->nk + 255) / 256)), dim3(256), 0,
-                               g_ctx.stream, ew->d_k, (int)ew->nk, Mb, Mc, ew->d_box);
-            const long long n_cells = (long long)(Ma + 1) * (Mb + 1) * (Mc + 1);
-            hipLaunchKernelGGL(fold_box_kernel, dim3((unsigned)((n_cells + 255) / 256)), dim3(256), 0, g_ctx.stream,
-                               ew->d_box, Ma, Mb, Mc, ew->d_frows, ew->d_fold);
-            e = hipGetLastError();
-        }
+        const double nr = (double)fw->rep[0] * fw->rep[1] * fw->rep[2];
+        hipLaunchKernelGGL(structure_factor_kernel, dim3((unsigned)ew->nk), dim3(64), 0, g_ctx.stream, fw->d_unit_q,
+                           (long long)fw->n_unit_q, reinterpret_cast<const int*>(ew->d_mem + o_m),
+                           reinterpret_cast<const double*>(ew->d_mem + o_w), nr, ew->d_k);
+        hipLaunchKernelGGL(fourier_box_kernel, dim3((unsigned)((ew->nk + 255) / 256)), dim3(256), 0, g_ctx.stream,
+                           ew->d_k, (int)ew->nk, Mb, Mc, ew->d_box);
+        const long long n_cells = (long long)(Ma + 1) * (Mb + 1) * (Mc + 1);
+        hipLaunchKernelGGL(fold_box_kernel, dim3((unsigned)((n_cells + 255) / 256)), dim3(256), 0, g_ctx.stream,
+                           ew->d_box, Ma, Mb, Mc, ew->d_frows, ew->d_fold);
+        e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(g_ctx.stream);
-    (void)hipFree(d_m);
-    (void)hipFree(d_w);
-    d_m = nullptr;
-    d_w = nullptr;
     if (e != hipSuccess) {
         std::string msg = std::string("pm_ewald_create: ") + hipGetErrorString(e);
-        cleanup();
+        (void)hipFree(ew->d_mem);
+        delete ew;
         return fail(PM_ERR_DEVICE, msg);
     }
     *out = ew;
@@ -1980,12 +1980,8 @@ int pm_ewald_create(const pm_framework* fw, double alpha, double sr_cutoff, int6
 int pm_ewald_destroy(pm_ewald* ew) {
     std::lock_guard<std::mutex> lk(g_mu);
     if (!ew) return PM_OK;
-    (void)hipFree(ew->d_k);
-    (void)hipFree(ew->d_box);
-    (void)hipFree(ew->d_erfc);
-    (void)hipFree(ew->d_erfc64);
+    (void)hipFree(ew->d_mem);
     (void)hipFree(ew->d_box_t);
-    (void)hipFree(ew->d_rows);
     delete ew;
     return PM_OK;
 }
