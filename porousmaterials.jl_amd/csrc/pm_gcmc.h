@@ -79,6 +79,15 @@ struct GcmcChain {
     long long outer_target;  // outer cycle the current pm_gcmc_run call ends at
 };
 
+// A value that the compiler holds in a vector register instead of loading it again.
+template <typename T>
+__device__ inline T gc_keep(T v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+__device__ inline int gc_keep_s(int v) { return __builtin_amdgcn_readfirstlane(gc_keep(v)); }
+
 // Where a chain's molecules live during a launch.  GcMolsMem: device memory
 // in the handle's layout ([species][capacity][PM_MAX_SITES] sites,
 // [species][capacity] centres).  GcMolsLds: LDS, compact per species
@@ -100,11 +109,14 @@ struct GcMolsMem {
 struct GcMolsLds {
     double4* base;
     int cap;
-    __device__ double4* site_base(const GcmcParams& p, int s) const { return base + p.site_prefix[s] * cap; }
-    __device__ int stride(const GcmcParams& p, int s) const { return p.n_sites[s]; }
-    __device__ double4* com_base(const GcmcParams& p, int s) const { return base + (p.total_sites + s) * cap; }
+    int n_sites0, total_sites;  // of the parameters (species 0 needs no load)
+    __device__ double4* site_base(const GcmcParams& p, int s) const {
+        return s == 0 ? base : base + p.site_prefix[s] * cap;
+    }
+    __device__ int stride(const GcmcParams& p, int s) const { return s == 0 ? n_sites0 : p.n_sites[s]; }
+    __device__ double4* com_base(const GcmcParams& p, int s) const { return base + (total_sites + s) * cap; }
     __device__ double4& site(const GcmcParams& p, int s, int m, int k) const {
-        return site_base(p, s)[m * p.n_sites[s] + k];
+        return site_base(p, s)[m * stride(p, s) + k];
     }
     __device__ double4& com(const GcmcParams& p, int s, int m) const { return com_base(p, s)[m]; }
 };
@@ -123,214 +135,365 @@ __device__ inline void gc_mols_copy(const GcmcParams& p, const From& from, const
 }
 
 // The 10 uniforms of move t of a chain: species, move, molecule, position or
-// step (3), rotation (3), acceptance.
-__device__ inline void gcmc_uniforms(unsigned long long seed, unsigned chain, unsigned long long t, double u[10]) {
-#pragma unroll
-    for (uint32_t w = 0; w < 5; ++w) {
-        uint32_t c[4] = {(uint32_t)t, (uint32_t)(t >> 32), chain, 0x47434D00u | w};
-        philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
-        u[2 * w] = u53(c[0], c[1]);
-        u[2 * w + 1] = u53(c[2], c[3]);
-    }
-}
-
-// The same uniforms for GC_BATCH consecutive moves at once: lane l < 60 of
-// every wave holds the Philox block (t0 + l / 5, word l % 5), so one pass of
-// integer work serves 12 moves; a move reads its five blocks with readlane.
+// step (3), rotation (3), acceptance; two from each of five Philox blocks.  Lane
+// l < 60 of every wave holds those of move t0 + l / 5, block l % 5, so one pass
+// serves GC_BATCH moves; a move reads the ones it needs with readlane.
 constexpr int GC_BATCH = 12;
 struct GcRng {
     unsigned long long t0;
-    uint32_t c[4];
+    double v[2];
+    // uniform k of move t
+    __device__ __attribute__((always_inline)) double get(unsigned long long t, int k) const {
+        const int l = 5 * (int)(t - t0) + (k >> 1);
+        return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v[k & 1]), l),
+                                __builtin_amdgcn_readlane(__double2loint(v[k & 1]), l));
+    }
 };
 
 __device__ inline void gc_rng_fill(GcRng& r, unsigned long long seed, unsigned chain, unsigned long long t0) {
     const uint32_t l = (uint32_t)min((int)(threadIdx.x & 63), 5 * GC_BATCH - 1);
     const unsigned long long t = t0 + l / 5;
-    r.c[0] = (uint32_t)t;
-    r.c[1] = (uint32_t)(t >> 32);
-    r.c[2] = chain;
-    r.c[3] = 0x47434D00u | (l % 5);
-    philox4x32_10(r.c, (uint32_t)seed, (uint32_t)(seed >> 32));
+    uint32_t c[4] = {(uint32_t)t, (uint32_t)(t >> 32), chain, 0x47434D00u | (l % 5)};
+    philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+    r.v[0] = u53(c[0], c[1]);
+    r.v[1] = u53(c[2], c[3]);
     r.t0 = t0;
 }
 
-__device__ inline void gc_rng_get(const GcRng& r, unsigned long long t, double u[10]) {
-    const int l0 = 5 * (int)(t - r.t0);
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)r.c[0], l0 + k);
-        const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)r.c[1], l0 + k);
-        const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)r.c[2], l0 + k);
-        const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)r.c[3], l0 + k);
-        u[2 * k] = u53(a, b);
-        u[2 * k + 1] = u53(e, f);
-    }
-}
-
-// Sum over the 64 lanes of a wave by DPP row shifts and row broadcasts
-// (the total lands in lane 63), returned to every lane.
-template <int CTRL, int ROW_MASK>
+// The sums over the 64 lanes of a wave of four values at once: lanes 0-15 return
+// the total of a, 16-31 of c, 32-47 of b, 48-63 of d.  Two swaps of wave halves and
+// one of rows leave each row a quarter-sum of one value; four row rotations add it
+// up.  Four separate sums by row shifts and broadcasts took 24 dependent steps.
+template <int CTRL>
 __device__ inline double gc_dpp(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROW_MASK, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROW_MASK, 0xf, true);
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
 }
 
-__device__ inline double gc_wave_total(double v) {
-    v += gc_dpp<0x111, 0xf>(v);  // row_shr:1
-    v += gc_dpp<0x112, 0xf>(v);  // row_shr:2
-    v += gc_dpp<0x114, 0xf>(v);  // row_shr:4
-    v += gc_dpp<0x118, 0xf>(v);  // row_shr:8  -> lane 15 of each row holds the row's sum
-    v += gc_dpp<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-    v += gc_dpp<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3 -> lane 63 holds the total
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
-    return __hiloint2double(hi, lo);
+// lanes 0-31 of (a + the upper half's a), then 32-63 of b likewise
+__device__ inline double gc_fold32(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+
+// rows 0 and 2 of (a + its next row), rows 1 and 3 of b likewise
+__device__ inline double gc_fold16(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+
+__device__ inline double gc_wave_totals(double a, double b, double c, double d) {
+    double v = gc_fold16(gc_fold32(a, b), gc_fold32(c, d));
+    v += gc_dpp<0x128>(v);  // row_ror:8
+    v += gc_dpp<0x124>(v);
+    v += gc_dpp<0x122>(v);
+    v += gc_dpp<0x121>(v);
+    return v;
 }
 
 // sigma^2 / r^2 through the hardware reciprocal and two Newton steps (within
 // an ulp of the quotient), then 4 eps ratio (ratio - 1), ratio = x^3.
-__device__ inline double lj_pair(double r2, double2 se) {
-    double inv = __builtin_amdgcn_rcp(r2);
-    inv = fma(fma(-r2, inv, 1.0), inv, inv);
-    inv = fma(fma(-r2, inv, 1.0), inv, inv);
-    const double x = se.x * inv;
-    const double ratio = x * x * x;
-    return 4.0 * se.y * ratio * (ratio - 1.0);
+template <int Q>
+__device__ __attribute__((always_inline)) inline void gc_lj(const double (&r2)[Q], const double2 (&se)[Q], double (&e)[Q]) {
+    double inv[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) inv[q] = __builtin_amdgcn_rcp(r2[q]);
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) inv[q] = fma(fma(-r2[q], inv[q], 1.0), inv[q], inv[q]);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const double x = se[q].x * inv[q];
+        const double ratio = x * x * x;
+        e[q] = 4.0 * se[q].y * ratio * (ratio - 1.0);
+    }
 }
 
-// Accumulates the LJ pair (x site, y other) with the nearest image.
-__device__ inline void gc_pair(const GcmcParams& p, double4 x, double4 y, double2 se, double& acc, bool& ovl) {
-    double dx = y.x - x.x, dy = y.y - x.y, dz = y.z - x.z;
-    dx -= rint(dx);
-    dy -= rint(dy);
-    dz -= rint(dz);
-    const double cx = p.f[0] * dx + p.f[3] * dy + p.f[6] * dz;
-    const double cy = p.f[1] * dx + p.f[4] * dy + p.f[7] * dz;
-    const double cz = p.f[2] * dx + p.f[5] * dy + p.f[8] * dz;
-    const double r2 = cx * cx + cy * cy + cz * cz;
-    if (r2 < p.r2_cut) {
-        if (r2 < R2_OVERLAP) ovl = true;
-        else acc += lj_pair(r2, se);
+// x / y, inv = 1 / y: within an ulp of the quotient
+__device__ inline double gc_quotient(double x, double y, double inv) {
+    const double q = x * inv;
+    return isfinite(q) ? fma(fma(-q, y, x), inv, q) : q;
+}
+
+// What every move reads of the parameters, in vector registers for the launch: left
+// to itself the compiler loads it again each time, and a move waited for a dozen
+// scalar loads one after another.
+struct GcHot {
+    double f[6];    // f_to_c, upper triangle by columns
+    double c2f[9];
+    double r2_cut, omega;
+    int n_atoms, n_ads_types, n_species, n_sites0, type00, rot0;  // the last three of species 0, and of its first site
+};
+
+__device__ inline GcHot gc_hot(const GcmcParams& p) {
+    GcHot h;
+    constexpr int up[6] = {0, 3, 4, 6, 7, 8};
+#pragma unroll
+    for (int i = 0; i < 6; ++i) h.f[i] = gc_keep(p.f[up[i]]);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) h.c2f[i] = gc_keep(p.c2f[i]);
+    h.r2_cut = gc_keep(p.r2_cut);
+    h.omega = gc_keep(p.omega);
+    h.n_atoms = gc_keep_s(p.n_atoms);
+    h.n_ads_types = gc_keep_s(p.n_ads_types);
+    h.n_species = gc_keep_s(p.n_species);
+    h.n_sites0 = gc_keep_s(p.n_sites[0]);
+    h.type00 = gc_keep_s(p.site_type[0][0]);
+    h.rot0 = gc_keep_s(p.rotatable[0]);
+    return h;
+}
+
+// Sites of species s, and the type of its site k.
+__device__ inline int gc_n_sites(const GcmcParams& p, const GcHot& h, int s) { return s == 0 ? h.n_sites0 : p.n_sites[s]; }
+__device__ inline int gc_site_type(const GcmcParams& p, const GcHot& h, int s, int k) {
+    return (s | k) == 0 ? h.type00 : p.site_type[s][k];
+}
+
+// Q LJ pairs (x site, y other) with the nearest image: energies, zero where not ok,
+// past the cutoff or overlapping (then near).  Stage by stage over the pairs and
+// without branches, so that their dependent FP64 steps interleave.
+template <int Q>
+__device__ __attribute__((always_inline)) inline void gc_pairs(const GcHot& h, const double4 (&x)[Q],
+                                                               const double4 (&y)[Q], const double2 (&se)[Q],
+                                                               const bool (&ok)[Q], double (&e)[Q], bool (&near)[Q]) {
+    double dx[Q], dy[Q], dz[Q], r2[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        dx[q] = y[q].x - x[q].x;
+        dy[q] = y[q].y - x[q].y;
+        dz[q] = y[q].z - x[q].z;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        dx[q] -= rint(dx[q]);
+        dy[q] -= rint(dy[q]);
+        dz[q] -= rint(dz[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const double cx = h.f[0] * dx[q] + h.f[1] * dy[q] + h.f[3] * dz[q];  // (a along x)
+        const double cy = h.f[2] * dy[q] + h.f[4] * dz[q];
+        const double cz = h.f[5] * dz[q];
+        r2[q] = cx * cx + cy * cy + cz * cz;
+    }
+    gc_lj<Q>(r2, se, e);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const bool in = ok[q] && r2[q] < h.r2_cut, close = r2[q] < R2_OVERLAP;
+        near[q] = in && close;
+        e[q] = in && !close ? e[q] : 0.0;
     }
 }
 
 // Guest site jj of the flattened (species, molecule, site) list of stored
 // molecules, unless it lies past the end or belongs to the excluded molecule.
 template <typename Mols>
-__device__ inline bool gc_guest(const GcmcParams& p, const Mols& mols, const int* n, int jj, int total,
+__device__ inline bool gc_guest(const GcmcParams& p, const GcHot& hot, const Mols& mols, const int* n, int jj, int total,
                                 int ex_s, int ex_m, double4& y, int& ty) {
     if (jj >= total) return false;
-    int s2 = 0;
-    while (jj >= n[s2] * p.n_sites[s2]) {
-        jj -= n[s2] * p.n_sites[s2];
-        ++s2;
+    int m2 = jj, k2 = 0, s2 = 0;
+    if (hot.n_species > 1) {
+        while (m2 >= n[s2] * gc_n_sites(p, hot, s2)) {
+            m2 -= n[s2] * gc_n_sites(p, hot, s2);
+            ++s2;
+        }
     }
-    const int ns2 = p.n_sites[s2];
-    const int m2 = jj / ns2, k2 = jj - m2 * ns2;
+    const int ns2 = gc_n_sites(p, hot, s2);
+    if (ns2 > 1) {
+        k2 = m2 % ns2;
+        m2 /= ns2;
+    }
     if (s2 == ex_s && m2 == ex_m) return false;
     y = mols.site(p, s2, m2, k2);
-    ty = p.site_type[s2][k2];
+    ty = gc_site_type(p, hot, s2, k2);
     return true;
 }
 
-// Guest-host and guest-guest energy of a molecule of species ts with sites
-// trial[0..n_sites), against the framework and every stored molecule except
+// LDS of gc_energy: per parity the waves' sums (guest-host and guest-guest of the
+// first molecule, then of the second) and their overlap flags.
+constexpr int GC_WAVES = GC_WG / 64;
+static_assert(GC_WAVES == 4, "the flags of the waves are read as an int4");
+struct GcRed {
+    double sum[2][4][GC_WAVES];
+    int4 flags[2];
+};
+
+// Guest-host and guest-guest energies of NE molecules of species ts with sites
+// trial[e][0..n_sites), against the framework and every stored molecule except
 // (ex_s, ex_m).  Each work-item sums its atoms in index order, then its guest
-// sites; waves reduce by DPP and the four wave sums are added in wave order.
+// sites; the waves' sums are added in a fixed order.
 // +Inf on overlap.  `red` alternates between two halves (`par`), so the next
 // evaluation needs no barrier before writing its partial sums.
-template <typename Mols>
-__device__ __attribute__((always_inline)) inline void gc_energy(const GcmcParams& p, const Mols& mols,
+//
+// A chain is one evaluation after another, each bound by the latency of its
+// steps, not by their number (a chain's four waves have a SIMD each to themselves;
+// of some 4200 cycles per move 1600 issue vector instructions, 1700 wait): a
+// move's old and new position are evaluated together (NE = 2), reading every atom
+// once and reducing once; the pairs of a work-item and its first guest site go
+// through one batch.  8 methane chains of 600 cycles, 424 atoms: 23.8 -> 16.5 ms.
+template <int NE, typename Mols>
+__device__ __attribute__((always_inline)) inline void gc_energy(const GcmcParams& p, const GcHot& hot, const Mols& mols,
                                                                 const double4* atoms, const double2* fg,
                                                                 const double2* ggt, const int* n,
-                                                                const double4* trial, int ts, int ex_s, int ex_m,
-                                                                bool cells, double* red, int& par, double& gh,
-                                                                double& gg) {
+                                                                const double4* const (&trial)[NE], int ts, int ex_s,
+                                                                int ex_m, bool cells, GcRed& red, int& par,
+                                                                double (&gh)[NE], double (&gg)[NE]) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int ns = p.n_sites[ts];
-    const int na = p.n_ads_types;
+    const int ns = gc_n_sites(p, hot, ts);
+    const int na = hot.n_ads_types, n_atoms = hot.n_atoms;
     int total = 0;
 #pragma unroll
-    for (int q = 0; q < GC_NS; ++q) total += q < p.n_species ? n[q] * p.n_sites[q] : 0;
+    for (int q = 0; q < GC_NS; ++q) total += q < hot.n_species ? n[q] * gc_n_sites(p, hot, q) : 0;
     // the first guest site is loaded ahead of the framework loop
     int jj = tid;
     double4 y = make_double4(0.0, 0.0, 0.0, 0.0);
     int ty = 0;
-    bool have = gc_guest(p, mols, n, jj, total, ex_s, ex_m, y, ty);
-    double agh = 0.0, agg = 0.0;
-    bool ogh = false, ogg = false;
-    for (int k = 0; k < ns; ++k) {
-        const double4 x = trial[k];
-        const double2* col = fg + p.site_type[ts][k];
-        if (cells) {
-            // the atoms of the site's cell list; the others are beyond r_c
-            const double w0 = x.x - floor(x.x), w1 = x.y - floor(x.y), w2 = x.z - floor(x.z);
-            const int c0 = min(p.n_cell[0] - 1, (int)(w0 * p.n_cell[0]));
-            const int c1 = min(p.n_cell[1] - 1, (int)(w1 * p.n_cell[1]));
-            const int c2 = min(p.n_cell[2] - 1, (int)(w2 * p.n_cell[2]));
-            const int cell = __builtin_amdgcn_readfirstlane(c0 + p.n_cell[0] * (c1 + p.n_cell[1] * c2));
-            const int e = p.cell_start[cell + 1];
-            int j = p.cell_start[cell] + tid;
-            for (; j + 3 * GC_WG < e; j += 4 * GC_WG) {
-                const int i0 = p.cell_atoms[j], i1 = p.cell_atoms[j + GC_WG];
-                const int i2 = p.cell_atoms[j + 2 * GC_WG], i3 = p.cell_atoms[j + 3 * GC_WG];
-                const double4 a0 = atoms[i0], a1 = atoms[i1], a2 = atoms[i2], a3 = atoms[i3];
-                gc_pair(p, x, a0, col[(int)a0.w * na], agh, ogh);
-                gc_pair(p, x, a1, col[(int)a1.w * na], agh, ogh);
-                gc_pair(p, x, a2, col[(int)a2.w * na], agh, ogh);
-                gc_pair(p, x, a3, col[(int)a3.w * na], agh, ogh);
-            }
-            for (; j < e; j += GC_WG) {
-                const double4 at = atoms[p.cell_atoms[j]];
-                gc_pair(p, x, at, col[(int)at.w * na], agh, ogh);
-            }
-            continue;
-        }
-        int a = tid;
-        for (; a + 3 * GC_WG < p.n_atoms; a += 4 * GC_WG) {
-            const double4 a0 = atoms[a], a1 = atoms[a + GC_WG], a2 = atoms[a + 2 * GC_WG], a3 = atoms[a + 3 * GC_WG];
-            const double2 e0 = col[(int)a0.w * na], e1 = col[(int)a1.w * na];
-            const double2 e2 = col[(int)a2.w * na], e3 = col[(int)a3.w * na];
-            gc_pair(p, x, a0, e0, agh, ogh);
-            gc_pair(p, x, a1, e1, agh, ogh);
-            gc_pair(p, x, a2, e2, agh, ogh);
-            gc_pair(p, x, a3, e3, agh, ogh);
-        }
-        for (; a < p.n_atoms; a += GC_WG) {
-            const double4 at = atoms[a];
-            gc_pair(p, x, at, col[(int)at.w * na], agh, ogh);
-        }
-    }
-    while (jj < total) {
-        if (have)
-            for (int k = 0; k < ns; ++k) gc_pair(p, trial[k], y, ggt[p.site_type[ts][k] * na + ty], agg, ogg);
-        jj += GC_WG;
-        have = gc_guest(p, mols, n, jj, total, ex_s, ex_m, y, ty);
-    }
-    agh = gc_wave_total(agh);
-    agg = gc_wave_total(agg);
-    const bool bh = __ballot(ogh) != 0ull, bg = __ballot(ogg) != 0ull;
-    double* r = red + par * (4 * (GC_WG / 64));
-    par ^= 1;
-    if (lane == 0) {
-        r[wave] = agh;
-        r[GC_WG / 64 + wave] = agg;
-        r[2 * (GC_WG / 64) + wave] = bh ? 1.0 : 0.0;
-        r[3 * (GC_WG / 64) + wave] = bg ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    double sh = 0.0, sg = 0.0;
-    bool oh = false, og = false;
+    bool have = gc_guest(p, hot, mols, n, jj, total, ex_s, ex_m, y, ty);
+    double agh[NE], agg[NE];
+    bool ogh[NE], ogg[NE];
 #pragma unroll
-    for (int w = 0; w < GC_WG / 64; ++w) {
-        sh += r[w];
-        sg += r[GC_WG / 64 + w];
-        oh |= r[2 * (GC_WG / 64) + w] != 0.0;
-        og |= r[3 * (GC_WG / 64) + w] != 0.0;
+    for (int e = 0; e < NE; ++e) {
+        agh[e] = agg[e] = 0.0;
+        ogh[e] = ogg[e] = false;
     }
-    gh = oh ? INFINITY : sh;
-    gg = og ? INFINITY : sg;
+    // N others y against the NE sites x, added to acc and ovl in their order
+    const auto batch = [&](auto nc, const double4(&x)[NE], const auto& y_, const auto& se_, const auto& ok_, auto add) {
+        constexpr int N = decltype(nc)::value, Q = N * NE;
+        double4 xs[Q], ys[Q];
+        double2 se[Q];
+        bool ok[Q], near[Q];
+        double en[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            xs[q] = x[q % NE];
+            ys[q] = y_[q / NE];
+            se[q] = se_[q / NE];
+            ok[q] = ok_[q / NE];
+        }
+        gc_pairs<Q>(hot, xs, ys, se, ok, en, near);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) add(q / NE, q % NE, en[q], near[q]);
+    };
+    const auto add_host = [&](int, int e, double v, bool o) {
+        agh[e] += v;
+        ogh[e] |= o;
+    };
+    for (int k = 0; k < ns; ++k) {
+        double4 x[NE];
+#pragma unroll
+        for (int e = 0; e < NE; ++e) x[e] = trial[e][k];
+        const int tk = gc_site_type(p, hot, ts, k);
+        const double2* col = fg + tk;
+        int base = 0;
+        if (cells) {
+            // the atoms of each site's cell list; the others are beyond r_c
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+                const double w0 = x[e].x - floor(x[e].x), w1 = x[e].y - floor(x[e].y), w2 = x[e].z - floor(x[e].z);
+                const int c0 = min(p.n_cell[0] - 1, (int)(w0 * p.n_cell[0]));
+                const int c1 = min(p.n_cell[1] - 1, (int)(w1 * p.n_cell[1]));
+                const int c2 = min(p.n_cell[2] - 1, (int)(w2 * p.n_cell[2]));
+                const int cell = __builtin_amdgcn_readfirstlane(c0 + p.n_cell[0] * (c1 + p.n_cell[1] * c2));
+                const int end = p.cell_start[cell + 1];
+                for (int j = p.cell_start[cell] + tid; j < end; j += 4 * GC_WG) {
+                    double4 xs[4], at[4];
+                    double2 se[4];
+                    bool ok[4], near[4];
+                    double en[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        ok[q] = j + q * GC_WG < end;
+                        xs[q] = x[e];
+                        at[q] = atoms[p.cell_atoms[ok[q] ? j + q * GC_WG : j]];
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) se[q] = col[(int)at[q].w * na];
+                    gc_pairs<4>(hot, xs, at, se, ok, en, near);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) add_host(q, e, en[q], near[q]);
+                }
+            }
+            base = n_atoms;
+        }
+        for (; n_atoms - base > 2 * GC_WG; base += 4 * GC_WG) {
+            double4 at[4];
+            double2 se[4];
+            bool ok[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int a = base + tid + q * GC_WG;
+                ok[q] = a < n_atoms;
+                at[q] = atoms[ok[q] ? a : 0];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) se[q] = col[(int)at[q].w * na];
+            batch(std::integral_constant<int, 4>{}, x, at, se, ok, add_host);
+        }
+        // the last two and the first guest site together
+        double4 at[3];
+        double2 se[3];
+        bool ok[3];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int a = base + tid + q * GC_WG;
+            ok[q] = a < n_atoms;
+            at[q] = atoms[ok[q] ? a : 0];
+        }
+        at[2] = y;
+        ok[2] = have;
+        se[2] = ggt[tk * na + ty];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) se[q] = col[(int)at[q].w * na];
+        batch(std::integral_constant<int, 3>{}, x, at, se, ok, [&](int q, int e, double v, bool o) {
+            if (q < 2) {
+                agh[e] += v;
+                ogh[e] |= o;
+            } else {
+                agg[e] += v;
+                ogg[e] |= o;
+            }
+        });
+    }
+    for (jj += GC_WG; jj < total; jj += GC_WG) {
+        have = gc_guest(p, hot, mols, n, jj, total, ex_s, ex_m, y, ty);
+        for (int k = 0; k < ns; ++k) {
+            double4 x[NE];
+#pragma unroll
+            for (int e = 0; e < NE; ++e) x[e] = trial[e][k];
+            const double4 y1[1] = {y};
+            const double2 se[1] = {ggt[gc_site_type(p, hot, ts, k) * na + ty]};
+            const bool ok[1] = {have};
+            batch(std::integral_constant<int, 1>{}, x, y1, se, ok, [&](int, int e, double v, bool o) {
+                agg[e] += v;
+                ogg[e] |= o;
+            });
+        }
+    }
+    int flags = 0;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        flags |= (__ballot(ogh[e]) != 0ull ? 1 << e : 0) | (__ballot(ogg[e]) != 0ull ? 4 << e : 0);
+    }
+    const double tot = gc_wave_totals(agh[0], NE > 1 ? agh[NE - 1] : 0.0, agg[0], NE > 1 ? agg[NE - 1] : 0.0);
+    double (&r)[4][GC_WAVES] = red.sum[par];
+    int4& fl = red.flags[par];
+    par ^= 1;
+    if ((lane & 15) == 0) r[lane >> 4][wave] = tot;
+    if (lane == 0) reinterpret_cast<int*>(&fl)[wave] = flags;
+    __syncthreads();
+    const int4 f4 = fl;
+    const int any = f4.x | f4.y | f4.z | f4.w;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        const double* h = r[2 * e];
+        const double* q = r[2 * e + 1];
+        gh[e] = any & (1 << e) ? INFINITY : (h[0] + h[1]) + (h[2] + h[3]);
+        gg[e] = any & (4 << e) ? INFINITY : (q[0] + q[1]) + (q[2] + q[3]);
+    }
 }
 
 // Removes molecule m of species s, keeping the order of the others (splice!,
@@ -449,7 +612,8 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
     extern __shared__ double4 s_dyn[];
     __shared__ double4 s_trial[PM_MAX_SITES];
     __shared__ double4 s_old[PM_MAX_SITES];
-    __shared__ double s_red[2 * 4 * (GC_WG / 64)];
+    __shared__ GcRed s_red;
+    __shared__ unsigned long long s_count[2][GC_NM];
     const GcmcParams& p = *pp;
     GcmcChain& ch = chains[blockIdx.x];
     const int tid = threadIdx.x;
@@ -470,7 +634,7 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
     const GcMolsMem gmols{ch.sites, ch.com, p.capacity};
     using Mols = typename std::conditional<LDS_MOLS, GcMolsLds, GcMolsMem>::type;
     Mols mols;
-    if constexpr (LDS_MOLS) mols = GcMolsLds{lds_next, lds_cap};
+    if constexpr (LDS_MOLS) mols = GcMolsLds{lds_next, lds_cap, gc_keep_s(p.n_sites[0]), gc_keep_s(p.total_sites)};
     else mols = gmols;
     double fug[GC_NS];
 #pragma unroll
@@ -478,7 +642,7 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
     int par = 0;
     const bool cells_on = p.cell_start != nullptr;
     const unsigned chain = blockIdx.x;
-    const double T = ch.temperature;
+    const double T = ch.temperature, inv_T = 1.0 / T;
     int n[GC_NS];
 #pragma unroll
     for (int s = 0; s < GC_NS; ++s) n[s] = ch.n[s];
@@ -493,11 +657,19 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
     const long long target = resume ? ch.outer_target : outer + n_cycles;
     const long long outer_start = outer;
     bool stopped = false;
-    long long n_prop[GC_NM], n_acc[GC_NM];
-#pragma unroll
-    for (int k = 0; k < GC_NM; ++k) { n_prop[k] = ch.n_prop[k]; n_acc[k] = ch.n_acc[k]; }
+    // move counters: one work-item adds, nobody waits for it
+    if (tid < GC_NM) {
+        s_count[0][tid] = (unsigned long long)ch.n_prop[tid];
+        s_count[1][tid] = (unsigned long long)ch.n_acc[tid];
+    }
     int block = ch.block, error = 0;
-    const int S = p.n_species;
+    const int S = gc_keep_s(p.n_species), capacity = gc_keep_s(p.capacity);
+    const long long n_burn = gc_keep(p.n_burn);
+    const int sample_frequency = gc_keep_s((int)p.sample_frequency);
+    const GcHot hot = gc_hot(p);
+    double cum[GC_NM - 1];
+#pragma unroll
+    for (int q = 0; q < GC_NM - 1; ++q) cum[q] = gc_keep(p.cum[q]);
     // countdowns to the next multiple of each period (no 64-bit division per move)
     long long to_sample = p.sample_frequency - t % p.sample_frequency;
     long long to_snap = p.snapshot_frequency - outer % p.snapshot_frequency;
@@ -508,17 +680,16 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
     gc_rng_fill(rng, p.seed, chain, (unsigned long long)t + 1);
     // sums of the current statistics block, added to the chain's block at a
     // block change and at the end of the launch
-    long long acc_samples = 0, acc_n[GC_NS], acc_n2[GC_NS];
+    // (molecule counts: work-item q holds species q)
+    long long acc_samples = 0, acc_n = 0, acc_n2 = 0;
     double acc_gh = 0.0, acc_gg = 0.0, acc_gh2 = 0.0, acc_gg2 = 0.0, acc_un = 0.0;
-#pragma unroll
-    for (int q = 0; q < GC_NS; ++q) { acc_n[q] = 0; acc_n2[q] = 0; }
     auto flush = [&]() {
+        if (tid < GC_NS && acc_samples > 0) {
+            ch.blk_n[block][tid] += acc_n;
+            ch.blk_n2[block][tid] += acc_n2;
+        }
         if (tid == 0 && acc_samples > 0) {
             ch.blk_samples[block] += acc_samples;
-            for (int q = 0; q < GC_NS; ++q) {
-                ch.blk_n[block][q] += acc_n[q];
-                ch.blk_n2[block][q] += acc_n2[q];
-            }
             ch.blk_gh[block] += acc_gh;
             ch.blk_gg[block] += acc_gg;
             ch.blk_gh2[block] += acc_gh2;
@@ -527,7 +698,7 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
         }
         acc_samples = 0;
         acc_gh = acc_gg = acc_gh2 = acc_gg2 = acc_un = 0.0;
-        for (int q = 0; q < GC_NS; ++q) { acc_n[q] = 0; acc_n2[q] = 0; }
+        acc_n = acc_n2 = 0;
     };
     __syncthreads();
 
@@ -548,70 +719,75 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
         for (long long it = 0; it < inner; ++it) {
             ++t;
             if ((unsigned long long)t >= rng.t0 + GC_BATCH) gc_rng_fill(rng, p.seed, chain, (unsigned long long)t);
-            double u[10];
-            gc_rng_get(rng, (unsigned long long)t, u);
-            const int s = S > 1 ? min(S - 1, (int)(u[0] * (double)S)) : 0;
+            const auto u = [&](int k) { return rng.get((unsigned long long)t, k); };
+            const double u_acc = u(9);
+            const int s = S > 1 ? min(S - 1, (int)(u(0) * (double)S)) : 0;
             const int n_i = n[s];
-            int mv = 0;
-            while (mv < GC_NM - 1 && !(u[1] < p.cum[mv])) ++mv;
-            n_prop[mv] += 1;
-            const int ns = p.n_sites[s];
-            const bool rot = p.rotatable[s] != 0;
-            const int m = n_i > 0 ? min(n_i - 1, (int)(u[2] * (double)n_i)) : 0;
+            // the first move whose cumulative probability lies above
+            const double u_mv = u(1);
+            int mv = GC_NM - 1;
+#pragma unroll
+            for (int q = GC_NM - 2; q >= 0; --q) mv = u_mv < cum[q] ? q : mv;
+            if (tid == 0) atomicAdd(&s_count[0][mv], 1ull);
+            const int ns = gc_n_sites(p, hot, s);
+            const bool rot = (s == 0 ? hot.rot0 : p.rotatable[s]) != 0;
+            const int m = n_i > 0 ? min(n_i - 1, (int)(u(2) * (double)n_i)) : 0;
             if (mv == MV_INSERTION) {
-                if (n_i == p.capacity) {
+                if (n_i == capacity) {
                     error = 1;
                     break;
                 }
                 double R[9];
-                if (rot) arvo_rotation(&u[6], R);
-                const double4 com = make_double4(u[3], u[4], u[5], 0.0);
+                if (rot) {
+                    const double ur[3] = {u(6), u(7), u(8)};
+                    arvo_rotation(ur, R);
+                }
+                const double4 com = make_double4(u(3), u(4), u(5), 0.0);
                 if (tid < ns) s_trial[tid] = gc_new_site(p, s, tid, com, R, rot);
                 __syncthreads();
-                double gh, gg;
-                gc_energy(p, mols, atoms, s_fg, s_gg, n, s_trial, s, -1, -1, cells_on, s_red, par, gh, gg);
-                const double dE = (gg + 0.0) + gh + 0.0;
-                const double acc = fug[s] * p.omega / ((double)(n_i + 1) * GC_KB * T) * exp(-dE / T);
-                if (u[9] < acc) {
+                double gh[1], gg[1];
+                gc_energy<1>(p, hot, mols, atoms, s_fg, s_gg, n, {s_trial}, s, -1, -1, cells_on, s_red, par, gh, gg);
+                const double dE = (gg[0] + 0.0) + gh[0] + 0.0;
+                // (an overlap is rejected without the exponential)
+                if (dE < INFINITY &&
+                    u_acc < fug[s] * hot.omega / ((double)(n_i + 1) * GC_KB * T) * exp(-gc_quotient(dE, T, inv_T))) {
                     gc_store(p, mols, s, n_i, s_trial, com);
                     n[s] = n_i + 1;
-                    n_acc[mv] += 1;
-                    e_gh += gh;
-                    e_gg += gg;
+                    if (tid == 0) atomicAdd(&s_count[1][mv], 1ull);
+                    e_gh += gh[0];
+                    e_gg += gg[0];
                 }
             } else if (mv == MV_DELETION && n_i != 0) {
                 if (tid < ns) s_trial[tid] = mols.site(p, s, m, tid);
                 __syncthreads();
-                double gh, gg;
-                gc_energy(p, mols, atoms, s_fg, s_gg, n, s_trial, s, s, m, cells_on, s_red, par, gh, gg);
-                const double dE = (gg + 0.0) + gh + 0.0;
-                const double acc = (double)n_i * GC_KB * T / (fug[s] * p.omega) * exp(dE / T);
-                if (u[9] < acc) {
+                double gh[1], gg[1];
+                gc_energy<1>(p, hot, mols, atoms, s_fg, s_gg, n, {s_trial}, s, s, m, cells_on, s_red, par, gh, gg);
+                const double dE = (gg[0] + 0.0) + gh[0] + 0.0;
+                const double acc = (double)n_i * GC_KB * T / (fug[s] * hot.omega) * exp(gc_quotient(dE, T, inv_T));
+                if (u_acc < acc) {
                     gc_remove(p, mols, s, m, n_i);
                     n[s] = n_i - 1;
-                    n_acc[mv] += 1;
-                    e_gh -= gh;
-                    e_gg -= gg;
+                    if (tid == 0) atomicAdd(&s_count[1][mv], 1ull);
+                    e_gh -= gh[0];
+                    e_gg -= gg[0];
                 }
             } else if ((mv == MV_TRANSLATION || (mv == MV_ROTATION && rot) || mv == MV_REINSERTION) && n_i != 0) {
                 if (mv == MV_TRANSLATION) ntp += 1;
                 const double4 com0 = mols.com(p, s, m);
-                if (tid < ns) s_old[tid] = mols.site(p, s, m, tid);
-                __syncthreads();
-                double gh0, gg0, gh1, gg1;
-                gc_energy(p, mols, atoms, s_fg, s_gg, n, s_old, s, s, m, cells_on, s_red, par, gh0, gg0);
+                const double4 old = tid < ns ? mols.site(p, s, m, tid) : make_double4(0.0, 0.0, 0.0, 0.0);
+                if (tid < ns) s_old[tid] = old;
                 double4 com1 = com0;
                 {
 #pragma clang fp contract(off)
                     if (mv == MV_TRANSLATION) {
                         // Cartesian step in a cube of side delta, then periodic COM
                         // (random_translation!, src/mc_helpers.jl:142-153)
-                        const double d0 = delta * (u[3] - 0.5), d1 = delta * (u[4] - 0.5), d2 = delta * (u[5] - 0.5);
-                        const double* c = p.c2f;
+                        const double d0 = delta * (u(3) - 0.5), d1 = delta * (u(4) - 0.5), d2 = delta * (u(5) - 0.5);
+                        const double* c = hot.c2f;
                         const double f0 = c[0] * d0 + c[3] * d1 + c[6] * d2;
                         const double f1 = c[1] * d0 + c[4] * d1 + c[7] * d2;
                         const double f2 = c[2] * d0 + c[5] * d1 + c[8] * d2;
-                        double4 x = tid < ns ? s_old[tid] : make_double4(0.0, 0.0, 0.0, 0.0);
+                        double4 x = old;
                         x.x += f0; x.y += f1; x.z += f2;
                         com1.x += f0; com1.y += f1; com1.z += f2;
                         if (com1.x > 1.0 || com1.y > 1.0 || com1.z > 1.0 || com1.x < 0.0 || com1.y < 0.0 ||
@@ -627,16 +803,17 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
                         }
                         if (tid < ns) s_trial[tid] = x;
                     } else {
-                        double4 x = tid < ns ? s_old[tid] : make_double4(0.0, 0.0, 0.0, 0.0);
+                        double4 x = old;
                         if (mv == MV_REINSERTION) {
                             // translate_to! a uniform point (random_reinsertion!, src/mc_helpers.jl:168-182)
-                            const double e0 = u[3] - com0.x, e1 = u[4] - com0.y, e2 = u[5] - com0.z;
+                            const double e0 = u(3) - com0.x, e1 = u(4) - com0.y, e2 = u(5) - com0.z;
                             x.x += e0; x.y += e1; x.z += e2;
                             com1.x += e0; com1.y += e1; com1.z += e2;
                         }
                         if (rot) {
                             double R[9], Rf[9];
-                            arvo_rotation(&u[6], R);
+                            const double ur[3] = {u(6), u(7), u(8)};
+                            arvo_rotation(ur, R);
                             gc_frac_rotation(p, R, Rf);
                             x = gc_rotate_site(Rf, x, com1);
                         }
@@ -644,45 +821,51 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
                     }
                 }
                 __syncthreads();
-                gc_energy(p, mols, atoms, s_fg, s_gg, n, s_trial, s, s, m, cells_on, s_red, par, gh1, gg1);
-                const double e_new = (gg1 + 0.0) + gh1 + 0.0, e_old = (gg0 + 0.0) + gh0 + 0.0;
-                if (u[9] < exp(-(e_new - e_old) / T)) {
+                double gh[2], gg[2];
+                gc_energy<2>(p, hot, mols, atoms, s_fg, s_gg, n, {s_old, s_trial}, s, s, m, cells_on, s_red, par, gh, gg);
+                const double e_new = (gg[1] + 0.0) + gh[1] + 0.0, e_old = (gg[0] + 0.0) + gh[0] + 0.0;
+                const double dE = e_new - e_old;
+                // (a step downhill or into an overlap is decided without the exponential)
+                if (dE <= 0.0 || (dE < INFINITY && u_acc < exp(-gc_quotient(dE, T, inv_T)))) {
                     gc_store(p, mols, s, m, s_trial, com1);
-                    n_acc[mv] += 1;
+                    if (tid == 0) atomicAdd(&s_count[1][mv], 1ull);
                     if (mv == MV_TRANSLATION) nta += 1;
-                    e_gh += gh1 - gh0;
-                    e_gg += gg1 - gg0;
+                    e_gh += gh[1] - gh[0];
+                    e_gg += gg[1] - gg[0];
                 }
             } else if (mv == MV_IDENTITY && n_i != 0) {
                 // src/gcmc.jl:566-613
                 const double4 com0 = mols.com(p, s, m);
                 if (tid < ns) s_old[tid] = mols.site(p, s, m, tid);
                 __syncthreads();
-                double gh0, gg0, gh1, gg1;
-                gc_energy(p, mols, atoms, s_fg, s_gg, n, s_old, s, s, m, cells_on, s_red, par, gh0, gg0);
+                double gh0[1], gg0[1], gh1[1], gg1[1];
+                gc_energy<1>(p, hot, mols, atoms, s_fg, s_gg, n, {s_old}, s, s, m, cells_on, s_red, par, gh0, gg0);
                 gc_remove(p, mols, s, m, n_i);
                 n[s] = n_i - 1;
-                int pick = min(S - 2, (int)(u[3] * (double)(S - 1)));
+                int pick = min(S - 2, (int)(u(3) * (double)(S - 1)));
                 const int s2 = pick < s ? pick : pick + 1;
                 const int n_j = n[s2];
-                if (n_j == p.capacity) {
+                if (n_j == capacity) {
                     error = 1;
                     break;
                 }
                 double R[9];
                 const bool rot2 = p.rotatable[s2] != 0;
-                if (rot2) arvo_rotation(&u[6], R);
+                if (rot2) {
+                    const double ur[3] = {u(6), u(7), u(8)};
+                    arvo_rotation(ur, R);
+                }
                 if (tid < p.n_sites[s2]) s_trial[tid] = gc_new_site(p, s2, tid, com0, R, rot2);
                 __syncthreads();
-                gc_energy(p, mols, atoms, s_fg, s_gg, n, s_trial, s2, -1, -1, cells_on, s_red, par, gh1, gg1);
-                const double e_new = (gg1 + 0.0) + gh1 + 0.0, e_old = (gg0 + 0.0) + gh0 + 0.0;
-                const double acc = ((double)n_i * fug[s2] / ((double)(n_j + 1) * fug[s])) * exp(-(e_new - e_old) / T);
-                if (u[9] < acc) {
+                gc_energy<1>(p, hot, mols, atoms, s_fg, s_gg, n, {s_trial}, s2, -1, -1, cells_on, s_red, par, gh1, gg1);
+                const double e_new = (gg1[0] + 0.0) + gh1[0] + 0.0, e_old = (gg0[0] + 0.0) + gh0[0] + 0.0;
+                const double acc = ((double)n_i * fug[s2] / ((double)(n_j + 1) * fug[s])) * exp(-gc_quotient(e_new - e_old, T, inv_T));
+                if (u_acc < acc) {
                     gc_store(p, mols, s2, n_j, s_trial, com0);
                     n[s2] = n_j + 1;
-                    n_acc[mv] += 1;
-                    e_gh += gh1 - gh0;
-                    e_gg += gg1 - gg0;
+                    if (tid == 0) atomicAdd(&s_count[1][mv], 1ull);
+                    e_gh += gh1[0] - gh0[0];
+                    e_gg += gg1[0] - gg0[0];
                 } else {
                     // the original molecule goes back at the end of its species' list
                     gc_store(p, mols, s, n[s], s_old, com0);
@@ -690,15 +873,16 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
                 }
             }
             const bool sample_now = --to_sample == 0;
-            if (sample_now) to_sample = p.sample_frequency;
-            if (outer > p.n_burn && sample_now) {
-                long long ntot = 0;
+            if (sample_now) to_sample = sample_frequency;
+            if (outer > n_burn && sample_now) {
+                int ntot = 0, mine = 0;
 #pragma unroll
                 for (int q = 0; q < GC_NS; ++q) {
                     ntot += n[q];
-                    acc_n[q] += n[q];
-                    acc_n2[q] += (long long)n[q] * n[q];
+                    mine = tid == q ? n[q] : mine;
                 }
+                acc_n += mine;
+                acc_n2 += (long long)mine * mine;
                 acc_samples += 1;
                 acc_gh += e_gh;
                 acc_gg += e_gg;
@@ -747,6 +931,10 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
         if (fits && outer != outer_start) gc_mols_copy(p, mols, gmols, n);
         if (stopped && tid == 0) atomicAdd(incomplete, 1);
     }
+    if (tid < GC_NM) {
+        ch.n_prop[tid] = (long long)s_count[0][tid];
+        ch.n_acc[tid] = (long long)s_count[1][tid];
+    }
     if (tid == 0) {
         ch.outer_target = target;
         for (int s = 0; s < GC_NS; ++s) ch.n[s] = n[s];
@@ -758,7 +946,6 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
         ch.n_trans_prop = ntp;
         ch.n_trans_acc = nta;
         ch.num_snapshots = nsnap;
-        for (int k = 0; k < GC_NM; ++k) { ch.n_prop[k] = n_prop[k]; ch.n_acc[k] = n_acc[k]; }
         ch.block = block;
         ch.error = error;
     }
@@ -769,23 +956,24 @@ __global__ __launch_bounds__(GC_WG) void gcmc_kernel(const GcmcParams* __restric
 __global__ __launch_bounds__(GC_WG) void gcmc_total_energy_kernel(const GcmcParams* __restrict__ pp,
                                                                   GcmcChain* chains, double* out) {
     __shared__ double4 s_trial[PM_MAX_SITES];
-    __shared__ double s_red[2 * 4 * (GC_WG / 64)];
+    __shared__ GcRed s_red;
     const GcmcParams& p = *pp;
     GcmcChain& ch = chains[blockIdx.x];
     const GcMolsMem mols{ch.sites, ch.com, p.capacity};
     int n[GC_NS];
 #pragma unroll
     for (int s = 0; s < GC_NS; ++s) n[s] = ch.n[s];
+    const GcHot hot = gc_hot(p);
     int par = 0;
     double tgh = 0.0, tgg = 0.0;
     for (int s = 0; s < p.n_species; ++s) {
         for (int m = 0; m < n[s]; ++m) {
             if (threadIdx.x < p.n_sites[s]) s_trial[threadIdx.x] = mols.site(p, s, m, threadIdx.x);
             __syncthreads();
-            double gh, gg;
-            gc_energy(p, mols, p.atoms, p.lj_fg, p.lj_gg, n, s_trial, s, s, m, false, s_red, par, gh, gg);
-            tgh += gh;
-            tgg += gg;
+            double gh[1], gg[1];
+            gc_energy<1>(p, hot, mols, p.atoms, p.lj_fg, p.lj_gg, n, {s_trial}, s, s, m, false, s_red, par, gh, gg);
+            tgh += gh[0];
+            tgg += gg[0];
         }
     }
     if (threadIdx.x == 0) {
