@@ -867,7 +867,7 @@ struct TypeSums {
 // tile never spans two bins), so each tile's candidates are taken type by type,
 // with the type's parameters held in registers, and folded into the type's FP64
 // sums once.
-template <int ESM, typename Real, int NT, int SPLIT>
+template <int ESM, typename Real, int NT, int SPLIT, int PW>
 __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs& a, bool valid, double px, double py, double pz,
                                    int site, const LJC<Real>* s_lj, const double2* s_gc,
                                    const PairLds& L, double& acc_lj, double& acc_sr, bool& ovl,
@@ -920,9 +920,10 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                 acc_lj += part_lj;
                 acc_sr += part_sr;
             } else {
-                // (each part belongs to one wave of the workgroup)
-                if (part_lj != 0.0) L.part[part * 64 + lane] = part_lj;
-                if (part_sr != 0.0) L.part[(LIST_PARTS + part) * 64 + lane] = part_sr;
+                // (each part of a point belongs to one wave of the workgroup)
+                constexpr int NP = 64 * PW;
+                if (part_lj != 0.0) L.part[part * NP + (tid & (NP - 1))] = part_lj;
+                if (part_sr != 0.0) L.part[(LIST_PARTS + part) * NP + (tid & (NP - 1))] = part_sr;
             }
             part_lj = 0.0;
             part_sr = 0.0;
@@ -937,7 +938,7 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                 const double rr = Rc + sp.w;
                 hit = sx * sx + sy * sy + sz * sz < rr * rr;
                 if constexpr (SPLIT > 1)
-                    hit = hit && (tile_part(tb + lane, n_tiles) & (SPLIT - 1)) == (tid >> 6);
+                    hit = hit && (tile_part(tb + lane, n_tiles) & (SPLIT - 1)) == tid / (64 * PW);
             }
             for (unsigned long long hm = __ballot(hit); hm != 0ull; hm &= hm - 1ull) {
                 const int ti = tb + __builtin_ctzll(hm);
@@ -1035,28 +1036,29 @@ constexpr int pair_waves() {
     return sizeof(Real) == 4 && NT == 6 ? 4 : 1;
 }
 
-// Work-items of a pair workgroup.  SPLIT = 1: a slice of WG points, a wave for 64
-// of them.  SPLIT = 4, 16: 64 points, whose image list SPLIT waves share out.
-constexpr int pair_wg(int split) { return split == 16 ? 1024 : WG; }
+// A pair workgroup has 64 PW points, and SPLIT waves for each 64 of them that
+// share out the image list.
+constexpr int pair_wg(int split, int pw) { return 64 * split * pw; }
 // LDS of the SPLIT kernels for the parts' LJ and real-space sums [part][point]
 // and the waves' overlap masks.
-constexpr int pair_lds_parts(int split) {
-    return split > 1 ? (2 * LIST_PARTS * 64 + split) * (int)sizeof(double) : 0;
+constexpr int pair_lds_parts(int split, int pw) {
+    return split > 1 ? (2 * LIST_PARTS * 64 + split) * pw * (int)sizeof(double) : 0;
 }
 
 // NT = 0: energies.  NT > 0: a gradient run of at most NT framework types.
 // SPLIT (energies, image-list path): a small launch leaves most of the 1024
 // SIMDs without a wave while a few walk the whole list, one dependent load after
 // another; with the list shared out each wave's chain is SPLIT times shorter, for
-// SPLIT times the tile tests and table loads (1000 CH4 insertions, 424 atoms: 70
-// -> 28 us; 1000 CO2, 600 atoms: 182 -> 55, in FP64 252 -> 80).  The first wave
-// adds the parts' sums from LDS.
-template <typename Real, int NT, int SPLIT>
-__global__ __launch_bounds__(pair_wg(SPLIT), (pair_waves<Real, NT>())) void point_pair_kernel(GroupArgs g, int extra_off) {
+// SPLIT times the tile tests (1000 CH4 insertions, 424 atoms: 70 -> 28 us; 1000
+// CO2, 600 atoms: 182 -> 55, in FP64 252 -> 80; 20000: 138 -> 94).  More points per
+// workgroup (PW) share a load of the tables.
+template <typename Real, int NT, int SPLIT, int PW>
+__global__ __launch_bounds__(pair_wg(SPLIT, PW), (pair_waves<Real, NT>())) void point_pair_kernel(GroupArgs g, int extra_off) {
     constexpr bool GRAD = NT > 0;
     static_assert(!GRAD || SPLIT == 1, "gradient runs are not split");
-    constexpr int SUB = SPLIT == 1 ? 1 : WG / 64;  // workgroups per slice or brick
-    constexpr int NTH = pair_wg(SPLIT);
+    constexpr int NP = 64 * PW;      // points
+    constexpr int SUB = WG / NP;     // workgroups per slice or brick
+    constexpr int NTH = pair_wg(SPLIT, PW);
     extern __shared__ __align__(16) unsigned char smem[];
     float4* s_erfc = reinterpret_cast<float4*>(smem);
     double2* s_erfc64 = reinterpret_cast<double2*>(smem);
@@ -1070,7 +1072,7 @@ __global__ __launch_bounds__(pair_wg(SPLIT), (pair_waves<Real, NT>())) void poin
 
     const int tid = threadIdx.x;
     const unsigned wg = blockIdx.x / SUB;                                            // slice or brick
-    const int pt = SPLIT == 1 ? tid : (int)(blockIdx.x % SUB) * 64 + (tid & 63);     // point of it
+    const int pt = (int)(blockIdx.x % SUB) * NP + (tid & (NP - 1));                  // point of it
     int si;
     uint4 it = make_uint4(0u, 0u, 0u, 0u);
     if (g.mode == MODE_WIDOM) {
@@ -1091,6 +1093,8 @@ __global__ __launch_bounds__(pair_wg(SPLIT), (pair_waves<Real, NT>())) void poin
     int site;
     if (g.mode == MODE_WIDOM) {
         const unsigned k = g.point_off[it.x] + it.y * WG + pt;
+        if constexpr (SPLIT > 1)
+            if (k - (unsigned)(tid & (NP - 1)) >= g.point_off[it.x + 1]) return;  // the whole workgroup
         valid = k < g.point_off[it.x + 1];
         pid = valid ? (long long)g.order[k] : sg.slot_base;
         const double4 p = valid ? g.pos[pid] : make_double4(0.0, 0.0, 0.0, 0.0);
@@ -1113,8 +1117,6 @@ __global__ __launch_bounds__(pair_wg(SPLIT), (pair_waves<Real, NT>())) void poin
         pz = grid_coord(k, n3, a.repd[2]);
         site = 0;
     }
-    if constexpr (SPLIT > 1)
-        if (__ballot(valid) == 0ull) return;  // the whole workgroup: its waves hold the same points
     const int n_tab = a.n_types * a.nsite;
     const LJC<Real>* gtab = reinterpret_cast<const LJC<Real>*>(a.ljtab);
     for (int t = tid; t < n_tab; t += NTH) s_lj[t] = gtab[t];
@@ -1129,7 +1131,7 @@ __global__ __launch_bounds__(pair_wg(SPLIT), (pair_waves<Real, NT>())) void poin
         if (a.esm != 0)
             for (int t = tid; t < ERFC64_TAB; t += NTH) s_erfc64[t] = a.erfc64_tab[t];
     if constexpr (SPLIT > 1)
-        for (int t = tid; t < 2 * LIST_PARTS * 64; t += NTH) L.part[t] = 0.0;
+        for (int t = tid; t < 2 * LIST_PARTS * NP; t += NTH) L.part[t] = 0.0;
     __syncthreads();
 
     double acc_lj = 0.0, acc_sr = 0.0;
@@ -1137,13 +1139,13 @@ __global__ __launch_bounds__(pair_wg(SPLIT), (pair_waves<Real, NT>())) void poin
     unsigned long long n_cand = 0;
     TypeSums<Real, (NT > 0 ? NT : 1)> ts;
     if (a.esm == 0)
-        chunk_pairs<0, Real, NT, SPLIT>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
+        chunk_pairs<0, Real, NT, SPLIT, PW>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
                                  n_cand, ts);
     else if (a.esm == 1)
-        chunk_pairs<1, Real, NT, SPLIT>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
+        chunk_pairs<1, Real, NT, SPLIT, PW>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
                                  n_cand, ts);
     else
-        chunk_pairs<2, Real, NT, SPLIT>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
+        chunk_pairs<2, Real, NT, SPLIT, PW>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
                                  n_cand, ts);
     if (g.cand_pairs != nullptr) {
         const unsigned long long m = __ballot(valid);
@@ -1151,18 +1153,18 @@ __global__ __launch_bounds__(pair_wg(SPLIT), (pair_waves<Real, NT>())) void poin
             atomicAdd(g.cand_pairs, (unsigned long long)__popcll(m) * n_cand);
     }
     if constexpr (SPLIT > 1) {
-        // the first wave adds up the parts' sums, in the order of the list
-        unsigned long long* const s_ovl = reinterpret_cast<unsigned long long*>(L.part + 2 * LIST_PARTS * 64);
+        // a wave per 64 points adds up the parts' sums, in the order of the list
+        unsigned long long* const s_ovl = reinterpret_cast<unsigned long long*>(L.part + 2 * LIST_PARTS * NP);
         const unsigned long long om = __ballot(ovl);
         if ((tid & 63) == 0) s_ovl[tid >> 6] = om;
         __syncthreads();
-        if (tid >= 64) return;
+        if (tid >= NP) return;
         unsigned long long any = 0ull;
-        for (int w = 0; w < SPLIT; ++w) any |= s_ovl[w];
-        ovl = (any >> tid) & 1ull;
+        for (int w = 0; w < SPLIT; ++w) any |= s_ovl[w * PW + (tid >> 6)];
+        ovl = (any >> (tid & 63)) & 1ull;
         for (int p = 0; p < LIST_PARTS; ++p) {
-            acc_lj += L.part[p * 64 + tid];
-            acc_sr += L.part[(LIST_PARTS + p) * 64 + tid];
+            acc_lj += L.part[p * NP + tid];
+            acc_sr += L.part[(LIST_PARTS + p) * NP + tid];
         }
     }
     if (valid) {

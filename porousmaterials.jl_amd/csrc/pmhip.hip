@@ -982,26 +982,31 @@ int grid_prepare(const pm_grid_run& in, PointRun& r) {
     return PM_OK;
 }
 
-template <typename Real, int NT, int SPLIT = 1>
+template <typename Real, int NT, int SPLIT = 1, int PW = WG / 64>
 void pair_launch_t(const GroupArgs& g, int n_wg, size_t shm, int extra_off) {
-    constexpr int sub = SPLIT == 1 ? 1 : WG / 64;
-    hipLaunchKernelGGL((point_pair_kernel<Real, NT, SPLIT>), dim3(n_wg * sub), dim3(pair_wg(SPLIT)),
-                       shm + pair_lds_parts(SPLIT), g_ctx.stream, g, extra_off);
+    constexpr int sub = WG / (64 * PW);
+    hipLaunchKernelGGL((point_pair_kernel<Real, NT, SPLIT, PW>), dim3(n_wg * sub), dim3(pair_wg(SPLIT, PW)),
+                       shm + pair_lds_parts(SPLIT, PW), g_ctx.stream, g, extra_off);
 }
 
-// Waves that share out the image list of 64 points, by the 64-point waves of the
-// launch: one from a wave per SIMD on, four below, sixteen where even four leave
-// most SIMDs idle.  Pair kernel with 1, 4 and 16 (us): 156 waves (CH4 insertions)
-// 153, 85, 52; 469 (CO2) 146, 99, 126; 469 (CH4) 121, 76, 119; 1406 (CO2) 142,
-// 129, 335, in FP64 212, 238, 367; 1562 (CH4) 118, 129, 361; 2197 (50^3 grid) 64,
-// 131, 447.
-int pair_split(long long n_waves) { return n_waves >= 1024 ? 1 : n_waves >= 192 ? 4 : 16; }
+// Waves that share out the image list of each 64 points, by the 64-point waves of
+// the launch (pair kernel, us: one wave; 2 in workgroups of 256 points; 8 of 128; 16
+// of 64).  CO2 in 600 atoms: 141 waves 196, 127, 83, 62; 469 waves 148, 98, 74, 128;
+// 937 waves 138, 94, 123, 230; 1406 waves 143, 116, 173, 340; 2812 waves 167, 168,
+// 316, 648; in FP64, 937 waves 192, 137, 158, 262; 1406 waves 209, 222, 217, 369.
+// CH4 in 600 atoms: 156 waves 158, 99, 68, 54; 469 waves 122, 81, 69, 121; 1562 waves
+// 122, 93, 204, 363.  CH4 grids: 216 waves 52, 36, 31, 55; 512 waves 49, 36, 60, 112;
+// 1000 waves 51, 47, 107, 209; 2548 waves 65, 87, 227, 449.
+int pair_split(long long n_waves, bool fp64) {
+    return n_waves < 160 ? 16 : n_waves < 640 ? 8 : n_waves < (fp64 ? 1024 : 1792) ? 2 : 1;
+}
 
 template <typename Real>
 void pair_launch_plain(const GroupArgs& g, int n_wg, size_t shm, int extra_off, int split) {
     switch (split) {
-        case 16: pair_launch_t<Real, 0, 16>(g, n_wg, shm, extra_off); break;
-        case 4: pair_launch_t<Real, 0, 4>(g, n_wg, shm, extra_off); break;
+        case 16: pair_launch_t<Real, 0, 16, 1>(g, n_wg, shm, extra_off); break;
+        case 8: pair_launch_t<Real, 0, 8, 2>(g, n_wg, shm, extra_off); break;
+        case 2: pair_launch_t<Real, 0, 2, 4>(g, n_wg, shm, extra_off); break;
         default: pair_launch_t<Real, 0>(g, n_wg, shm, extra_off); break;
     }
 }
@@ -1436,11 +1441,11 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
             if (fp64) pair_launch_grad<double>(g, (int)pair_wg, shm, extra_off, nt_grad);
             else pair_launch_grad<float>(g, (int)pair_wg, shm, extra_off, nt_grad);
         } else {
-            // (a run on the all-atoms path is not split, nor one whose tables fill
-            // the LDS that any kernel may take)
+            // (a run on the all-atoms path is not split, nor one whose tables leave too
+            // little LDS)
             const long long n_waves = (widom ? gr.n_slots : gr.n_wg * WG) / 64;
-            const bool can_split = all_fast && shm + pair_lds_parts(16) <= 65536;
-            const int split = can_split ? pair_split(n_waves) : 1;
+            const bool can_split = all_fast && shm + pair_lds_parts(2, 4) <= g_ctx.max_lds;
+            const int split = can_split ? pair_split(n_waves, fp64) : 1;
             if (fp64) pair_launch_plain<double>(g, (int)pair_wg, shm, extra_off, split);
             else pair_launch_plain<float>(g, (int)pair_wg, shm, extra_off, split);
         }

@@ -1,4 +1,4 @@
-"""Small launches share the image list of 64 points out over 4 or 16 waves; a
+"""Small launches share the image list of 64 points out over 2, 8 or 16 waves; a
 point's energies are the same bit for bit whichever kernel takes them, because
 the FP64 sums run over fixed parts of the list in fixed order.
 
@@ -17,7 +17,8 @@ from test_gpu_batch import _handles
 
 pytestmark = pytest.mark.gpu
 
-SIZES = {"CH4": (1, 64, 65, 12_200, 12_300, 65_400, 65_600), "CO2": (1, 65, 4_090, 4_100, 21_800, 21_900)}
+SIZES = {"CH4": (1, 64, 65, 10_000, 10_500, 40_700, 41_200, 65_200, 65_800, 114_400, 115_000),
+         "CO2": (1, 65, 3_300, 3_500, 13_500, 13_800, 21_700, 22_000, 38_100, 38_400)}
 
 
 @pytest.mark.parametrize("name", ["CH4", "CO2"])
@@ -41,7 +42,7 @@ def test_list_of_fewer_tiles_than_parts(pm, precision):
                    np.array([[0.1, 0.6], [0.2, 0.5], [0.3, 0.5]]))
     fw, pr = pm.device.framework(x, ff), pm.device.probe(pm.lj_sphere("CH4"), ff)
     en = [pm.device.widom(fw, ff, None, pr, 298.0, 5, 1, n, precision, return_energies=True)[1]
-          for n in (1000, 20_000, 70_000)]
+          for n in (1000, 20_000, 50_000, 120_000)]
     assert (en[0] != 0.0).any()
     for e in en[:-1]:
         np.testing.assert_array_equal(e, en[-1][:len(e)])
