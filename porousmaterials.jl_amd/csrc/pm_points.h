@@ -416,6 +416,9 @@ __global__ void stage_points_kernel(const uint2* cell, long long n_pts, const un
 // super-bin's points are a contiguous stretch of the sorted order) and, within
 // the super-bin, their slice offsets (ceil(count / WG) slices per cell), then
 // every point to its (cell, slab)'s stretch of `order`.
+// The offsets come from a scan over the keys and another over the cells' slices
+// (a walk over each cell's slabs by one work-item: 48 screening runs, 69 us
+// instead of 42).
 __global__ __launch_bounds__(SCAN_WG) void cell_sort_kernel(const uint2* stage, const unsigned* sb_off, int sb_shift,
                                                             int zstride, int n_cells, unsigned* count,
                                                             unsigned* point_off, unsigned* slice_loc,
@@ -443,36 +446,40 @@ __global__ __launch_bounds__(SCAN_WG) void cell_sort_kernel(const uint2* stage, 
                 atomicAdd(&s_n[((cl[j] & CELL_MASK) - c_lo) * zstride + (cl[j] >> 24)], 1u);
     }
     __syncthreads();
-    // each work-item a run of consecutive cells
+    // keys: exclusive offsets, each work-item a run of consecutive keys
+    constexpr int KEYS = SB_KEYS_MAX / SCAN_WG;
+    unsigned v[KEYS], p = 0u, none = 0u, tp, ts;
+#pragma unroll
+    for (int j = 0; j < KEYS; ++j) {
+        const int k = tid * KEYS + j;
+        v[j] = k < nk ? s_n[k] : 0u;
+        p += v[j];
+    }
+    scan_pair_1024(p, none, tp, ts);  // (its barriers also order the reads above before the writes below)
+    p += lo;
+#pragma unroll
+    for (int j = 0; j < KEYS; ++j) {
+        const int k = tid * KEYS + j;
+        if (k < nk) s_n[k] = p;  // the next free position of the (cell, slab)
+        p += v[j];
+    }
+    __syncthreads();
+    // cells: a run of consecutive ones each, their counts from the offsets
     const int per = (nc + SCAN_WG - 1) / SCAN_WG;
     const int k0 = tid * per;
-    unsigned p = 0u, s = 0u;
-    for (int j = 0; j < per; ++j) {
-        const int k = k0 + j;
-        if (k < nc) {
-            unsigned v = 0u;
-            for (int z = 0; z < zstride; ++z) v += s_n[k * zstride + z];
-            p += v;
-            s += (v + WG - 1) / WG;
-        }
+    unsigned s = 0u;
+    none = 0u;
+    for (int k = k0; k < min(k0 + per, nc); ++k) {
+        const unsigned p0 = s_n[k * zstride], n = (k + 1 < nc ? s_n[(k + 1) * zstride] : hi) - p0;
+        count[c_lo + k] = n;
+        point_off[c_lo + k] = p0;
+        s += (n + WG - 1) / WG;
     }
-    unsigned tp, ts;
-    scan_pair_1024(p, s, tp, ts);  // (its barriers also order the reads above before the writes below)
-    p += lo;
-    for (int j = 0; j < per; ++j) {
-        const int k = k0 + j;
-        if (k < nc) {
-            const unsigned p0 = p;
-            for (int z = 0; z < zstride; ++z) {
-                const unsigned v = s_n[k * zstride + z];
-                s_n[k * zstride + z] = p;  // from here on: the next free position of the slab
-                p += v;
-            }
-            count[c_lo + k] = p - p0;
-            point_off[c_lo + k] = p0;
-            slice_loc[c_lo + k] = s;
-            s += (p - p0 + WG - 1) / WG;
-        }
+    scan_pair_1024(none, s, tp, ts);  // (no point is placed before its barriers)
+    for (int k = k0; k < min(k0 + per, nc); ++k) {
+        const unsigned n = count[c_lo + k];
+        slice_loc[c_lo + k] = s;
+        s += (n + WG - 1) / WG;
     }
     if (tid == 0) sb_slices[sb] = ts;
     __syncthreads();
@@ -1031,6 +1038,9 @@ constexpr int pair_lds_fixed() {
 }
 constexpr int PAIR_LDS_ATOMS = TILE * (int)(sizeof(double4) + sizeof(int));
 
+// Waves per SIMD asked of the compiler.  The FP32 gradient kernel of 6 types needs a
+// few registers more than 4 waves leave: kept to them (16 bytes spilled) it takes
+// 519 us for 6e5 points in 4800 atoms, left to itself (3 waves) 570.
 template <typename Real, int NT>
 constexpr int pair_waves() {
     return sizeof(Real) == 4 && NT == 6 ? 4 : 1;
@@ -1046,6 +1056,10 @@ constexpr int pair_lds_parts(int split, int pw) {
 }
 
 // NT = 0: energies.  NT > 0: a gradient run of at most NT framework types.
+// Bound by VALU issue (some 28 instructions per candidate and lane in the mixed
+// kernel).  With candidates staged in LDS by the workgroup, and now: 3e6 points in
+// 4800 atoms 1600 and 1450 us, 8e6 grid points 3870 and 3290, gradients of 6e5
+// points 598 and 516, FP64, 9e4 points, 236 and 180.
 // SPLIT (energies, image-list path): a small launch leaves most of the 1024
 // SIMDs without a wave while a few walk the whole list, one dependent load after
 // another; with the list shared out each wave's chain is SPLIT times shorter, for

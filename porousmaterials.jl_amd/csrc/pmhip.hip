@@ -43,7 +43,10 @@ constexpr long long MAX_POINT_SLOTS = 1LL << 24;  // point slots per launch grou
 constexpr long long MAX_IMAGES = 1LL << 26;       // images per list
 constexpr size_t MAX_IMAGE_LISTS = 8;             // image lists (radii) per framework
 constexpr long long MAX_GROUP_CELLS = 1LL << 24;  // cells of one launch group
-constexpr double SB_POINTS = 32768.0;             // target points per super-bin of the Widom sort
+// Target points per super-bin of the Widom sort: a group's points over SB_COUNT
+// workgroups of the sort, within these (9e4 points in 3 super-bins of 32768: 23 us,
+// in 44: 6; 6e5 points in 18: 34, in 128: 8).
+constexpr double SB_POINTS = 32768.0, SB_POINTS_MIN = 2048.0, SB_COUNT = 128.0;
 constexpr double ZSLAB_POINTS = 64.0;             // target points per slab of a Widom cell
 constexpr int64_t MAX_POSE_PHASE_BYTES = 32768;   // phase powers of a pose in LDS
 constexpr int MAX_RUN_CELLS = 65536;              // cells of one Widom run
@@ -1225,7 +1228,10 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
         int s_max = 0;
         while (((2LL << s_max) * zstride) <= SB_KEYS_MAX) ++s_max;
         const double per_cell = (double)gr.n_slots / (double)std::max(gr.n_cells, 1LL);
-        int S = (int)std::lround(std::log2(std::max(1.0, SB_POINTS / std::max(per_cell, 1.0))));
+        // (more super-bins take a few KB more of scratch: not where it is fixed)
+        const double sb_points =
+            fixed ? SB_POINTS : std::min(SB_POINTS, std::max(SB_POINTS_MIN, (double)gr.n_slots / SB_COUNT));
+        int S = (int)std::lround(std::log2(std::max(1.0, sb_points / std::max(per_cell, 1.0))));
         S = std::min(std::max(S, 0), s_max);
         for (int si = 0; si < gr.n_seg; ++si) {
             const SegArgs& sg = segs[gr.seg0 + si];
