@@ -390,7 +390,10 @@ __device__ __attribute__((always_inline)) inline void gc_energy(const GcmcParams
         const double2* col = fg + tk;
         int base = 0;
         if (cells) {
-            // the atoms of each site's cell list; the others are beyond r_c
+            // the atoms of each site's cell list, the lists in step (their index
+            // loads wait together: Xe among 4320 atoms, 4.93 -> 4.45 us per move); the
+            // others are beyond r_c
+            int next[NE], end[NE];
 #pragma unroll
             for (int e = 0; e < NE; ++e) {
                 const double w0 = x[e].x - floor(x[e].x), w1 = x[e].y - floor(x[e].y), w2 = x[e].z - floor(x[e].z);
@@ -398,24 +401,32 @@ __device__ __attribute__((always_inline)) inline void gc_energy(const GcmcParams
                 const int c1 = min(p.n_cell[1] - 1, (int)(w1 * p.n_cell[1]));
                 const int c2 = min(p.n_cell[2] - 1, (int)(w2 * p.n_cell[2]));
                 const int cell = __builtin_amdgcn_readfirstlane(c0 + p.n_cell[0] * (c1 + p.n_cell[1] * c2));
-                const int end = p.cell_start[cell + 1];
-                for (int j = p.cell_start[cell] + tid; j < end; j += 4 * GC_WG) {
-                    double4 xs[4], at[4];
-                    double2 se[4];
-                    bool ok[4], near[4];
-                    double en[4];
+                next[e] = p.cell_start[cell];
+                end[e] = p.cell_start[cell + 1];
+            }
+            while (next[0] < end[0] || next[NE - 1] < end[NE - 1]) {
+                constexpr int Q = 4 * NE;
+                int at[Q];
+                double4 xs[Q], ys[Q];
+                double2 se[Q];
+                bool ok[Q], near[Q];
+                double en[Q];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        ok[q] = j + q * GC_WG < end;
-                        xs[q] = x[e];
-                        at[q] = atoms[p.cell_atoms[ok[q] ? j + q * GC_WG : j]];
-                    }
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) se[q] = col[(int)at[q].w * na];
-                    gc_pairs<4>(hot, xs, at, se, ok, en, near);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) add_host(q, e, en[q], near[q]);
+                for (int q = 0; q < Q; ++q) {
+                    const int e = q % NE, j = next[e] + tid + q / NE * GC_WG;
+                    ok[q] = j < end[e];
+                    at[q] = p.cell_atoms[ok[q] ? j : 0];
+                    xs[q] = x[e];
                 }
+#pragma unroll
+                for (int q = 0; q < Q; ++q) ys[q] = atoms[at[q]];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) se[q] = col[(int)ys[q].w * na];
+                gc_pairs<Q>(hot, xs, ys, se, ok, en, near);
+#pragma unroll
+                for (int q = 0; q < Q; ++q) add_host(q, q % NE, en[q], near[q]);
+#pragma unroll
+                for (int e = 0; e < NE; ++e) next[e] += 4 * GC_WG;
             }
             base = n_atoms;
         }
