@@ -1257,7 +1257,7 @@ __device__ inline FourierPoint fourier_point(const GroupArgs& g, const SegArgs& 
 // c_mc, s_mc = cos, sin(2 pi mc u_c), Uc, Us, Vc, Vs complex.  Stream, row by row
 // of (ma, mb >= 0): Uc, Vc of mc = 0 (4 doubles), then Uc, Us, Vc, Vs of mc = 1
 // .. hi (8 doubles each); frows: per row the stream offset and hi (-1: empty row).
-constexpr int FOLD_HEAD = 4, FOLD_CELL = 8, FOLD_PAD = 16;
+constexpr int FOLD_HEAD = 4, FOLD_CELL = 8, FOLD_PAD = 32;
 
 __global__ void fold_box_kernel(const double2* box, int Ma, int Mb, int Mc, const int2* frows, double* fold) {
     const long long n = (long long)(Ma + 1) * (Mb + 1) * (Mc + 1);
@@ -1291,7 +1291,7 @@ __global__ void fold_box_kernel(const double2* box, int Ma, int Mb, int Mc, cons
 
 // f(0), f(1), ... as compile-time constants while it returns true
 template <typename F, int... I>
-__device__ __attribute__((always_inline)) inline void while_each(F& f, std::integer_sequence<int, I...>) {
+__device__ __attribute__((always_inline)) inline void while_each(const F& f, std::integer_sequence<int, I...>) {
     (void)(f(std::integral_constant<int, I>{}) && ...);
 }
 
@@ -1311,54 +1311,81 @@ __device__ __attribute__((always_inline)) inline void fourier_row(const gconst_p
         Vi[k] = co[3];
     }
     gconst_ptr<double> e = co + FOLD_HEAD;
-    double w[FOLD_CELL];  // the next cell (past the row's end: the next row's or the padding)
+    constexpr int PAIR = 2 * FOLD_CELL;
+    double v[PAIR], w[PAIR];  // two cells, and the next two (past the row's end: the next row's or the padding)
 #pragma unroll
-    for (int d = 0; d < FOLD_CELL; ++d) w[d] = e[d];
-    auto cell = [&](const double (&cm)[FOURIER_PTS], const double (&sm)[FOURIER_PTS]) {
-        double v[FOLD_CELL];
-#pragma unroll
-        for (int d = 0; d < FOLD_CELL; ++d) v[d] = w[d];
-        e += FOLD_CELL;
-#pragma unroll
-        for (int d = 0; d < FOLD_CELL; ++d) w[d] = e[d];
+    for (int d = 0; d < PAIR; ++d) w[d] = e[d];
+    const auto cell = [&](const double* c, const double (&cm)[FOURIER_PTS], const double (&sm)[FOURIER_PTS]) {
 #pragma unroll
         for (int k = 0; k < FOURIER_PTS; ++k) {
-            Ur[k] = fma(v[2], sm[k], fma(v[0], cm[k], Ur[k]));
-            Ui[k] = fma(v[3], sm[k], fma(v[1], cm[k], Ui[k]));
+            Ur[k] = fma(c[2], sm[k], fma(c[0], cm[k], Ur[k]));
+            Ui[k] = fma(c[3], sm[k], fma(c[1], cm[k], Ui[k]));
             if constexpr (V) {
-                Vr[k] = fma(v[6], sm[k], fma(v[4], cm[k], Vr[k]));
-                Vi[k] = fma(v[7], sm[k], fma(v[5], cm[k], Vi[k]));
+                Vr[k] = fma(c[6], sm[k], fma(c[4], cm[k], Vr[k]));
+                Vi[k] = fma(c[7], sm[k], fma(c[5], cm[k], Vi[k]));
             }
         }
-        // used here, so that the load of the next cell is issued before this one's FMAs
-        asm volatile("" ::"s"(w[0]), "s"(w[1]), "s"(w[2]), "s"(w[3]), "s"(w[4]), "s"(w[5]), "s"(w[6]), "s"(w[7]));
     };
+    const auto advance = [&]() {
+        e += PAIR;
+#pragma unroll
+        for (int d = 0; d < PAIR; ++d) {
+            v[d] = w[d];
+            w[d] = e[d];
+        }
+    };
+    // the next two cells used between the first and the second: their loads are
+    // issued before the first one's FMAs, and the wait comes once per two cells
+    const auto hold = [&]() {
+#pragma unroll
+        for (int d = 0; d < PAIR; d += 8)
+            asm volatile("" ::"s"(w[d]), "s"(w[d + 1]), "s"(w[d + 2]), "s"(w[d + 3]), "s"(w[d + 4]), "s"(w[d + 5]),
+                         "s"(w[d + 6]), "s"(w[d + 7]));
+    };
+    double cm[FOURIER_PTS], sm[FOURIER_PTS];
     if constexpr (MC > 0) {
         // (unrolled by the pack: the basis stays in registers)
-        auto step = [&](auto mi) {
-            constexpr int m = decltype(mi)::value + 1;
-            if (m > hi) return false;
-            double cm[FOURIER_PTS], sm[FOURIER_PTS];
+        const auto pick = [&](auto mi) {
+            constexpr int m = decltype(mi)::value;
 #pragma unroll
             for (int k = 0; k < FOURIER_PTS; ++k) {
                 cm[k] = cc[k][m];
                 sm[k] = sc[k][m];
             }
-            cell(cm, sm);
+        };
+        const auto step = [&](auto ci) {
+            constexpr int m = 2 * decltype(ci)::value + 1;
+            if (m > hi) return false;
+            advance();
+            pick(std::integral_constant<int, m>{});
+            cell(v, cm, sm);
+            hold();
+            if constexpr (m < MC) {
+                if (m + 1 > hi) return false;
+                pick(std::integral_constant<int, m + 1>{});
+                cell(v + FOLD_CELL, cm, sm);
+            }
             return true;
         };
-        while_each(step, std::make_integer_sequence<int, MC>{});
+        while_each(step, std::make_integer_sequence<int, (MC + 1) / 2>{});
     } else {
-        double cm[FOURIER_PTS], sm[FOURIER_PTS];
 #pragma unroll
         for (int k = 0; k < FOURIER_PTS; ++k) {
             cm[k] = cc[k][1];
             sm[k] = sc[k][1];
         }
-        for (int m = 1; m <= hi; ++m) {
-            cell(cm, sm);
+        const auto rotate = [&]() {
 #pragma unroll
             for (int k = 0; k < FOURIER_PTS; ++k) rotate_phase(cm[k], sm[k], cc[k][1], sc[k][1]);
+        };
+        for (int m = 1; m <= hi; m += 2) {
+            advance();
+            cell(v, cm, sm);
+            rotate();
+            hold();
+            if (m == hi) break;
+            cell(v + FOLD_CELL, cm, sm);
+            rotate();
         }
     }
 #pragma unroll
@@ -1376,12 +1403,13 @@ __device__ __attribute__((always_inline)) inline void fourier_row(const gconst_p
 // fractional), FP64, from the folded coefficients: two FMAs per kept k-vector
 // and point, where complex Horner steps took four.  The coefficients are the same
 // for every lane: they are read by scalar loads (through the scalar cache, into
-// SGPR operands of the FMAs), a cell ahead of their use.  The cosines and sines
+// SGPR operands of the FMAs), two cells at a time ahead of their use.  The cosines and sines
 // of the c axis are held in registers (MC >= the runs' Mc) or, MC = 0, stepped
 // along each row by the same recurrence, with the same bits.  Bound by FP64
 // issue: of some 3700 instructions per wave (461 k-vectors, 128 points) half are
 // these FMAs, a quarter the 33 rows' own, a quarter the phases.  3e6 points, 461
-// k-vectors: 379 -> 212 us; 48 screening runs: 424 -> 297.  Point slots of a
+// k-vectors: 379 -> 192 us (206 with loads one cell ahead); 48 screening runs,
+// whose coefficients exceed the scalar cache: 424 -> 230 (297).  Point slots of a
 // segment start at a multiple of WG, so a workgroup lies in one segment.
 template <int MC>
 __global__ __launch_bounds__(FOURIER_WG) void point_fourier_kernel(GroupArgs g) {

@@ -1031,8 +1031,9 @@ void pair_launch_grad(const GroupArgs& g, int n_wg, size_t shm, int extra_off, i
 
 // The Fourier kernel by the group's largest third index: the smallest that holds
 // it, whose registers (66 + 8 per index) allow the most waves per SIMD; past 12
-// (3 waves) the one that steps the phases along each row.  Held and stepped: 3e6
-// points of index 5 206 and 292 us, 48 runs of index up to 10 297 and 316.
+// (3 waves) the one that steps the phases along each row.  Held and stepped, with
+// loads one cell ahead: 3e6 points of index 5 206 and 292 us, 48 runs of index up
+// to 10 297 and 316.
 template <int MC>
 void fourier_launch_t(const GroupArgs& g, unsigned n_wg) {
     hipLaunchKernelGGL(point_fourier_kernel<MC>, dim3(n_wg), dim3(FOURIER_WG), 0, g_ctx.stream, g);
