@@ -65,7 +65,7 @@ struct RunArgs {
     double chunk_r;          // bound on |point - chunk centre| (Cartesian)
     double inv4pe;
     int esm;                 // 0 no electrostatics, 1 LJ and Ewald share r_c, 2 separate cutoffs
-    int fast;                // the image list covers r_cmax + chunk_r around every chunk
+    int fast;                // the image list serves the run (chunk_r within the limit)
     int nsite, n_types, n_img, n_atoms, n_tiles;
     unsigned site_lj_mask, site_q_mask;
     const double4* img;      // images near the box, in spatial tiles: Cartesian xyz (A), and the charge (FP64 runs)
@@ -1004,6 +1004,8 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                 for (int gi = 0; gi < nt; gi += 64) {
                     PairSums<Real> S;
                     const int ge = min(nt, gi + 64);
+                    // (two atoms' latencies overlap: 4845 points, 4896 atoms, 736 -> 546 us)
+#pragma unroll 2
                     for (int j = gi; j < ge; ++j) {
                         const double4 at = L.c[j];
                         double ex = at.x - px, ey = at.y - py, ez = at.z - pz;
@@ -1014,8 +1016,12 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                         const double cy = f22 * ey + f23 * ez;
                         const double cz = f33 * ez;
                         const double r2 = cx * cx + cy * cy + cz * cz;
-                        const int tt = __builtin_amdgcn_readfirstlane(L.t[j]);
-                        if constexpr (GRAD) ts.type(tt, nsite, s_gc[tt + site], S, is_lj);
+                        // (energies: the type stays in a vector register, a wait less per atom)
+                        int tt = L.t[j];
+                        if constexpr (GRAD) {
+                            tt = __builtin_amdgcn_readfirstlane(tt);
+                            ts.type(tt, nsite, s_gc[tt + site], S, is_lj);
+                        }
                         pair_term<ESM, Real, GRAD, true>(r2, at.w, (float)at.w, s_lj[tt + site], is_lj, r2lj, r2sr, et,
                                                          ovl, S);
                     }
