@@ -1043,6 +1043,13 @@ constexpr int pair_lds_fixed() {
     return sizeof(Real) == 4 ? ERFC_TAB * (int)sizeof(float4) : ERFC64_TAB * (int)sizeof(double2);
 }
 constexpr int PAIR_LDS_ATOMS = TILE * (int)(sizeof(double4) + sizeof(int));
+// bytes of an LJ table of n_tab entries (8 or 16 each), up to the fold constants
+// after it; both sides take it from here: with an entry counted too many the
+// constants of the last type ran into the all-atoms path's first atom
+template <typename Real>
+__host__ __device__ constexpr int pair_lds_lj(int n_tab) {
+    return (n_tab * (int)sizeof(LJC<Real>) + 15) / 16 * 16;
+}
 
 // Waves per SIMD asked of the compiler.  The FP32 gradient kernel of 6 types needs a
 // few registers more than 4 waves leave: kept to them (16 bytes spilled) it takes
@@ -1104,8 +1111,8 @@ __global__ __launch_bounds__(pair_wg(SPLIT, PW), (pair_waves<Real, NT>())) void 
     }
     const SegArgs sg = g.segs[si];
     const RunArgs& a = g.runs[sg.run];
-    // (16-byte aligned: the LJ table's entries are 8 or 16 bytes)
-    double2* s_gc = reinterpret_cast<double2*>(s_lj + ((a.n_types * a.nsite + 1) & ~1));
+    const int n_tab = a.n_types * a.nsite;
+    double2* s_gc = reinterpret_cast<double2*>(smem + pair_lds_fixed<Real>() + pair_lds_lj<Real>(n_tab));
 
     bool valid;
     long long pid;
@@ -1137,7 +1144,6 @@ __global__ __launch_bounds__(pair_wg(SPLIT, PW), (pair_waves<Real, NT>())) void 
         pz = grid_coord(k, n3, a.repd[2]);
         site = 0;
     }
-    const int n_tab = a.n_types * a.nsite;
     const LJC<Real>* gtab = reinterpret_cast<const LJC<Real>*>(a.ljtab);
     for (int t = tid; t < n_tab; t += NTH) s_lj[t] = gtab[t];
     if constexpr (GRAD) {

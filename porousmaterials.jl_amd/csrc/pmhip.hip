@@ -1257,7 +1257,9 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
         else build_ljtab<float>(r.fw, r.ff, r.ns, r.pr->site, r.pr->lj_species, r.tab);
         r.tab_off = tab_total;
         tab_total += align256(r.tab.size());
-        lj_lds = std::max(lj_lds, (r.tab.size() + 15) / 16 * 16 + (grad ? r.gtab.size() : 0));
+        const int n_tab = std::max((int)r.fw->species_global.size(), 1) * r.ns;
+        lj_lds = std::max(lj_lds, (size_t)(fp64 ? pair_lds_lj<double>(n_tab) : pair_lds_lj<float>(n_tab)) +
+                                      (grad ? r.gtab.size() : 0));
         if (grad) {
             r.gtab_off = tab_total;
             tab_total += align256(r.gtab.size());
