@@ -49,6 +49,7 @@ constexpr long long MAX_GROUP_CELLS = 1LL << 24;  // cells of one launch group
 constexpr double SB_POINTS = 32768.0, SB_POINTS_MIN = 2048.0, SB_COUNT = 128.0;
 constexpr double ZSLAB_POINTS = 64.0;             // target points per slab of a Widom cell
 constexpr int64_t MAX_POSE_PHASE_BYTES = 32768;   // phase powers of a pose in LDS
+constexpr int64_t POSE_SLICE = 1LL << 23;         // poses per launch: a launch takes fewer than 2^32 work-items
 constexpr int MAX_RUN_CELLS = 65536;              // cells of one Widom run
 static_assert(MAX_POINT_SLOTS <= (long long)pmk::SB_SLOT_MASK + 1, "a super-bin slot fits below the copy bits");
 static_assert(MAX_GROUP_CELLS <= (long long)pmk::CELL_MASK + 1, "a group's cell index fits below the slab bits");
@@ -560,21 +561,24 @@ int run_poses(const pm_framework* fw, const pm_forcefield* ff, const pm_ewald* e
     double* d_out = reinterpret_cast<double*>(base + o_out);
     PM_HIP(hipMemcpyAsync(d_pose, site_xf, (size_t)n * a.ns * 3 * sizeof(double), hipMemcpyHostToDevice,
                           g_ctx.stream));
-    a.pose_xf = d_pose;
-    a.out_e = d_out;
-    a.out_g = out_grad ? reinterpret_cast<double*>(base + o_grad) : nullptr;
+    double* d_grad = out_grad ? reinterpret_cast<double*>(base + o_grad) : nullptr;
     const size_t shm = (size_t)pose_lds(es, table, a.nz, a.n_types, a.ns, fp64, out_grad != nullptr).bytes;
-    const int n_wg = (int)n;  // one workgroup per pose
     PM_HIP(hipEventRecord(g_ctx.ev0, g_ctx.stream));
-    const int rc = out_grad ? pose_launch<true>(a, n_wg, shm, fp64, es) : pose_launch<false>(a, n_wg, shm, fp64, es);
-    if (rc != PM_OK) return rc;
-    PM_HIP(hipGetLastError());
+    for (int64_t first = 0; first < n; first += POSE_SLICE) {
+        const int n_wg = (int)std::min(POSE_SLICE, n - first);  // one workgroup per pose
+        a.pose_xf = d_pose + first * a.ns * 3;
+        a.out_e = d_out + first * 3;
+        a.out_g = d_grad ? d_grad + first * a.ns * 3 : nullptr;
+        const int rc = out_grad ? pose_launch<true>(a, n_wg, shm, fp64, es) : pose_launch<false>(a, n_wg, shm, fp64, es);
+        if (rc != PM_OK) return rc;
+        PM_HIP(hipGetLastError());
+    }
     PM_HIP(hipEventRecord(g_ctx.ev1, g_ctx.stream));
     out3.resize((size_t)n * 3);
     PM_HIP(hipMemcpyAsync(out3.data(), d_out, (size_t)n * 3 * sizeof(double), hipMemcpyDeviceToHost,
                           g_ctx.stream));
     if (out_grad)
-        PM_HIP(hipMemcpyAsync(out_grad, a.out_g, (size_t)n * a.ns * 3 * sizeof(double), hipMemcpyDeviceToHost,
+        PM_HIP(hipMemcpyAsync(out_grad, d_grad, (size_t)n * a.ns * 3 * sizeof(double), hipMemcpyDeviceToHost,
                               g_ctx.stream));
     return finish_timing((double)n * a.ns * fw->n_rep);
 }
