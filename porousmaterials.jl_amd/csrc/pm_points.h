@@ -1063,9 +1063,9 @@ constexpr int pair_waves() {
 // share out the image list.
 constexpr int pair_wg(int split, int pw) { return 64 * split * pw; }
 // LDS of the SPLIT kernels for the parts' LJ and real-space sums [part][point]
-// and the waves' overlap masks.
+// the candidate counts of each 64 points and the waves' overlap masks.
 constexpr int pair_lds_parts(int split, int pw) {
-    return split > 1 ? (2 * LIST_PARTS * 64 + split) * pw * (int)sizeof(double) : 0;
+    return split > 1 ? (2 * LIST_PARTS * 64 + 1 + split) * pw * (int)sizeof(double) : 0;
 }
 
 // NT = 0: energies.  NT > 0: a gradient run of at most NT framework types.
@@ -1076,8 +1076,8 @@ constexpr int pair_lds_parts(int split, int pw) {
 // SPLIT (energies, image-list path): a small launch leaves most of the 1024
 // SIMDs without a wave while a few walk the whole list, one dependent load after
 // another; with the list shared out each wave's chain is SPLIT times shorter, for
-// SPLIT times the tile tests (1000 CH4 insertions, 424 atoms: 70 -> 28 us; 1000
-// CO2, 600 atoms: 182 -> 55, in FP64 252 -> 80; 20000: 138 -> 94).  More points per
+// SPLIT times the tile tests (1000 CH4 insertions, 424 atoms: 75 -> 26 us; 1000
+// CO2, 600 atoms: 187 -> 53, in FP64 257 -> 71; 20000: 133 -> 92).  More points per
 // workgroup (PW) share a load of the tables.
 template <typename Real, int NT, int SPLIT, int PW>
 __global__ __launch_bounds__(pair_wg(SPLIT, PW), (pair_waves<Real, NT>())) void point_pair_kernel(GroupArgs g, int extra_off) {
@@ -1098,8 +1098,13 @@ __global__ __launch_bounds__(pair_wg(SPLIT, PW), (pair_waves<Real, NT>())) void 
     L.t = reinterpret_cast<int*>(L.c + TILE);
 
     const int tid = threadIdx.x;
-    const unsigned wg = blockIdx.x / SUB;                                            // slice or brick
-    const int pt = (int)(blockIdx.x % SUB) * NP + (tid & (NP - 1));                  // point of it
+    // the slice or brick, and its point.  The first NP points of every slice come
+    // first: a sparse run's slices have no others, and in order of slices its points
+    // would all go to every SUB-th workgroup, that is to 8 / SUB of the 8 XCDs (993
+    // slices of 5 points, 4 waves each: 112 -> 49 us)
+    const unsigned n_wg = gridDim.x / SUB, sub = SUB > 1 ? blockIdx.x / n_wg : 0u;
+    const unsigned wg = blockIdx.x - sub * n_wg;
+    const int pt = (int)sub * NP + (tid & (NP - 1));
     int si;
     uint4 it = make_uint4(0u, 0u, 0u, 0u);
     if (g.mode == MODE_WIDOM) {
@@ -1157,7 +1162,7 @@ __global__ __launch_bounds__(pair_wg(SPLIT, PW), (pair_waves<Real, NT>())) void 
         if (a.esm != 0)
             for (int t = tid; t < ERFC64_TAB; t += NTH) s_erfc64[t] = a.erfc64_tab[t];
     if constexpr (SPLIT > 1)
-        for (int t = tid; t < 2 * LIST_PARTS * NP; t += NTH) L.part[t] = 0.0;
+        for (int t = tid; t < 2 * LIST_PARTS * NP + PW; t += NTH) L.part[t] = 0.0;  // (and the counts)
     __syncthreads();
 
     double acc_lj = 0.0, acc_sr = 0.0;
@@ -1173,18 +1178,27 @@ __global__ __launch_bounds__(pair_wg(SPLIT, PW), (pair_waves<Real, NT>())) void 
     else
         chunk_pairs<2, Real, NT, SPLIT, PW>(a, valid, px, py, pz, site, s_lj, s_gc, L, acc_lj, acc_sr, ovl,
                                  n_cand, ts);
-    if (g.cand_pairs != nullptr) {
+    const bool counts = g.cand_pairs != nullptr;
+    if (SPLIT == 1 && counts) {
         const unsigned long long m = __ballot(valid);
         if ((tid & 63) == 0 && m != 0ull)
             atomicAdd(g.cand_pairs, (unsigned long long)__popcll(m) * n_cand);
     }
     if constexpr (SPLIT > 1) {
-        // a wave per 64 points adds up the parts' sums, in the order of the list
-        unsigned long long* const s_ovl = reinterpret_cast<unsigned long long*>(L.part + 2 * LIST_PARTS * NP);
+        // a wave per 64 points adds up the parts' sums, in the order of the list; the
+        // waves' candidates are counted by one atomic for them all (one for each wave:
+        // 469 groups of 16 waves 128 us instead of 92)
+        unsigned long long* const s_cand = reinterpret_cast<unsigned long long*>(L.part + 2 * LIST_PARTS * NP);
+        unsigned long long* const s_ovl = s_cand + PW;
         const unsigned long long om = __ballot(ovl);
-        if ((tid & 63) == 0) s_ovl[tid >> 6] = om;
+        if ((tid & 63) == 0) {
+            s_ovl[tid >> 6] = om;
+            atomicAdd(&s_cand[(tid >> 6) & (PW - 1)], n_cand);
+        }
         __syncthreads();
         if (tid >= NP) return;
+        if (const unsigned long long m = __ballot(valid); counts && (tid & 63) == 0 && m != 0ull)
+            atomicAdd(g.cand_pairs, (unsigned long long)__popcll(m) * s_cand[tid >> 6]);
         unsigned long long any = 0ull;
         for (int w = 0; w < SPLIT; ++w) any |= s_ovl[w * PW + (tid >> 6)];
         ovl = (any >> (tid & 63)) & 1ull;

@@ -869,7 +869,7 @@ struct PointRun {
     bool es = false;
     int ns = 0;
     int64_t n_wg = 0;      // Widom: insertion workgroups; grid: bricks
-    int64_t n_points = 0;  // grid points (grid runs)
+    int64_t n_points = 0;  // grid points, or a Widom run's sites of every insertion
     int64_t n_cells = 0;   // Widom cells
     double cost = 0.0;     // scheduling estimate per point
     double* host_out = nullptr;
@@ -930,6 +930,7 @@ int widom_prepare(const pm_widom_run& in, PointRun& r) {
     const double pts = std::min((double)in.n_blocks * (double)in.n_per_block * ns, (double)MAX_POINT_SLOTS);
     choose_cells(fw, pts, a.ncell, &a.chunk_r, &a.zbins);
     r.n_cells = (int64_t)a.ncell[0] * a.ncell[1] * a.ncell[2];
+    r.n_points = in.n_blocks * in.n_per_block * ns;
     const double vol = std::fabs(fw->F[0] * fw->F[4] * fw->F[8]);
     r.cost = (double)fw->n_rep / vol * std::pow(a.r_cmax + a.chunk_r, 3);
     return PM_OK;
@@ -996,16 +997,27 @@ void pair_launch_t(const GroupArgs& g, int n_wg, size_t shm, int extra_off) {
                        shm + pair_lds_parts(SPLIT, PW), g_ctx.stream, g, extra_off);
 }
 
-// Waves that share out the image list of each 64 points, by the 64-point waves of
-// the launch (pair kernel, us: one wave; 2 in workgroups of 256 points; 8 of 128; 16
-// of 64).  CO2 in 600 atoms: 141 waves 196, 127, 83, 62; 469 waves 148, 98, 74, 128;
-// 937 waves 138, 94, 123, 230; 1406 waves 143, 116, 173, 340; 2812 waves 167, 168,
-// 316, 648; in FP64, 937 waves 192, 137, 158, 262; 1406 waves 209, 222, 217, 369.
-// CH4 in 600 atoms: 156 waves 158, 99, 68, 54; 469 waves 122, 81, 69, 121; 1562 waves
-// 122, 93, 204, 363.  CH4 grids: 216 waves 52, 36, 31, 55; 512 waves 49, 36, 60, 112;
-// 1000 waves 51, 47, 107, 209; 2548 waves 65, 87, 227, 449.
-int pair_split(long long n_waves, bool fp64) {
-    return n_waves < 160 ? 16 : n_waves < 640 ? 8 : n_waves < (fp64 ? 1024 : 1792) ? 2 : 1;
+// Waves that share out the image list of each 64 points: 16 in workgroups of 64
+// points, 8 of 128, 2 of 256, 4 of 64 or one.  By the launch's point slots, its cells,
+// and the cells expected to hold a point (a grid: none); the fewer workgroups have
+// points, the more waves each takes.  Pair kernel, us, one wave, 2, 8, 16.  CO2 in 600 atoms:
+// 156 waves of 64 points 181, 125, 77, 55; 468 waves 148, 104, 69, 96; 937 waves 133,
+// 99, 116, 177; 1406 waves 138, 111, 152, 241; 2343 waves 158, 158, 224, 372; in FP64,
+// 937 waves 185, 132, 154, 251; 1406 waves 200, 207, 202, 348.  CH4 grids: 216 waves
+// 54, 36, 26, 25; 512 waves 50, 35, 27, 43; 1000 waves 51, 38, 45, 76; 2548 waves 64,
+// 63, 94, 169.
+// In a large unit cell a run's cells stay small (the 6 A of the candidate sphere) and
+// hold few points each; a workgroup then has one wave of points whatever its size, and
+// workgroups without points cost the launch time.  CH4, one wave, 4, 8, 16: 80 of 216
+// cells 54, 36, 28, 30; 214 of 216 71, 44, 34, 35; 99 of 6859 40, 28, 35, 54; 544 of
+// 729 73, 40, 75, 72; 993 of 1000 74, 49, 120, 123; 2608 of 3375 68, 73, 237, 259; in
+// FP64, 993 of 1000 84, 73, 142, 143; 2608 of 3375 102, 113, 275, 293.  More cells than
+// measured (a batch) would also reach the launch limit of 2^32 work-items.
+int pair_split(double slots, double n_cells, double occupied, bool fp64) {
+    if (std::max(slots / 64.0, n_cells) < 160.0) return 16;
+    if (std::max(slots / 128.0, n_cells) < 320.0) return 8;
+    if (std::max(slots / 256.0, n_cells) < (fp64 ? 256.0 : 448.0)) return 2;
+    return occupied > slots / 64.0 && occupied < 1536.0 && n_cells < 65536.0 ? 4 : 1;
 }
 
 template <typename Real>
@@ -1013,6 +1025,7 @@ void pair_launch_plain(const GroupArgs& g, int n_wg, size_t shm, int extra_off, 
     switch (split) {
         case 16: pair_launch_t<Real, 0, 16, 1>(g, n_wg, shm, extra_off); break;
         case 8: pair_launch_t<Real, 0, 8, 2>(g, n_wg, shm, extra_off); break;
+        case 4: pair_launch_t<Real, 0, 4, 1>(g, n_wg, shm, extra_off); break;
         case 2: pair_launch_t<Real, 0, 2, 4>(g, n_wg, shm, extra_off); break;
         default: pair_launch_t<Real, 0>(g, n_wg, shm, extra_off); break;
     }
@@ -1160,6 +1173,7 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
         int n_seg = 0;
         long long n_wg = 0, n_slots = 0, n_cells = 0;
         long long n_gen = 0;  // Widom: generator workgroups (GEN_CHUNKS insertion workgroups each)
+        double occupied = 0.0;  // Widom: cells expected to hold a point
         bool es = false;
         int sb_shift = 0;    // Widom: super-bins of 2^sb_shift cells
         int zstride = 1;     // Widom: the sort's slabs per cell (the largest of the group's runs)
@@ -1199,6 +1213,8 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
                 cur.n_gen += (take + GEN_CHUNKS - 1) / GEN_CHUNKS;
                 cur.n_slots += take * per_wg;
                 cur.n_cells += r.n_cells;
+                const double points = (double)r.n_points * (double)take / (double)r.n_wg, cells = (double)r.n_cells;
+                cur.occupied += cells * (1.0 - std::exp(-points / cells));
                 cur.es = cur.es || r.es;
                 w += take;
             }
@@ -1456,9 +1472,10 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
         } else {
             // (a run on the all-atoms path is not split, nor one whose tables leave too
             // little LDS)
-            const long long n_waves = (widom ? gr.n_slots : gr.n_wg * WG) / 64;
             const bool can_split = all_fast && shm + pair_lds_parts(2, 4) <= g_ctx.max_lds;
-            const int split = can_split ? pair_split(n_waves, fp64) : 1;
+            const int split = !can_split ? 1
+                              : widom    ? pair_split((double)gr.n_slots, (double)gr.n_cells, gr.occupied, fp64)
+                                         : pair_split((double)(gr.n_wg * WG), 0.0, 0.0, fp64);
             if (fp64) pair_launch_plain<double>(g, (int)pair_wg, shm, extra_off, split);
             else pair_launch_plain<float>(g, (int)pair_wg, shm, extra_off, split);
         }
