@@ -997,27 +997,36 @@ void pair_launch_t(const GroupArgs& g, int n_wg, size_t shm, int extra_off) {
                        shm + pair_lds_parts(SPLIT, PW), g_ctx.stream, g, extra_off);
 }
 
+// What a launch's pair workgroups hold.  A grid has slots alone.
+struct PairLoad {
+    double slots = 0.0, cells = 0.0;
+    double points = 0.0;    // Widom: the points of the slots
+    double occupied = 0.0;  // cells expected to hold a point
+    double work = 0.0, longest = 0.0;  // candidates of all groups of 64 points, and the most of one of them
+};
+
 // Waves that share out the image list of each 64 points: 16 in workgroups of 64
-// points, 8 of 128, 2 of 256, 4 of 64 or one.  By the launch's point slots, its cells,
-// and the cells expected to hold a point (a grid: none); the fewer workgroups have
-// points, the more waves each takes.  Pair kernel, us, one wave, 2, 8, 16.  CO2 in 600 atoms:
-// 156 waves of 64 points 181, 125, 77, 55; 468 waves 148, 104, 69, 96; 937 waves 133,
-// 99, 116, 177; 1406 waves 138, 111, 152, 241; 2343 waves 158, 158, 224, 372; in FP64,
-// 937 waves 185, 132, 154, 251; 1406 waves 200, 207, 202, 348.  CH4 grids: 216 waves
-// 54, 36, 26, 25; 512 waves 50, 35, 27, 43; 1000 waves 51, 38, 45, 76; 2548 waves 64,
-// 63, 94, 169.
-// In a large unit cell a run's cells stay small (the 6 A of the candidate sphere) and
-// hold few points each; a workgroup then has one wave of points whatever its size, and
-// workgroups without points cost the launch time.  CH4, one wave, 4, 8, 16: 80 of 216
-// cells 54, 36, 28, 30; 214 of 216 71, 44, 34, 35; 99 of 6859 40, 28, 35, 54; 544 of
-// 729 73, 40, 75, 72; 993 of 1000 74, 49, 120, 123; 2608 of 3375 68, 73, 237, 259; in
-// FP64, 993 of 1000 84, 73, 142, 143; 2608 of 3375 102, 113, 275, 293.  More cells than
-// measured (a batch) would also reach the launch limit of 2^32 work-items.
-int pair_split(double slots, double n_cells, double occupied, bool fp64) {
-    if (std::max(slots / 64.0, n_cells) < 160.0) return 16;
-    if (std::max(slots / 128.0, n_cells) < 320.0) return 8;
-    if (std::max(slots / 256.0, n_cells) < (fp64 ? 256.0 : 448.0)) return 2;
-    return occupied > slots / 64.0 && occupied < 1536.0 && n_cells < 65536.0 ? 4 : 1;
+// points, 8 of 128, 2 of 256, 4 of 64 or one.  The fewer workgroups have points, the
+// more waves each takes.  Pair kernel, us, one wave, 2, 8, 16.  CO2 in 600 atoms: 156
+// waves of 64 points 181, 125, 77, 55; 468 waves 148, 104, 69, 96; 937 waves 133, 99,
+// 116, 177; 1406 waves 138, 111, 152, 241; 2343 waves 158, 158, 224, 372; in FP64, 937
+// waves 185, 132, 154, 251; 1406 waves 200, 207, 202, 348.  CH4 grids: 216 waves 54,
+// 36, 26, 25; 512 waves 50, 35, 27, 43; 1000 waves 51, 38, 45, 76; 2548 waves 64, 63,
+// 94, 169.
+// In a large unit cell, or a batch, a run's cells stay small (the 6 A of the candidate
+// sphere) and hold few points each; a workgroup then has one wave of points whatever
+// its size, and those without any cost the launch time.  One wave takes as long as its
+// candidates; if that is most of the launch, 4 waves share them.  CH4, one wave, 4, 8,
+// 16: 80 of 216 cells occupied 54, 36, 28, 30; 214 of 216 71, 44, 34, 35; 99 of 6859
+// 40, 28, 35, 54; 544 of 729 73, 40, 75, 72; 993 of 1000 74, 49, 120, 123; 2608 of
+// 3375 68, 73, 237, 259; in FP64, 993 of 1000 84, 73, 142, 143; 2608 of 3375 102, 113,
+// 275, 293; 64 frameworks of 5 x 100 insertions, 6900 of 6974 469, 220, 336, 371.
+// More cells than measured would also reach the launch limit of 2^32 work-items.
+int pair_split(const PairLoad& l, bool fp64) {
+    if (std::max(l.slots / 64.0, l.cells) < 160.0) return 16;
+    if (std::max(l.slots / 128.0, l.cells) < 320.0) return 8;
+    if (l.occupied > 0.5 * l.points / 64.0 && l.work < 1.75 * 1024.0 * l.longest && l.cells < 65536.0) return 4;
+    return std::max(l.slots / 256.0, l.cells) < (fp64 ? 256.0 : 448.0) ? 2 : 1;
 }
 
 template <typename Real>
@@ -1173,7 +1182,7 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
         int n_seg = 0;
         long long n_wg = 0, n_slots = 0, n_cells = 0;
         long long n_gen = 0;  // Widom: generator workgroups (GEN_CHUNKS insertion workgroups each)
-        double occupied = 0.0;  // Widom: cells expected to hold a point
+        PairLoad load;
         bool es = false;
         int sb_shift = 0;    // Widom: super-bins of 2^sb_shift cells
         int zstride = 1;     // Widom: the sort's slabs per cell (the largest of the group's runs)
@@ -1213,8 +1222,12 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
                 cur.n_gen += (take + GEN_CHUNKS - 1) / GEN_CHUNKS;
                 cur.n_slots += take * per_wg;
                 cur.n_cells += r.n_cells;
-                const double points = (double)r.n_points * (double)take / (double)r.n_wg, cells = (double)r.n_cells;
-                cur.occupied += cells * (1.0 - std::exp(-points / cells));
+                const double points = (double)r.n_points * (double)take / (double)r.n_wg, cells = (double)r.n_cells,
+                             occupied = cells * (1.0 - std::exp(-points / cells));
+                cur.load.points += points;
+                cur.load.occupied += occupied;
+                cur.load.work += std::max(points / 64.0, occupied) * r.cost;
+                cur.load.longest = std::max(cur.load.longest, r.cost);
                 cur.es = cur.es || r.es;
                 w += take;
             }
@@ -1473,9 +1486,10 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
             // (a run on the all-atoms path is not split, nor one whose tables leave too
             // little LDS)
             const bool can_split = all_fast && shm + pair_lds_parts(2, 4) <= g_ctx.max_lds;
-            const int split = !can_split ? 1
-                              : widom    ? pair_split((double)gr.n_slots, (double)gr.n_cells, gr.occupied, fp64)
-                                         : pair_split((double)(gr.n_wg * WG), 0.0, 0.0, fp64);
+            PairLoad load = gr.load;
+            load.slots = (double)(widom ? gr.n_slots : gr.n_wg * WG);
+            load.cells = (double)gr.n_cells;
+            const int split = can_split ? pair_split(load, fp64) : 1;
             if (fp64) pair_launch_plain<double>(g, (int)pair_wg, shm, extra_off, split);
             else pair_launch_plain<float>(g, (int)pair_wg, shm, extra_off, split);
         }
