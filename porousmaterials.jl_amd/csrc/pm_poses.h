@@ -36,9 +36,11 @@ struct PoseArgs {
 // queued pairs per wave: fewer than 64, and 64 for every site of a round
 __host__ __device__ constexpr int pose_queue(int ns) { return 64 * (ns + 1); }
 
-// Whether a pose kernel reads the FP64 erfc table: FP64 energies, and forces.
+// Whether a pose kernel takes erfc in FP64: energies in FP64, and forces.  From the
+// table (its template argument TABLE) only where that is as exact as the function,
+// erfc64_table_exact().
 template <bool ES, typename Real, bool GRAD>
-constexpr bool pose_table() {
+constexpr bool pose_erfc64() {
     return ES && (sizeof(Real) == 8 || GRAD);
 }
 
@@ -92,17 +94,16 @@ __device__ inline double erfc_tab64(double r, double inv_h, const double2* tab) 
 // phases z_a^m, z_b^m, z_c^m of every site from LDS (one sincospi per site, axis
 // and power instead of one per site and k-vector).  4096 CO2 poses with forces,
 // FP64, 4800 atoms, 461 k-vectors: 521 us with every pair and k-vector evaluated
-// in full, one wave per pose; 108 us so.  Energies of 2048 poses: 191 -> 47 us
+// in full, one wave per pose; 105 us so.  Energies of 2048 poses: 191 -> 47 us
 // (Ewald), 59 -> 31 us (LJ).  Bound by instruction issue and the latency of the
 // queue's gathers at four waves per SIMD.
 //   LJ      d/dx_s = 6 eps4 (2u^2 - u) / r^2 * d,   u = (sigma^2 / r^2)^3
 //   real    d/dx_s = q_s q_a [erfc(a r) / r + 2a/sqrt(pi) e^{-a^2 r^2}] / r^2 * d / (4 pi eps0)
 //   Fourier d/dx_s = q_s 2 pi C^T sum_k (-A_re sin th + A_im cos th) (m o rep),  th = 2 pi m.(rep o x)
 // with d = x_atom - x_s (nearest image, Cartesian) and C the replicated box's c_to_f.
-template <int NS, bool ES, typename Real, bool GRAD>
+template <int NS, bool ES, typename Real, bool GRAD, bool TABLE>
 __global__ __launch_bounds__(WG) void pose_kernel(PoseArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr bool TABLE = pose_table<ES, Real, GRAD>();
     constexpr int NV = 3 + (GRAD ? 3 * NS : 0);  // sums per pose
     const PoseLds L = pose_lds(ES, TABLE, a.nz, a.n_types, NS, sizeof(Real) == 8, GRAD);
     double2* const s_tab = reinterpret_cast<double2*>(smem);
@@ -283,7 +284,12 @@ __global__ __launch_bounds__(WG) void pose_kernel(PoseArgs a) {
                 if constexpr (ES) {
                     const bool ins = (r2 < r2sr) & (p.w != 0.0);
                     double t = 0.0;  // erfc(alpha r) / r
-                    if constexpr (TABLE) t = y * erfc_tab64(ins ? r2 * y : 0.0, a.erfc64_inv_h, s_tab);
+                    if constexpr (TABLE) {
+                        t = y * erfc_tab64(ins ? r2 * y : 0.0, a.erfc64_inv_h, s_tab);
+                    } else if constexpr (pose_erfc64<ES, Real, GRAD>()) {
+                        const double r = sqrt(r2);
+                        t = erfc(alpha * r) / r;
+                    }
                     if constexpr (sizeof(Real) == 4)
                         acc_sr += ins ? x.w * (double)PairMath<float>::coul(r2, p.w, alpha) : 0.0;
                     else
