@@ -557,14 +557,15 @@ int run_poses(const pm_framework* fw, const pm_forcefield* ff, const pm_ewald* e
     }
     // FP32 squared distances below which a pair is looked at in FP64.  A distance
     // from FP32 fractional coordinates is off by a few 2^-24 of the box's edges.
-    // In a box narrower than the cutoff sphere the FP32 nearest image may be
-    // another one than the FP64 one: every pair is looked at.
+    // The FP32 nearest image is another one than the FP64 one only half a box away,
+    // within those roundings: in a box that is not wider than the cutoff sphere by
+    // more than them, or narrower, every pair is looked at.
     {
         const double r2 = std::max(a.r2_lj, a.r2_sr), rc = std::sqrt(r2);
         double edge = rc;
         for (int c = 0; c < 3; ++c) edge += std::fabs(fw->F[3 * c]) + std::fabs(fw->F[3 * c + 1]) + std::fabs(fw->F[3 * c + 2]);
         const double wide = std::min(fw->width[0], std::min(fw->width[1], fw->width[2]));
-        a.r2_keep = wide >= 2.0 * rc ? (float)(r2 + 4e-6 * rc * edge + 1e-9) : INFINITY;
+        a.r2_keep = wide >= 2.0 * rc * (1.0 + 1e-6) ? (float)(r2 + 4e-6 * rc * edge + 1e-9) : INFINITY;
     }
     size_t tab_bytes = 0;
     if (int rc = stage_ljtab(fw, ff, a.ns, a.site, site_species, precision, &tab_bytes)) return rc;
