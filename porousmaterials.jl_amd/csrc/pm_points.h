@@ -545,8 +545,8 @@ struct PairSums {
 // 3.0-3.7, v_rsq_f32 1.1, v_rsq_f64 0.6, and an LDS read takes the LDS as long
 // for 8 bytes as for 16 (0.58).  So:
 // - a pair outside the cutoff is masked once, through its 1/r (every masked
-//   term is then an exact zero and reads a valid table entry), not term by
-//   term; the overlap test is left to the caller, who follows the smallest r^2
+//   term is then an exact zero, or in FP64 real-space sums below 1e-313, which
+//   unmasked_sum takes out, and reads a valid table entry), not term by term; the overlap test is left to the caller, who follows the smallest r^2
 //   of a tile's candidates (tile_close) instead of comparing every pair;
 // - FP64: 1/r by v_rsq_f64 and one third-order step, y (1 + e/2 + 3 e^2/8) with
 //   e = 1 - r^2 y^2 (the estimate's 2^-22 cubes to below an ulp); index and
@@ -635,6 +635,14 @@ __device__ __attribute__((always_inline)) inline Real pair_term(double r2, doubl
         }
         return r2;
     }
+}
+
+// A real-space sum without what masked FP64 pairs left of it: a sum of nothing else
+// is zero (a real-space term itself would be below 1e-300 only past alpha r = 26).
+template <typename Real>
+__device__ inline double unmasked_sum(Real s) {
+    if constexpr (sizeof(Real) == 4) return (double)s;
+    else return fabs(s) < 1e-300 ? 0.0 : s;
 }
 
 // The image list as the pair loops read it: Cartesian xyz, and in the fourth
@@ -830,13 +838,13 @@ struct TypeSums {
         const double2 e = sums(S, c);
         g[k] += is_lj ? e.x : 0.0;
         g[NT + k] += is_lj ? c.y * e.y : 0.0;
-        g[2 * NT + k] += (double)S.sq;
+        g[2 * NT + k] += unmasked_sum(S.sq);
     }
     __device__ __attribute__((always_inline)) inline void add_dyn(int t, PairSums<Real>& S, bool is_lj) {
         const double2 f = sums(S, gc);
         const double e = is_lj ? f.x : 0.0;
         const double d = is_lj ? gc.y * f.y : 0.0;
-        const double c = (double)S.sq;
+        const double c = unmasked_sum(S.sq);
 #pragma unroll
         for (int k = 0; k < NT; ++k) {
             g[k] += (k == t) ? e : 0.0;
@@ -985,7 +993,7 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                 }
                 tile_close<ESM, Real>(C, m, P, lj_stride, lj_site, is_lj, r2lj, r2sr, et, small, ovl, S.plj, S.psr);
                 part_lj += (double)S.plj;
-                part_sr += (double)S.psr;
+                part_sr += unmasked_sum(S.psr);
             }
         }
         close_part();
@@ -1026,7 +1034,7 @@ __device__ __attribute__((always_inline)) inline void chunk_pairs(const RunArgs&
                                                          ovl, S);
                     }
                     acc_lj += (double)S.plj;
-                    acc_sr += (double)S.psr;
+                    acc_sr += unmasked_sum(S.psr);
                     if constexpr (GRAD) ts.flush(nsite, S, is_lj);  // FP64 per 64 candidates, as the energies
                 }
             }
