@@ -124,38 +124,20 @@ __device__ inline float erfc_f32(float x) {
     return t * __builtin_amdgcn_exp2f(y * 1.4426950408889634f);
 }
 
-template <typename Real>
-struct PairMath;
+// 4 eps s^3 (s^3 - 1), s = sigma^2 / r^2, in FP32
+__device__ inline float lj_f32(double r2, float sig2, float eps4) {
+    float s = sig2 * __builtin_amdgcn_rcpf((float)r2);
+    float s3 = s * s * s;
+    return eps4 * fmaf(s3, s3, -s3);
+}
 
-template <>
-struct PairMath<float> {
-    // 4 eps s^3 (s^3 - 1), s = sigma^2 / r^2
-    __device__ static inline float lj(double r2, float sig2, float eps4) {
-        float s = sig2 * __builtin_amdgcn_rcpf((float)r2);
-        float s3 = s * s * s;
-        return eps4 * fmaf(s3, s3, -s3);
-    }
-    // q erfc(alpha r) / r
-    __device__ static inline float coul(double r2, double q, double alpha) {
-        float rf2 = (float)r2;
-        float rinv = __builtin_amdgcn_rsqf(rf2);
-        float r = rf2 * rinv;
-        return (float)q * erfc_f32((float)alpha * r) * rinv;
-    }
-};
-
-template <>
-struct PairMath<double> {
-    __device__ static inline double lj(double r2, double sig2, double eps4) {
-        double s = sig2 / r2;
-        double s3 = s * s * s;
-        return eps4 * s3 * (s3 - 1.0);
-    }
-    __device__ static inline double coul(double r2, double q, double alpha) {
-        double r = sqrt(r2);
-        return q / r * erfc(r * alpha);
-    }
-};
+// q erfc(alpha r) / r in FP32
+__device__ inline float coul_f32(double r2, double q, double alpha) {
+    float rf2 = (float)r2;
+    float rinv = __builtin_amdgcn_rsqf(rf2);
+    float r = rf2 * rinv;
+    return (float)q * erfc_f32((float)alpha * r) * rinv;
+}
 
 // --------------------------------------------------------- reductions ----
 __device__ inline double wave_sum(double v) {

@@ -49,7 +49,6 @@ constexpr int SCAN_WG = 1024;      // work-items of the scan kernels
 constexpr int GT = PM_MAX_GRAD_TYPES;  // framework types of a gradient run (fixed stride)
 constexpr int GQ = 4;                  // per-type sums per point: d/d eps, d/d sigma, erfc/r, Fourier
 constexpr int GK = 3 + 3 * GT;         // per-workgroup partials of a gradient run
-static_assert(7 * GT <= 64, "a tile's cumulative type counts (at most 64, 7 bits each) fill one 64-bit word");
 
 // Points of a grid brick (a pair workgroup's points) per axis.
 constexpr int GRID_BRICK[3] = {8, 8, 4};
@@ -66,7 +65,7 @@ struct RunArgs {
     double inv4pe;
     int esm;                 // 0 no electrostatics, 1 LJ and Ewald share r_c, 2 separate cutoffs
     int fast;                // the image list serves the run (chunk_r within the limit)
-    int nsite, n_types, n_img, n_atoms, n_tiles;
+    int nsite, n_types, n_atoms, n_tiles;
     unsigned site_lj_mask, site_q_mask;
     const double4* img;      // images near the box, in spatial tiles: Cartesian xyz (A), and the charge (FP64 runs)
                              // or the type and FP32 charge (mixed runs); 64 more at the end

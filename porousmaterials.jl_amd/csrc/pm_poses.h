@@ -269,7 +269,7 @@ __global__ __launch_bounds__(WG) void pose_kernel(PoseArgs a) {
                 const double y = rsq64(r2);
                 const double i2 = y * y;
                 if constexpr (sizeof(Real) == 4) {
-                    acc_lj += in ? (double)PairMath<float>::lj(r2, c.sig2, c.eps4) : 0.0;
+                    acc_lj += in ? (double)lj_f32(r2, c.sig2, c.eps4) : 0.0;
                 } else {
                     const double w = c.sig2 * i2;
                     const double u = w * w * w;
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(WG) void pose_kernel(PoseArgs a) {
                         t = erfc(alpha * r) / r;
                     }
                     if constexpr (sizeof(Real) == 4)
-                        acc_sr += ins ? x.w * (double)PairMath<float>::coul(r2, p.w, alpha) : 0.0;
+                        acc_sr += ins ? x.w * (double)coul_f32(r2, p.w, alpha) : 0.0;
                     else
                         acc_sr += ins ? x.w * (p.w * t) : 0.0;
                     if constexpr (GRAD)

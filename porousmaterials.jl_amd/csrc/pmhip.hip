@@ -1161,7 +1161,6 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
     for (auto& r : runs) {
         RunArgs& a = r.ra;
         a.fast = 0;
-        a.n_img = 0;
         a.img = nullptr;
         a.img_type = nullptr;
         a.tile_sph = nullptr;
@@ -1184,7 +1183,6 @@ int execute_points(std::vector<PointRun>& runs, int mode, int precision, double*
                 a.fast = 1;
                 a.img = fp64 ? im->d_img : im->d_img_m;
                 a.img_type = im->d_type;
-                a.n_img = (int)im->n;
                 a.tile_sph = im->d_tile_sph;
                 a.tile_rng = im->d_tile_rng;
                 a.n_tiles = (int)im->n_tiles;
